@@ -213,7 +213,7 @@ int32_t ot2d_batch_compact(ot2d_case* c, int32_t* running);
  * (converged, retired or failed): parameters p (same model, precision and
  * instance count as the batch) and mesh md, which must fit the memory the
  * slot holds (its cells, vertices, LU workspace and residual tiles, and no
- * more rows per lane of the FP64 sweep than the batch's).  The slot's
+ * more groups of 64 rows than the batch's tallest mesh).  The slot's
  * memory is cleared as for a new case, its step counter and status reset,
  * and the captured step re-made at the next iteration; call ot2d_set_grid
  * (and ot2d_set_convergence) for it next.  Batches of one mesh per case

@@ -71,7 +71,7 @@ struct ot2d_case {
   DevConst c;
   int nmesh = 0, nspec = 1, nq = 5, nv = 4, lamin = 1, iturb = -1;
   int device = 0;
-  int lu_rl = 1;             // rows per lane of the LU-SGS sweeps
+  int lu_rl = 1;             // ceil(rows / 64) of the tallest mesh: slot sizes of ot2d_batch_admit
   int weno = 0;              // some case reconstructs with WENO5 (wider residual tiles)
   LaunchCfg cfg;             // launch choices that change no result (ot2d_set_launch, ot2d_autotune)
   int ncase = 1;             // independent cases (batch: one per mesh; otherwise 1)
@@ -541,7 +541,6 @@ static int32_t mesh_records(ot2d_case* c, int im, const ot2d_params* pc) {
     if (mb.xold) { M.xold = mb.xold + ov; M.yold = mb.yold + ov; M.xole = mb.xole + ov; M.yole = mb.yole + ov; }
     M.iblank = mb.iblank + o;
     M.lu = mb.lu + mb.lu_per * nsp;
-    M.lu_rl = c->lu_rl;
     M.lu_fp32 = p->lu_fp32 ? 1 : 0;
     M.bodyflag = 0;
     for (int ib = 0; ib < md.nbc; ++ib)
@@ -679,7 +678,6 @@ static int32_t create_impl(const ot2d_params* ps, int32_t ncase, int32_t nmesh, 
       return fail(OT2D_ERR_HIP, "spectral coefficients: %s", hipGetErrorString(e));
     }
   }
-  // rows per lane of the LU-SGS sweeps: one wavefront covers every row
   c->lu_rl = 1;
   for (int im = 0; im < nmesh; ++im) {
     int rl = (md[im].kmax - 1 + 63) / 64;
@@ -709,7 +707,7 @@ static int32_t create_impl(const ot2d_params* ps, int32_t ncase, int32_t nmesh, 
     if (md[im].nbc < 0 || md[im].nbc > OT2D_MAXBC) { free_case(c); return fail(OT2D_ERR_ARG, "nbc"); }
     if (md[im].kmax - 1 > 512) {
       free_case(c);
-      return fail(OT2D_ERR_UNSUPPORTED, "kmax=%d: the FP64 LU-SGS sweep holds at most 8 rows per lane, 512 rows",
+      return fail(OT2D_ERR_UNSUPPORTED, "kmax=%d: the LU-SGS sweep takes at most 512 rows",
                   md[im].kmax);
     }
     if (!c->lamin && (md[im].jmax - 1 > SA_LINE_MAX || md[im].kmax - 1 > SA_LINE_MAX)) {
@@ -717,10 +715,10 @@ static int32_t create_impl(const ot2d_params* ps, int32_t ncase, int32_t nmesh, 
       return fail(OT2D_ERR_UNSUPPORTED, "%d x %d: the turbulence line solves hold at most %d cells per line",
                   md[im].jmax, md[im].kmax, SA_LINE_MAX);
     }
-    if (lu_lds_need(md[im].jmax - 1, p->lu_fp32) > 160 * 1024) {
+    if (md[im].jmax - 1 > lu_max_ni(p->lu_fp32)) {
       free_case(c);
-      return fail(OT2D_ERR_UNSUPPORTED, "mesh %d (%d x %d) exceeds the LU-SGS sweep's LDS staging", im,
-                  md[im].jmax, md[im].kmax);
+      return fail(OT2D_ERR_UNSUPPORTED, "mesh %d (%d x %d): the LU-SGS sweep takes j lines of at most %d cells", im,
+                  md[im].jmax, md[im].kmax, lu_max_ni(p->lu_fp32));
     }
     mb.jmax = md[im].jmax; mb.kmax = md[im].kmax;
     mb.jd = mb.jmax + 1; mb.kd = mb.kmax + 1;
@@ -1769,8 +1767,9 @@ extern "C" int32_t ot2d_batch_admit(ot2d_case* c, int32_t icase, const ot2d_para
                 mb.jmax, mb.kmax);
   if (!c->lamin && (jmax - 1 > SA_LINE_MAX || kmax - 1 > SA_LINE_MAX))
     return fail(OT2D_ERR_UNSUPPORTED, "the turbulence line solves hold at most %d cells per line", SA_LINE_MAX);
-  if (lu_lds_need(jmax - 1, p->lu_fp32) > 160 * 1024)
-    return fail(OT2D_ERR_UNSUPPORTED, "%d x %d exceeds the LU-SGS sweep's LDS staging", jmax, kmax);
+  if (jmax - 1 > lu_max_ni(p->lu_fp32))
+    return fail(OT2D_ERR_UNSUPPORTED, "%d x %d: the LU-SGS sweep takes j lines of at most %d cells", jmax, kmax,
+                lu_max_ni(p->lu_fp32));
   if (c->iturb == 2 && !c->lamin)
     for (int ib = 0; ib < md->nbc; ++ib)
       if (md->bc[ib].ibtyp == 5) {

@@ -75,7 +75,6 @@ struct DevMesh {
   double *kw_f1, *kw_x, *kw_prod, *kw_cd;
   double *kw_s[2], *kw_a[2], *kw_b[2], *kw_c[2], *kw_ak[2], *kw_ck[2];
   double* lu;                // LU-SGS sweep records (workspace)
-  int lu_rl;                 // rows per lane of the LU-SGS sweeps (1..4)
   int lu_fp32;               // sweep arithmetic: 1 FP32, 0 FP64
   // per-case bookkeeping (shared by all instances of a case)
   int* status;               // 0 ok, 1 mstop, 2 norm
@@ -467,6 +466,8 @@ hipError_t launch_update_monitor(const DevMesh* dM, const DevMesh* hM, int nmi, 
 hipError_t launch_lu_finish(const DevMesh* dM, const DevMesh* hM, int nmi, int flags, int fp32, hipStream_t st);
 hipError_t launch_forces(const DevMesh* dM, int mi, double* out, hipStream_t st);
 hipError_t launch_tsrhs(const DevMesh* dM, const DevMesh* hM, int nmi, hipStream_t st);
+// bytes of one instance's LU-SGS workspace (rl: ceil(rows / 64) of the case's
+// tallest mesh, part of the size rule of batch slots)
 size_t lu_workspace_bytes(int jd, int kd, int rl);
 hipError_t launch_visrhs(const DevMesh* dM, const DevMesh* hM, int nmi, hipStream_t st, int norms = 0);
 // prim_done: the laminar viscosity and velocities are already in place
@@ -485,5 +486,6 @@ hipError_t launch_interp(const DevMesh* dM, const void* don, int ndon, const voi
                          hipStream_t st);
 size_t interp_donor_bytes();
 size_t interp_fringe_bytes();
-size_t lu_lds_need(int ni, int fp32);
+// longest j line (interior cells) a case may have
+int lu_max_ni(int fp32);
 }  // namespace ot2d

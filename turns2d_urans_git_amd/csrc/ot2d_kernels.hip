@@ -1127,85 +1127,74 @@ __device__ __forceinline__ void nb_k(const CellLoad& c, const LUCellF64& L, doub
 }
 
 // ----------------------------------------------------------------------
-// LU-SGS in three kernels.
+// LU-SGS in FP64 (the reference's arithmetic) in four kernels.
 //
 //  k_lu_prep    every cell in parallel: the quantities ilu2d derives per cell
 //               (src/lhs.f:524-564), s*tscale (src/step.f:141-148) and the
 //               point-Jacobi update of the halo sides (src/lhs.f:568-598),
-//               stored as 20-value records in the order the sweeps consume
-//               them (layout below).
-//  k_lu_sweep   one wavefront per instance and direction.  Lane l owns RL
-//               consecutive rows k = ks + l*RL + r and walks along j, one
-//               column per step, lane l one step behind lane l-1 (forward):
-//               cell (j,k) is done at step t = (j-js) + l.  Its j neighbour is
-//               the same lane's previous step (registers); its k neighbour is
-//               either the lane's own row below (same step) or lane l-1's top
-//               row of the previous step, passed by a DPP wavefront shift.
-//               No barrier and no LDS round trip sits on the dependent
-//               chain; records stream in D steps ahead.  The backward sweep
-//               mirrors this (t = (je-j) + (NL-1-l), DPP shift the other way).
-//               The result of every cell is the reference's (src/lhs.f:
-//               616-714 forward, 719-800 backward): a hyperplane order and
-//               this skewed order evaluate each cell from the same operands.
+//               stored as records in the order the sweeps consume them.
+//  k_lu_sweep64 the forward and the backward sweep (src/lhs.f:616-714,
+//               719-800), one workgroup per block of 32 rows.
 //  k_lu_finish  every cell in parallel: conservative restore of the in-place
 //               primitive conversion (src/lhs.f:805-811), the reference's s
 //               after ilu2d, and optionally the q update (src/step.f:205-211)
 //               and monitor (src/step.f:353-385).
 //
-// Record (20 values): s0..s3, sv, di, uu, vv, uv2, ge, xx, xy, qx, cj, pj,
-// yx, yy, qy, ck, pk (cj/pj and ck/pk: switch and spectral term of the
-// j and k directions for the sweep that reads the record).  FP32 packs it in
-// 5 float4, FP64 in 10 double2; vector q of entry n sits at plane q.
+// Rows k = ks .. ke are cut into W blocks of LU_R = 32.  Row r of a block
+// does column c at step t = c + r, where c = 0 is the halo column j = js-1
+// and c = ni+1 the halo column j = je+1: a halo cell is a record with
+// sv = 0 and di = 1, whose update returns its fixed s exactly, so every
+// neighbour term is formed the same way.  When the last block has a row to
+// spare (nk % 32 != 0) the halo row k = ke+1 is its last row, for the
+// backward sweep; otherwise that row, and always the halo row k = ks-1, is
+// kept apart (halo-row records) and enters as the block's fill.
 //
-// Workspace of one instance, in 16-byte vectors (NVEC = 10 planes reserved
-// so both precisions fit):
-//   F   forward records   entry n = (t*RL + r)*64 + l, t = (j-js) + l
-//   B   backward records  entry n = (t*RL + r)*64 + l, t = (je-j) + (NL-1-l);
-//       its s vectors receive the forward result, then the backward result
-//   HCF, HCB  halo column j = js-1 / je+1, entry r*64 + l
-//   HRF, HRB  halo row    k = ks-1 / ke+1, entry j-js
-//
-// T is the arithmetic of the sweep: double reproduces the reference, float
-// is the mixed-precision defect-correction variant (records rounded from the
-// FP64 values computed in k_lu_prep).
+// Record of one cell: 12 vectors of two doubles,
+//   0 (chk, spec) of j, 1 of k for the backward sweep; 2 (uu, vv);
+//   3 (uv2, ge); 4 (xx, xy); 5 (yx, yy); 6 (qx, qy); 7 (sv, di);
+//   8 (chk, spec) of j, 9 of k for the forward sweep; 10 (s1, s2); 11 (s3, s4)
+// stored per block and step as 12 planes of 32 rows, so the forward sweep
+// reads a step as the 5 KiB of planes 2-11 and the backward sweep as the
+// 4 KiB of planes 0-7.  A halo-row record has 7 vectors, plane-major over
+// the columns 1 .. ni: s, (uu, vv), (uv2, ge), (yx, yy), (-, qy), (chk, spec).
+// Results (forward H, backward H2) per block and step: 2 planes of 64
+// 16-byte units, lane 2r of plane p holding component 1+p and lane 2r+1
+// component 3+p of row r as (low word, tag, high word, tag).
+// Records of cells outside the grid are zero (the workspace is zero-filled
+// when the case is created, nothing else writes there) and give zeros.
 // ----------------------------------------------------------------------
 
-constexpr int LU_NVEC = 10;        // 16-byte planes reserved per array
-constexpr int LU32_R = 32;         // rows of one FP32 sweep workgroup (two lanes per row)
-constexpr int LU_MAXRL = 8;        // rows per lane: at most 512 rows
-
-template <typename T> struct LUV;
-template <> struct LUV<float> { static constexpr int N = 5; };
-template <> struct LUV<double> { static constexpr int N = 10; };
+constexpr int LU_R = 32;           // rows of one sweep workgroup (two lanes per row)
+constexpr int LU32_R = LU_R;
+constexpr int LU64_PL = 12;        // 16-byte vectors of an FP64 cell record
+constexpr int LU64_STEP = LU64_PL * LU_R;   // ... of one block and step
+constexpr int LU64_OUT = 4 * LU_R; // result units of one block and step
+constexpr int LU64_NF = 7;         // vectors of a halo-row record
 
 struct LUGeom {
-  int ni, nk, RL, NL, T;           // FP64 sweep: NL lanes, T steps
+  int ni, nk;
   int W, TW, TA;                   // FP32 sweep: W workgroups of LU32_R rows, TW steps each,
                                    // TA >= TW step rows of the record arrays (a multiple of 8)
-  long long nrec;                  // FP64: entries of F and of B
-  long long off_b, off_hcf, off_hcb, off_hrf, off_hrb;   // FP64 arrays (16-byte vectors)
+  int TD;                          // FP64 sweep: step rows of a block's arrays
+  long long off_dh, off_dh2, off_hrf, off_hrb, off_dtk;  // FP64 arrays (16-byte vectors; records at 0)
   long long ncell;                 // FP32: interior cells
   long long off_f32, off_b32, off_cb, off_h, off_h2;   // FP32 arrays
   long long off_tk;                // FP32 workgroup tickets (forward, backward): one vector
-  long long total;                 // vectors the workspace must hold (either layout)
 };
 
-__host__ __device__ inline LUGeom lu_geom(int ni, int nk, int RL) {
+__host__ __device__ inline LUGeom lu_geom(int ni, int nk) {
   LUGeom g;
-  g.ni = ni; g.nk = nk; g.RL = RL;
-  g.NL = (nk + RL - 1) / RL;
-  g.T = ni + g.NL - 1;
+  g.ni = ni; g.nk = nk;
   g.W = (nk + LU32_R - 1) / LU32_R;
   g.TW = ni + LU32_R - 1;
   g.TA = (g.TW + 7) & ~7;
-  g.nrec = (long long)g.T * RL * 64;
-  long long hc = (long long)RL * 64;
-  g.off_b = LU_NVEC * g.nrec;
-  g.off_hcf = 2 * LU_NVEC * g.nrec;
-  g.off_hcb = g.off_hcf + LU_NVEC * hc;
-  g.off_hrf = g.off_hcb + LU_NVEC * hc;
-  g.off_hrb = g.off_hrf + (long long)LU_NVEC * ni;
-  long long t64 = g.off_hrb + (long long)LU_NVEC * ni;
+  g.TD = ni + 2 + LU_R - 1;
+  const long long rows = (long long)g.W * g.TD;
+  g.off_dh = LU64_STEP * rows;
+  g.off_dh2 = g.off_dh + LU64_OUT * rows;
+  g.off_hrf = g.off_dh2 + LU64_OUT * rows;
+  g.off_hrb = g.off_hrf + (long long)LU64_NF * ni;
+  g.off_dtk = g.off_hrb + (long long)LU64_NF * ni;
   // FP32, all in step layout (per block and sweep step, a row of 64 lanes):
   // the forward records (4 vectors of 16 bytes per lane + one 8-byte pair:
   // 288 16-byte units), the backward records (4 vectors: 256 units), cB (8
@@ -1220,17 +1209,28 @@ __host__ __device__ inline LUGeom lu_geom(int ni, int nk, int RL) {
   g.off_h = g.off_cb + 32ll * g.W * g.TW;
   g.off_h2 = g.off_h + 64ll * g.W * g.TW;
   g.off_tk = g.off_h2 + 64ll * g.W * g.TW;
-  long long t32 = g.off_tk + 1;
-  g.total = t64 > t32 ? t64 : t32;
   return g;
 }
 
+// vectors an instance's workspace holds: either precision's arrays, and at
+// least 20 vectors per lane and step of 64-lane groups of rl rows, the size
+// slots were always given: a batch slot (ot2d_batch_admit) accepts a mesh
+// whose size by this rule fits its own
+static long long lu_total(int ni, int nk, int rl) {
+  const LUGeom g = lu_geom(ni, nk);
+  const int nl = (nk + rl - 1) / rl;
+  const long long a = 20ll * ((long long)(ni + nl - 1) * rl * 64 + (long long)rl * 64 + ni);
+  const long long b = g.off_dtk + 1, c = g.off_tk + 1;
+  return a > b ? (a > c ? a : c) : (b > c ? b : c);
+}
+
 __device__ __forceinline__ LUGeom lu_geom(const DevMesh& M) {
-  return lu_geom(M.je - M.js + 1, M.ke - M.ks + 1, M.lu_rl);
+  return lu_geom(M.je - M.js + 1, M.ke - M.ks + 1);
 }
 
 typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
+typedef double f64x2_t __attribute__((ext_vector_type(2)));
 struct D2 { double x, y; };
 struct F4 { float x, y, z, w; };
 struct F2 { float x, y; };
@@ -1246,69 +1246,6 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t uniform_rsrc(void* p, long lon
   return __builtin_amdgcn_make_buffer_rsrc(up, 0, nb, 0x00020000);
 }
 
-// one array of the workspace: plane q holds vector q of every entry
-struct LUArr {
-  D2* base;
-  long long n;     // entries per plane
-  __device__ __forceinline__ D2* at(int q, long long e) const { return base + q * n + e; }
-};
-
-__device__ __forceinline__ LUArr lu_arr(const DevMesh& M, long long off, long long n) {
-  LUArr a;
-  a.base = reinterpret_cast<D2*>(M.lu) + off;
-  a.n = n;
-  return a;
-}
-
-// write one record (FP64 values, rounded for the FP32 layout)
-template <typename T>
-__device__ __forceinline__ void rec_put(const LUArr& a, long long e, const double* f) {
-  if (sizeof(T) == 8) {
-#pragma unroll
-    for (int q = 0; q < 10; ++q) *a.at(q, e) = D2{f[2 * q], f[2 * q + 1]};
-  } else {
-#pragma unroll
-    for (int q = 0; q < 5; ++q)
-      *reinterpret_cast<F4*>(a.at(q, e)) = F4{(float)f[4 * q], (float)f[4 * q + 1], (float)f[4 * q + 2],
-                                              (float)f[4 * q + 3]};
-  }
-}
-
-template <typename T>
-__device__ __forceinline__ void rec_get(const LUArr& a, long long e, T* f) {
-  if constexpr (sizeof(T) == 8) {
-#pragma unroll
-    for (int q = 0; q < 10; ++q) { D2 v = *a.at(q, e); f[2 * q] = v.x; f[2 * q + 1] = v.y; }
-  } else {
-#pragma unroll
-    for (int q = 0; q < 5; ++q) {
-      F4 v = *reinterpret_cast<const F4*>(a.at(q, e));
-      f[4 * q] = v.x; f[4 * q + 1] = v.y; f[4 * q + 2] = v.z; f[4 * q + 3] = v.w;
-    }
-  }
-}
-
-template <typename T>
-__device__ __forceinline__ void rec_unpack(const u32x4_t* v, T* f) {
-  if constexpr (sizeof(T) == 8) {
-#pragma unroll
-    for (int q = 0; q < 10; ++q) { D2 d = __builtin_bit_cast(D2, v[q]); f[2 * q] = d.x; f[2 * q + 1] = d.y; }
-  } else {
-#pragma unroll
-    for (int q = 0; q < 5; ++q) {
-      F4 d = __builtin_bit_cast(F4, v[q]);
-      f[4 * q] = d.x; f[4 * q + 1] = d.y; f[4 * q + 2] = d.z; f[4 * q + 3] = d.w;
-    }
-  }
-}
-
-// entry of interior cell (j,k) in F (fwd) or B (bwd)
-__device__ __forceinline__ long long lu_entry(const DevMesh& M, const LUGeom& g, int j, int k, int dir) {
-  int kk = k - M.ks, l = kk / g.RL, r = kk - l * g.RL;
-  int t = dir > 0 ? (j - M.js) + l : (M.je - j) + (g.NL - 1 - l);
-  return ((long long)t * g.RL + r) * 64 + l;
-}
-
 // FP32 results of interior cell (j,k): workgroup w = (k-ks)/32 owns rows
 // ks+32w .. ks+32w+31, row r = (k-ks)%32 on lanes 2r (components 1, 2) and
 // 2r+1 (3, 4); forward step t = (j-js) + r, backward step t = (je-j) +
@@ -1321,240 +1258,104 @@ __device__ __forceinline__ long long lu_entry32(const DevMesh& M, const LUGeom& 
   return ((long long)w * g.TW + t) * 64 + 2 * r;
 }
 
+// A workgroup covers 8 rows of a block and 32 consecutive steps, 8
+// consecutive lanes being 8 rows at one step, so that each record plane is
+// stored as whole 128-byte runs; further workgroups take the halo rows.
+constexpr int LU64_PSTEPS = 32;
+__host__ __device__ inline int lu64_prep_tiles(const LUGeom& g) {
+  return g.W * (LU_R / 8) * ((g.TD + LU64_PSTEPS - 1) / LU64_PSTEPS);
+}
+
 __global__ __launch_bounds__(256) void k_lu_prep(const DevMesh* __restrict__ Ms) {
   const DevMesh& M = Ms[blockIdx.y];
   if (*M.status) return;
   const DevConst& C = M.c;
-  const int jd = M.jd, kd = M.kd, js = M.js, je = M.je, ks = M.ks, ke = M.ke;
   const double eps2 = C.epse * 2.;
   const double epsv = 1. + eps2;
   const LUGeom g = lu_geom(M);
-  const LUArr F = lu_arr(M, 0, g.nrec), B = lu_arr(M, g.off_b, g.nrec);
-  const LUArr HCF = lu_arr(M, g.off_hcf, (long long)g.RL * 64), HCB = lu_arr(M, g.off_hcb, (long long)g.RL * 64);
-  const LUArr HRF = lu_arr(M, g.off_hrf, g.ni), HRB = lu_arr(M, g.off_hrb, g.ni);
-  long long n2 = (long long)jd * kd;
-  for (long long i = blockIdx.x * 256ll + threadIdx.x; i < n2; i += 256ll * gridDim.x) {
-    int j = 1 + (int)(i % jd), k = 1 + (int)(i / jd);
-    double ts = M.tscale[i];
-    bool jin = (j >= js && j <= je), kin = (k >= ks && k <= ke);
-    if (!jin && !kin) {  // corner: only s*tscale
-      for (int n = 0; n < 4; ++n) M.s[n][i] = M.s[n][i] * ts;
-      continue;
+  D2* lu = reinterpret_cast<D2*>(M.lu);
+  const int tiles_t = (g.TD + LU64_PSTEPS - 1) / LU64_PSTEPS, tiles = lu64_prep_tiles(g);
+  const bool top_in = g.nk % LU_R != 0;   // the halo row k = ke+1 is the last block's last row
+  int c, kk, w = 0, t = -1;
+  if ((int)blockIdx.x < tiles) {
+    const int tb = (int)blockIdx.x % tiles_t, rest = (int)blockIdx.x / tiles_t;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int r = (rest % (LU_R / 8)) * 8 + (lane & 7);
+    w = rest / (LU_R / 8);
+    t = tb * LU64_PSTEPS + 8 * wave + (lane >> 3);
+    kk = LU_R * w + r;
+    c = t - r;
+    if (t >= g.TD || c < 0 || c > g.ni + 1 || kk > g.nk) return;
+    if (kk == g.nk && (!top_in || c == 0 || c == g.ni + 1)) return;
+  } else {
+    // the halo rows k = ks-1 and k = ke+1 (its corners alone when the last
+    // block holds it)
+    const int i = ((int)blockIdx.x - tiles) * 256 + threadIdx.x;
+    const int row = i / (g.ni + 2);
+    if (row > 1) return;
+    c = i % (g.ni + 2);
+    kk = row ? g.nk : -1;
+    if (row && top_in && c > 0 && c < g.ni + 1) return;
+  }
+  const long long i = cell(M, M.js - 1 + c, M.ks + kk);
+  const double ts = M.tscale[i];
+  const bool jin = c > 0 && c < g.ni + 1, kin = kk >= 0 && kk < g.nk;
+  if (!jin && !kin) {  // corner: only s*tscale
+    for (int n = 0; n < 4; ++n) M.s[n][i] = M.s[n][i] * ts;
+    return;
+  }
+  const CellLoad q = load_cell(M, i);
+  const LUCellF64 L = lu_of(C, q, epsv);
+  const bool interior = jin && kin;
+  double st[4];
+  for (int n = 0; n < 4; ++n) {
+    st[n] = M.s[n][i] * ts;
+    if (!interior) {
+      st[n] = st[n] * L.d;
+      M.s[n][i] = st[n];
     }
-    CellLoad c = load_cell(M, i);
-    LUCellF64 L = lu_of(C, c, epsv);
-    bool interior = jin && kin;
-    double st[4];
-    for (int n = 0; n < 4; ++n) {
-      st[n] = M.s[n][i] * ts;
-      if (!interior) {
-        st[n] = st[n] * L.d;
-        M.s[n][i] = st[n];
-      }
-    }
-    LUNb jf, jb, kf, kb;
-    nb_j(c, L, eps2, +1, jf);
-    nb_j(c, L, eps2, -1, jb);
-    nb_k(c, L, eps2, +1, kf);
-    nb_k(c, L, eps2, -1, kb);
-    double f[20] = {st[0], st[1], st[2], st[3], ts * 0.5, L.d, L.uu, L.vv, L.uv2, L.ge,
-                    c.xx, c.xy, L.qx, jf.chk, jf.spec, c.yx, c.yy, L.qy, kf.chk, kf.spec};
-    double b[20];
-    for (int n = 0; n < 20; ++n) b[n] = f[n];
-    b[13] = jb.chk; b[14] = jb.spec; b[18] = kb.chk; b[19] = kb.spec;
-    if (interior) {
-      rec_put<double>(F, lu_entry(M, g, j, k, +1), f);
-      rec_put<double>(B, lu_entry(M, g, j, k, -1), b);
-    } else if (kin) {  // halo column
-      int kk = k - ks, l = kk / g.RL, r = kk - l * g.RL;
-      long long e = (long long)r * 64 + l;
-      if (j == js - 1) rec_put<double>(HCF, e, f);
-      if (j == je + 1) rec_put<double>(HCB, e, b);
-    } else {           // halo row
-      long long e = j - js;
-      if (k == ks - 1) rec_put<double>(HRF, e, f);
-      if (k == ke + 1) rec_put<double>(HRB, e, b);
-    }
+  }
+  LUNb jf, jb, kf, kb;
+  nb_j(q, L, eps2, +1, jf);
+  nb_j(q, L, eps2, -1, jb);
+  nb_k(q, L, eps2, +1, kf);
+  nb_k(q, L, eps2, -1, kb);
+  if (t >= 0) {
+    D2* rec = lu + ((long long)w * g.TD + t) * LU64_STEP + (kk - LU_R * w);
+    rec[0 * LU_R] = D2{jb.chk, jb.spec};
+    rec[1 * LU_R] = D2{kb.chk, kb.spec};
+    rec[2 * LU_R] = D2{L.uu, L.vv};
+    rec[3 * LU_R] = D2{L.uv2, L.ge};
+    rec[4 * LU_R] = D2{q.xx, q.xy};
+    rec[5 * LU_R] = D2{q.yx, q.yy};
+    rec[6 * LU_R] = D2{L.qx, L.qy};
+    rec[7 * LU_R] = interior ? D2{ts * 0.5, L.d} : D2{0.0, 1.0};
+    rec[8 * LU_R] = D2{jf.chk, jf.spec};
+    rec[9 * LU_R] = D2{kf.chk, kf.spec};
+    rec[10 * LU_R] = D2{st[0], st[1]};
+    rec[11 * LU_R] = D2{st[2], st[3]};
+  } else {
+    const LUNb& b = kk < 0 ? kf : kb;
+    D2* h = lu + (kk < 0 ? g.off_hrf : g.off_hrb) + (c - 1);
+    h[0ll * g.ni] = D2{st[0], st[1]};
+    h[1ll * g.ni] = D2{st[2], st[3]};
+    h[2ll * g.ni] = D2{L.uu, L.vv};
+    h[3ll * g.ni] = D2{L.uv2, L.ge};
+    h[4ll * g.ni] = D2{q.yx, q.yy};
+    h[5ll * g.ni] = D2{0.0, L.qy};
+    h[6ll * g.ni] = D2{b.chk, b.spec};
   }
 }
 
-// what a cell needs of a neighbour: its new s and the static terms of the
-// direction it is a neighbour in
-template <typename T>
-struct NbT {
-  T s[4];
-  T uu, vv, uv2, ge, ri1, ri2, qq, chk, spec;
-};
-
-// A(+/-) or B(+/-) applied to the neighbour's s (src/lhs.f:633-651, 665-681)
-template <typename T>
-__device__ __forceinline__ void apply_nb(T gm1, const NbT<T>& n, T* a) {
-  T a4 = n.chk * (n.ri1 * n.s[1] + n.ri2 * n.s[2] - n.qq * n.s[0]);
-  T a2 = n.chk * gm1 * (n.uv2 * n.s[0] - (n.uu * n.s[1] + n.vv * n.s[2]) + n.s[3]);
-  a[0] = a4 + n.spec * n.s[0];
-  a[1] = n.ri1 * a2 + n.uu * a4 + n.spec * n.s[1];
-  a[2] = n.ri2 * a2 + n.vv * a4 + n.spec * n.s[2];
-  a[3] = n.qq * a2 + n.ge * a4 + n.spec * n.s[3];
-}
-
-template <typename T>
-__device__ __forceinline__ void jrole(const T* s, const T* f, NbT<T>& n) {
-  n.s[0] = s[0]; n.s[1] = s[1]; n.s[2] = s[2]; n.s[3] = s[3];
-  n.uu = f[6]; n.vv = f[7]; n.uv2 = f[8]; n.ge = f[9];
-  n.ri1 = f[10]; n.ri2 = f[11]; n.qq = f[12]; n.chk = f[13]; n.spec = f[14];
-}
-template <typename T>
-__device__ __forceinline__ void krole(const T* s, const T* f, NbT<T>& n) {
-  n.s[0] = s[0]; n.s[1] = s[1]; n.s[2] = s[2]; n.s[3] = s[3];
-  n.uu = f[6]; n.vv = f[7]; n.uv2 = f[8]; n.ge = f[9];
-  n.ri1 = f[15]; n.ri2 = f[16]; n.qq = f[17]; n.chk = f[18]; n.spec = f[19];
-}
-
-// wavefront shift of one value: DIR > 0 lane i receives lane i-1
-// (wave_shr:1), DIR < 0 lane i receives lane i+1 (wave_shl:1)
-template <int DIR>
-__device__ __forceinline__ int dpp_shift(int v) {
-  return __builtin_amdgcn_update_dpp(0, v, DIR > 0 ? 0x138 : 0x130, 0xf, 0xf, false);
-}
-template <int DIR>
-__device__ __forceinline__ float dpp_shift(float v) {
-  return __builtin_bit_cast(float, dpp_shift<DIR>(__builtin_bit_cast(int, v)));
-}
-template <int DIR>
-__device__ __forceinline__ double dpp_shift(double v) {
-  long long b = __builtin_bit_cast(long long, v);
-  int lo = dpp_shift<DIR>((int)(b & 0xffffffffll));
-  int hi = dpp_shift<DIR>((int)(b >> 32));
-  return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned int)lo);
-}
-template <int DIR, typename T>
-__device__ __forceinline__ NbT<T> dpp_shift_nb(const NbT<T>& x) {
-  NbT<T> y;
-#pragma unroll
-  for (int v = 0; v < 4; ++v) y.s[v] = dpp_shift<DIR>(x.s[v]);
-  y.uu = dpp_shift<DIR>(x.uu); y.vv = dpp_shift<DIR>(x.vv); y.uv2 = dpp_shift<DIR>(x.uv2);
-  y.ge = dpp_shift<DIR>(x.ge); y.ri1 = dpp_shift<DIR>(x.ri1); y.ri2 = dpp_shift<DIR>(x.ri2);
-  y.qq = dpp_shift<DIR>(x.qq); y.chk = dpp_shift<DIR>(x.chk); y.spec = dpp_shift<DIR>(x.spec);
-  return y;
-}
-
-constexpr int LU_HR = 13;   // values of a halo-row record kept in LDS
-
-template <typename T>
-__host__ __device__ inline size_t lu_lds_bytes(int ni) {
-  return sizeof(T) * (size_t)LU_HR * (size_t)ni;
-}
-
-template <typename T, int DIR, int RL, int D>
-__global__ __launch_bounds__(64) void k_lu_sweep(const DevMesh* __restrict__ Ms) {
-  extern __shared__ __attribute__((aligned(16))) double lds_raw[];
-  constexpr int NV = LUV<T>::N;
-  const DevMesh& M = Ms[blockIdx.x];
-  if (*M.status) return;
-  const int js = M.js, je = M.je, ks = M.ks, ke = M.ke;
-  const LUGeom g = lu_geom(M);
-  const int l = threadIdx.x;
-  const T gm1 = (T)M.c.gm1;
-  const int NT = g.T;
-  // records this sweep reads, and where its results go (the s vectors of B:
-  // forward writes entry T-1-t, backward overwrites entry t)
-  const long long roff = DIR > 0 ? 0 : g.off_b;
-  __amdgpu_buffer_rsrc_t rec[NV];
-#pragma unroll
-  for (int q = 0; q < NV; ++q) rec[q] = uniform_rsrc(reinterpret_cast<D2*>(M.lu) + roff + q * g.nrec, g.nrec * 16);
-  __amdgpu_buffer_rsrc_t outq[2];
-#pragma unroll
-  for (int q = 0; q < 2; ++q) outq[q] = uniform_rsrc(reinterpret_cast<D2*>(M.lu) + g.off_b + q * g.nrec, g.nrec * 16);
-  // halo row (k neighbour of the boundary lane) staged in LDS
-  T* hr = reinterpret_cast<T*>(lds_raw);
-  {
-    const LUArr HR = lu_arr(M, DIR > 0 ? g.off_hrf : g.off_hrb, g.ni);
-    for (int w = l; w < g.ni; w += 64) {
-      T f[20];
-      rec_get<T>(HR, w, f);
-      NbT<T> n;
-      krole(f, f, n);
-      T* x = hr + LU_HR * w;
-      x[0] = n.s[0]; x[1] = n.s[1]; x[2] = n.s[2]; x[3] = n.s[3]; x[4] = n.uu; x[5] = n.vv; x[6] = n.uv2;
-      x[7] = n.ge; x[8] = n.ri1; x[9] = n.ri2; x[10] = n.qq; x[11] = n.chk; x[12] = n.spec;
-    }
-  }
-  __syncthreads();
-  // j neighbour of every row's first cell: the halo column
-  NbT<T> A[RL];
-  {
-    const LUArr HC = lu_arr(M, DIR > 0 ? g.off_hcf : g.off_hcb, (long long)g.RL * 64);
-#pragma unroll
-    for (int r = 0; r < RL; ++r) {
-      T f[20];
-      rec_get<T>(HC, (long long)r * 64 + l, f);
-      jrole(f, f, A[r]);
-    }
-  }
-  NbT<T> kout;
-  jrole(hr, hr, kout);   // any finite values: only read by lanes that are inactive
-  const bool blane = DIR > 0 ? (l == 0) : (l == g.NL - 1);
-  const int vo = l * 16;
-  u32x4_t P[D][RL][NV];
-  auto fetch = [&](int tp, u32x4_t (&dst)[RL][NV]) {
-#pragma unroll
-    for (int r = 0; r < RL; ++r)
-#pragma unroll
-      for (int q = 0; q < NV; ++q)
-        dst[r][q] = __builtin_amdgcn_raw_buffer_load_b128(rec[q], vo, (tp * RL + r) * 1024, 0);
-  };
-#pragma unroll
-  for (int d = 0; d < D - 1; ++d)
-    if (d < NT) fetch(d, P[d]);
-  for (int t0 = 0; t0 < NT; t0 += D) {
-#pragma unroll
-    for (int d = 0; d < D; ++d) {
-      const int t = t0 + d;
-      if (t >= NT) break;
-      if (t + D - 1 < NT) fetch(t + D - 1, P[(d + D - 1) % D]);
-      const int j = DIR > 0 ? js + t - l : je - t + (g.NL - 1 - l);
-      const bool lact = l < g.NL && j >= js && j <= je;
-      NbT<T> kin = dpp_shift_nb<DIR>(kout);
-      if (blane) {
-        int jh = j - js;
-        jh = jh < 0 ? 0 : (jh >= g.ni ? g.ni - 1 : jh);
-        const T* x = hr + LU_HR * jh;
-        kin.s[0] = x[0]; kin.s[1] = x[1]; kin.s[2] = x[2]; kin.s[3] = x[3];
-        kin.uu = x[4]; kin.vv = x[5]; kin.uv2 = x[6]; kin.ge = x[7]; kin.ri1 = x[8]; kin.ri2 = x[9];
-        kin.qq = x[10]; kin.chk = x[11]; kin.spec = x[12];
-      }
-      const int ostep = DIR > 0 ? NT - 1 - t : t;
-#pragma unroll
-      for (int rr = 0; rr < RL; ++rr) {
-        const int r = DIR > 0 ? rr : RL - 1 - rr;
-        const int k = ks + l * RL + r;
-        const bool v = lact && k <= ke;
-        T f[20];
-        rec_unpack<T>(P[d][r], f);
-        T a[4], b[4], sn[4];
-        apply_nb(gm1, A[r], a);
-        apply_nb(gm1, kin, b);
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-          if (DIR > 0) sn[w] = (f[w] + f[4] * (a[w] + b[w])) * f[5];
-          else sn[w] = f[w] - f[4] * (a[w] + b[w]) * f[5];
-        }
-        if (v) {
-          const int so = (ostep * RL + r) * 1024;
-          if constexpr (sizeof(T) == 8) {
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, D2{sn[0], sn[1]}), outq[0], vo, so, 0);
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, D2{sn[2], sn[3]}), outq[1], vo, so, 0);
-          } else {
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, F4{sn[0], sn[1], sn[2], sn[3]}),
-                                                   outq[0], vo, so, 0);
-          }
-          jrole(sn, f, A[r]);
-          krole(sn, f, kin);
-        }
-      }
-      kout = kin;
-    }
-  }
+// A(+/-) or B(+/-) of a cell applied to its s (src/lhs.f:633-651, 665-681)
+struct LU64Op { double uu, vv, uv2, ge, ri1, ri2, qq, chk, spec; };
+__device__ __forceinline__ void lu64_apply(double gm1, const LU64Op& n, const double* s, double* a) {
+  const double a4 = n.chk * (n.ri1 * s[1] + n.ri2 * s[2] - n.qq * s[0]);
+  const double a2 = n.chk * gm1 * (n.uv2 * s[0] - (n.uu * s[1] + n.vv * s[2]) + s[3]);
+  a[0] = a4 + n.spec * s[0];
+  a[1] = n.ri1 * a2 + n.uu * a4 + n.spec * s[1];
+  a[2] = n.ri2 * a2 + n.vv * a4 + n.spec * s[2];
+  a[3] = n.qq * a2 + n.ge * a4 + n.spec * s[3];
 }
 
 // ------------------------------------------------- FP32 LU-SGS (matrix form)
@@ -2144,6 +1945,381 @@ __global__ __launch_bounds__(64 * (2 + NP)) void k_lu_sweep32(const DevMesh* __r
     if (l == 0) atomicCAS(M.status, 0, 3);
 }
 
+// ------------------------------------------------- FP64 LU-SGS sweeps
+// One FP64 sweep, every cell from the reference's operands in the
+// reference's order (-ffp-contract=off).  The workgroup's waves, the LDS
+// ring with its tags, the tickets, the tagged mail and the bounded waits are
+// k_lu_sweep32's (see there); what differs is the computing wave's work.
+// Lane pair 2r, 2r+1 holds row r, and both lanes hold the row's four s.  One
+// lane (role 0; the even one forward, the odd one backward) applies the row's
+// A term for the row's next column, the other (role 1) its B term for the
+// next row's cell of the same column, each from its own operators: 31
+// operations a lane and step instead of 62.  The next step's row takes the B
+// term by a wavefront shift of one lane, adds it to its own A term, forms
+// its s on role 0 and hands them to role 1 (two dependent hand-overs of four
+// values by DPP).  The block's first row takes the B term of its upstream
+// neighbour from the slot's fill (the shift's `old` operand, no select):
+// the mail wave forms it from the neighbour block's edge row (its mailed s
+// and its record) or from the halo-row records, 16 columns at a time.
+//
+// Bound by the dependent chain of ni + nk steps, each about 95 instructions
+// of one wave (215 ns).  Forward / backward: 141 / 147 us at 513x129, 70 / 73
+// at 257x65, 196 / 204 for 385x97 beside 401x401, 14 / 14 at 33x17.  The
+// sweep it replaced ran one wave per instance with ceil(nk/64) rows per
+// lane, applying both terms on every lane: 569 / 565, 203 / 202, 1740 / 1583
+// and 32 / 31 us, so no size is left to it.
+constexpr int LU64_SLOT = 10 * LU_R + 2;   // 16-byte units of a ring slot: 10 planes and the fill
+constexpr size_t lu64_lds(int S) { return (size_t)S * LU64_SLOT * 16 + 16 * ((S * 8 + 15) / 16) + 16 * 32; }
+
+// a double stored as (low word, tag, high word, tag)
+__device__ __forceinline__ double word_pair(u32x4_t v) {
+  return __builtin_bit_cast(double, ((unsigned long long)v.z << 32) | v.x);
+}
+template <int CTL>
+__device__ __forceinline__ double dpp_f64(double old, double v) {
+  const unsigned long long o = __builtin_bit_cast(unsigned long long, old), b = __builtin_bit_cast(unsigned long long, v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp((int)(unsigned)o, (int)(unsigned)b, CTL, 0xf, 0xf, false);
+  const unsigned hi =
+      (unsigned)__builtin_amdgcn_update_dpp((int)(unsigned)(o >> 32), (int)(unsigned)(b >> 32), CTL, 0xf, 0xf, false);
+  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+template <int CTL>
+__device__ __forceinline__ double dpp_f64_all(double v) {   // every lane has a source
+  const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)b, CTL, 0xf, 0xf, true);
+  const unsigned hi = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)(b >> 32), CTL, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+
+template <int DIR, int S, int NP, int PD>
+__global__ __launch_bounds__(64 * (2 + NP)) void k_lu_sweep64(const DevMesh* __restrict__ Ms) {
+  constexpr int R = LU_R;
+  // ring planes: the record planes in their order (forward 2-11, backward
+  // 0-7 with the forward result as planes 8, 9)
+  constexpr int P_UV = DIR > 0 ? 0 : 2, P_MET = P_UV + 2, P_QQ = P_UV + 4, P_SD = P_UV + 5;
+  constexpr int P_OP = DIR > 0 ? 6 : 0, P_S = 8;
+  extern __shared__ __attribute__((aligned(16))) double lds_raw[];
+  __shared__ int consumed, abort_flag, st0, wb_s;
+  __shared__ unsigned tag_s;
+  u32x4_t* ring = reinterpret_cast<u32x4_t*>(lds_raw);               // [S][LU64_SLOT]
+  int2* tags = reinterpret_cast<int2*>(ring + (size_t)S * LU64_SLOT);  // [S]: records, fill
+  unsigned* stage = reinterpret_cast<unsigned*>(ring + (size_t)S * LU64_SLOT + (S * 8 + 15) / 16);   // [16][8]
+  const DevMesh& M = Ms[blockIdx.y];
+  const LUGeom g = lu_geom(M);
+  D2* lu = reinterpret_cast<D2*>(M.lu);
+  if (threadIdx.x == 0) {
+    consumed = 0;
+    abort_flag = 0;
+    wb_s = 0;
+    tag_s = 0;
+    if ((int)blockIdx.x < g.W) {
+      unsigned long long* tk = reinterpret_cast<unsigned long long*>(lu + g.off_dtk) + (DIR > 0 ? 0 : 1);
+      const unsigned long long n = __hip_atomic_fetch_add(tk, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      wb_s = (int)(n % (unsigned long long)g.W);
+      tag_s = (unsigned)(n / (unsigned long long)g.W) + 1u;
+    }
+    st0 = *M.status;
+  }
+  __syncthreads();
+  if (st0 || (int)blockIdx.x >= g.W) return;
+  const int wb = wb_s;
+  const unsigned tag = tag_s;
+  const int w = DIR > 0 ? wb : g.W - 1 - wb;   // row block of this workgroup
+  // rows of the block (the halo row k = ke+1 among them where it has room)
+  // and its steps: forward step t is record step t, backward step t record
+  // step NT-1-t
+  const int left = g.nk - R * w;
+  const int nr = left >= R ? R : left + 1;
+  const int NT = g.ni + 1 + nr;
+  // where the fill of the first row comes from: the upstream block's edge
+  // row, a halo row kept apart, or nowhere (the halo row is in the block)
+  const bool from_block = DIR > 0 ? w > 0 : w < g.W - 1;
+  const bool has_in = from_block || DIR > 0 || nr == R && left == R;
+  if (threadIdx.x < S) {
+    tags[threadIdx.x] = int2{0, has_in ? 0 : INT_MAX};
+    u32x4_t* f = ring + (size_t)threadIdx.x * LU64_SLOT + 10 * R;
+    f[0] = u32x4_t{0u, 0u, 0u, 0u};
+    f[1] = u32x4_t{0u, 0u, 0u, 0u};
+  }
+  __syncthreads();
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63;
+  const long long rows = (long long)g.W * g.TD;
+  const __amdgpu_buffer_rsrc_t hnd = uniform_rsrc(lu + g.off_dh, rows * (LU64_OUT * 16));
+  const __amdgpu_buffer_rsrc_t hout = DIR > 0 ? hnd : uniform_rsrc(lu + g.off_dh2, rows * (LU64_OUT * 16));
+  const double gm1 = M.c.gm1;
+  if (wave == NP + 1) {
+    // ---------------------------------------------------------- mail wave
+    // Fill of this block's step te = e + 1 for columns e = 0 .. ni-1 in sweep
+    // order (column c = e+1 forward, ni-e backward): the B term of the
+    // upstream row at that column.  Lane i < 16 of a window forms column
+    // e0 + i; the operators of the next window are loaded while this one
+    // waits.  A poll reads the window's 16 entries, lane l word l%8 of
+    // entries l/8 and 8 + l/8: word v of an entry is half v%2 of
+    // component (v/4) + 2((v/2)%2).
+    if (!has_in) return;
+    const int wn = w - DIR;
+    gu64* const mail = (gu64*)(lu + (DIR > 0 ? g.off_dh : g.off_dh2));
+    // operators: planes at unit `ob` + `oc` x column + `op` x plane
+    const D2* ob;
+    long long oc;
+    int o_uv, o_ge, o_y, o_q, o_c;
+    const long long hb = DIR > 0 ? g.off_hrf : g.off_hrb;
+    if (from_block) {
+      // edge row: row R-1 at record step c + R-1, or row 0 at step c
+      ob = lu + ((long long)wn * g.TD + (DIR > 0 ? R - 1 : 0)) * LU64_STEP + (DIR > 0 ? R - 1 : 0);
+      oc = LU64_STEP;
+      o_uv = 2 * R; o_ge = 3 * R; o_y = 5 * R; o_q = 6 * R; o_c = (DIR > 0 ? 9 : 1) * R;
+    } else {
+      ob = lu + hb - 1;   // column c at entry c-1
+      oc = 1;
+      o_uv = 2 * g.ni; o_ge = 3 * g.ni; o_y = 4 * g.ni; o_q = 5 * g.ni; o_c = 6 * g.ni;
+    }
+    auto col = [&](int e) {
+      const int ec = e < g.ni ? e : g.ni - 1;
+      return DIR > 0 ? ec + 1 : g.ni - ec;
+    };
+    auto ops = [&](int e0, LU64Op& o) {
+      const D2* p = ob + oc * col(e0 + (l & 15));
+      const D2 a = p[o_uv], b = p[o_ge], y = p[o_y], q = p[o_q], c = p[o_c];
+      o.uu = a.x; o.vv = a.y; o.uv2 = b.x; o.ge = b.y; o.ri1 = y.x; o.ri2 = y.y; o.qq = q.y;
+      o.chk = c.x; o.spec = c.y;
+    };
+    // words of column c's entry: result unit ((wn*TD + step) * 128 + 64 p +
+    // edge lane), two 8-byte words each
+    auto word = [&](int e, int v) -> unsigned long long {
+      const long long step = (long long)wn * g.TD + col(e) + (DIR > 0 ? R - 1 : 0);
+      const long long u = (step * LU64_OUT + 64 * (v >> 2) + (DIR > 0 ? 62 : 0) + ((v >> 1) & 1)) * 2 + (v & 1);
+      return __hip_atomic_load(mail + u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    };
+    const int sw = (l >> 3) * 8 + (((l >> 2) & 1) + (l & 2)) * 2 + (l & 1);   // where word l%8 of entry l/8 is staged
+    // n fills from step t1 on, lane i < n holding the fill of step t1 + i,
+    // each into its slot as soon as the slot is free
+    auto deliver = [&](int t1, int i0, int n, const double* b) -> bool {
+      for (int done = 0; done < n;) {
+        const int tq = t1 + done;
+        const int c = __hip_atomic_load(&consumed, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
+        int m = c + S - tq;
+        if (m <= 0) {
+          if (!spin_until_ge<2>(&consumed, tq - S + 1, &abort_flag)) return false;
+          continue;
+        }
+        m = m < n - done ? m : n - done;
+        const int i = l - i0;
+        if (i >= done && i < done + m) {
+          const int te = t1 + i;
+          f64x2_t* f = reinterpret_cast<f64x2_t*>(ring + (size_t)(te % S) * LU64_SLOT + 10 * R);
+          f[0] = f64x2_t{b[0], b[1]};
+          f[1] = f64x2_t{b[2], b[3]};
+          __hip_atomic_store(&tags[te % S].y, te + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+        done += m;
+      }
+      return true;
+    };
+    const double zero[4] = {0.0, 0.0, 0.0, 0.0};
+    if (!deliver(0, 0, 1, zero)) return;   // the halo column takes no fill
+    LU64Op cur, nxt;
+    ops(0, cur);
+    bool ok = true;
+    for (int e0 = 0; e0 < g.ni && ok; e0 += 16) {
+      const int ne = g.ni - e0 < 16 ? g.ni - e0 : 16;
+      ops(e0 + 16, nxt);
+      double s[4], b[4];
+      if (!from_block) {
+        const D2* p = lu + hb + (col(e0 + (l & 15)) - 1);
+        const D2 a = p[0], c = p[g.ni];
+        s[0] = a.x; s[1] = a.y; s[2] = c.x; s[3] = c.y;
+        lu64_apply(gm1, cur, s, b);
+        ok = deliver(e0 + 1, 0, ne, b);
+      } else {
+        int done = 0;
+        unsigned long long t_wait = rt_now();
+        while (ok && done < ne) {
+          const unsigned long long x0 = word(e0 + (l >> 3), l & 7), x1 = word(e0 + 8 + (l >> 3), l & 7);
+          // entry i is ready when its eight lanes are: count the ready prefix
+          auto prefix = [](unsigned long long m) -> int {
+            m &= m >> 4; m &= m >> 2; m &= m >> 1;
+            const unsigned long long nr = ~(m | 0xFEFEFEFEFEFEFEFEull);
+            return nr ? (int)(__builtin_ctzll(nr) / 8) : 8;
+          };
+          int n = prefix(__ballot((unsigned)(x0 >> 32) == tag));
+          if (n == 8) n += prefix(__ballot((unsigned)(x1 >> 32) == tag));
+          n = n < ne ? n : ne;
+          if (n <= done) {
+            if (__hip_atomic_load(&abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) { ok = false; break; }
+            if (rt_now() - t_wait > LU32_WAIT) {
+              __hip_atomic_store(&abort_flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+              ok = false;
+              break;
+            }
+            __builtin_amdgcn_s_sleep(1);
+            continue;
+          }
+          t_wait = rt_now();
+          // gather each entry's four doubles in its lane through LDS (one
+          // wave's LDS operations run in order)
+          stage[sw] = (unsigned)x0;
+          stage[64 + sw] = (unsigned)x1;
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          const f64x2_t* q = reinterpret_cast<const f64x2_t*>(stage) + (l & 15) * 2;
+          const f64x2_t p0 = q[0], p1 = q[1];
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          s[0] = p0.x; s[1] = p0.y; s[2] = p1.x; s[3] = p1.y;
+          lu64_apply(gm1, cur, s, b);
+          ok = deliver(e0 + 1 + done, done, n - done, b);
+          done = n;
+        }
+      }
+      cur = nxt;
+    }
+    // past the last column: zero fills
+    for (int t = g.ni + 1; t < NT && ok; t += 16) ok = deliver(t, 0, NT - t < 16 ? NT - t : 16, zero);
+    return;
+  }
+  if (wave > 0) {
+    // ---------------------------------------------------------- producers
+    const __amdgpu_buffer_rsrc_t rec = uniform_rsrc(lu, rows * (LU64_STEP * 16));
+    constexpr int NL = DIR > 0 ? 5 : 6;
+    auto fetch = [&](int tt, u32x4_t (&v)[NL]) {
+      const int tc = tt < NT ? tt : NT - 1;
+      if constexpr (DIR > 0) {
+        const int so = (w * g.TD + tc) * (LU64_STEP * 16) + 2 * R * 16;
+#pragma unroll
+        for (int q = 0; q < 5; ++q) v[q] = __builtin_amdgcn_raw_buffer_load_b128(rec, l * 16, so + q * 1024, 0);
+      } else {
+        const int step = w * g.TD + NT - 1 - tc;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          v[q] = __builtin_amdgcn_raw_buffer_load_b128(rec, l * 16, step * (LU64_STEP * 16) + q * 1024, 0);
+        // the forward result: this lane's two components
+        v[4] = __builtin_amdgcn_raw_buffer_load_b128(hnd, l * 16, step * (LU64_OUT * 16), 0);
+        v[5] = __builtin_amdgcn_raw_buffer_load_b128(hnd, l * 16, step * (LU64_OUT * 16) + 1024, 0);
+      }
+    };
+    auto put = [&](int tt, const u32x4_t (&v)[NL]) -> bool {
+      if (tt >= NT) return true;
+      if (!spin_until_ge<4>(&consumed, tt - S + 1, &abort_flag)) return false;
+      u32x4_t* d = ring + (size_t)(tt % S) * LU64_SLOT;
+#pragma unroll
+      for (int q = 0; q < (DIR > 0 ? 5 : 4); ++q) d[q * 64 + l] = v[q];
+      if constexpr (DIR < 0)
+        d[P_S * R + (l & 1) * R + (l >> 1)] = u32x4_t{v[4].x, v[4].z, v[5].x, v[5].z};
+      if (l == 0) __hip_atomic_store(&tags[tt % S].x, tt + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+      return true;
+    };
+    // producer wave p handles steps p-1, p-1+NP, ...; buffer k % PD holds the
+    // k-th of them, fetched PD-1 deliveries ahead
+    u32x4_t vb[PD][NL];
+    const int t0 = wave - 1;
+#pragma unroll
+    for (int k = 0; k < PD - 1; ++k) fetch(t0 + k * NP, vb[k]);
+    bool ok = true;
+    for (int tb = t0; tb < NT && ok; tb += PD * NP) {
+#pragma unroll
+      for (int k = 0; k < PD; ++k) {
+        const int tt = tb + k * NP;
+        fetch(tt + (PD - 1) * NP, vb[(k + PD - 1) % PD]);
+        if (ok) ok = put(tt, vb[k]);
+      }
+    }
+    return;
+  }
+  // ------------------------------------------------------------- compute
+  __builtin_amdgcn_s_setprio(3);
+  const int r = l >> 1, h = DIR > 0 ? (l & 1) : 1 - (l & 1);
+  const bool odd = l & 1;
+  // byte offsets in a slot: by row, and by row and role
+  const int o_row = r * 16, o_role = (h * R + r) * 16, o_q = r * 16 + h * 8;
+  struct Rec {
+    f64x2_t uv, ge, met, op, sd, s01, s23, f01, f23;
+    double qq;
+  };
+  auto rd = [&](int slot, Rec& v, int& tv) {
+    const char* s = reinterpret_cast<const char*>(ring) + (size_t)slot * (LU64_SLOT * 16);
+    const int2 tp = tags[slot];
+    tv = tp.x < tp.y ? tp.x : tp.y;
+    asm volatile("" ::: "memory");   // the tags' read before the records'
+    auto ld = [&](int plane, int o) { return *reinterpret_cast<const f64x2_t*>(s + plane * (R * 16) + o); };
+    v.sd = ld(P_SD, o_row);
+    v.s01 = ld(P_S, o_row);
+    v.s23 = ld(P_S + 1, o_row);
+    v.f01 = ld(10, 0);
+    v.f23 = ld(10, 16);
+    v.uv = ld(P_UV, o_row);
+    v.ge = ld(P_UV + 1, o_row);
+    v.met = ld(P_MET, o_role);
+    v.op = ld(P_OP, o_role);
+    v.qq = *reinterpret_cast<const double*>(s + P_QQ * (R * 16) + o_q);
+  };
+  auto spin_tags = [&](int slot, int target) -> bool {
+    return spin_until_ge<1>(&tags[slot].x, target, &abort_flag) && spin_until_ge<1>(&tags[slot].y, target, &abort_flag);
+  };
+  bool ok = true;
+  double T[4] = {0.0, 0.0, 0.0, 0.0};   // this lane's term (A or B by role) of its row's last cell
+  u32x4_t hx = {0u, tag, 0u, tag}, hy = {0u, tag, 0u, tag};   // the stored words; the tags stay put
+  auto step = [&](int slot, int t, Rec& C, int& tc, Rec& N, int& tn) {
+    const int s2 = slot + 2 < S ? slot + 2 : slot + 2 - S;
+    if (__builtin_expect(__builtin_amdgcn_readfirstlane(tc) < t + 1, 0)) {
+      // read before its writers finished: wait for the tags, read again
+      ok = ok && spin_tags(slot, t + 1);
+      rd(slot, C, tc);
+    }
+    // slots up to step t are free: see k_lu_sweep32
+    if (slot % 3 == 2) {
+      asm volatile("" ::: "memory");
+      __hip_atomic_store(&consumed, t + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    rd(s2, N, tn);   // past the last step: a harmless read of a stale slot
+    constexpr int SH = DIR > 0 ? 0x138 : 0x130;      // wave_shr:1 / wave_shl:1
+    constexpr int BC = DIR > 0 ? 0xA0 : 0xF5;        // quad_perm: role 0 of each pair to both
+    const double fl[4] = {C.f01.x, C.f01.y, C.f23.x, C.f23.y};
+    const double f[4] = {C.s01.x, C.s01.y, C.s23.x, C.s23.y};
+    double sn[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const double b = dpp_f64<SH>(fl[v], T[v]);
+      double x;
+      if (DIR > 0) x = (f[v] + C.sd.x * (T[v] + b)) * C.sd.y;
+      else x = f[v] - C.sd.x * (T[v] + b) * C.sd.y;
+      sn[v] = dpp_f64_all<BC>(x);
+    }
+    const LU64Op op = {C.uv.x, C.uv.y, C.ge.x, C.ge.y, C.met.x, C.met.y, C.qq, C.op.x, C.op.y};
+    lu64_apply(gm1, op, sn, T);
+    const int orow = (w * g.TD + (DIR > 0 ? t : NT - 1 - t)) * (LU64_OUT * 16);
+    const unsigned long long x = __builtin_bit_cast(unsigned long long, odd ? sn[2] : sn[0]);
+    const unsigned long long y = __builtin_bit_cast(unsigned long long, odd ? sn[3] : sn[1]);
+    hx.x = (unsigned)x; hx.z = (unsigned)(x >> 32);
+    hy.x = (unsigned)y; hy.z = (unsigned)(y >> 32);
+    __builtin_amdgcn_raw_buffer_store_b128(hx, hout, l * 16, orow, LU32_SYS);
+    __builtin_amdgcn_raw_buffer_store_b128(hy, hout, l * 16, orow + 1024, LU32_SYS);
+  };
+  Rec C0, C1, C2;
+  int tc0 = 0, tc1 = 0, tc2 = 0;
+  ok = spin_tags(0, 1);
+  rd(0, C0, tc0);
+  rd(1, C1, tc1);   // checked (and read again if early) at step 1
+  static_assert(S % 3 == 0, "the ring holds a multiple of 3 steps");
+  int t0 = 0;
+  for (; t0 + S <= NT && ok; t0 += S) {
+#pragma unroll
+    for (int i = 0; i < S; i += 3) {
+      step(i, t0 + i, C0, tc0, C2, tc2);
+      step(i + 1, t0 + i + 1, C1, tc1, C0, tc0);
+      step(i + 2, t0 + i + 2, C2, tc2, C1, tc1);
+    }
+  }
+  if (ok) {
+#pragma unroll
+    for (int i = 0; i < S; i += 3) {
+      if (t0 + i < NT) step(i, t0 + i, C0, tc0, C2, tc2);
+      if (t0 + i + 1 < NT) step(i + 1, t0 + i + 1, C1, tc1, C0, tc0);
+      if (t0 + i + 2 < NT) step(i + 2, t0 + i + 2, C2, tc2, C1, tc1);
+    }
+  }
+  if (!ok || __hip_atomic_load(&abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP))
+    if (l == 0) atomicCAS(M.status, 0, 3);
+}
+
 __device__ __forceinline__ bool asq_bad(const DevConst& C, double q1, double q2, double q3, double q4) {
   double rho = q1;
   double qq = sq(q2) + sq(q3);
@@ -2161,8 +2337,8 @@ __global__ __launch_bounds__(256) void k_lu_finish(const DevMesh* __restrict__ M
   const int fuse_update = flags & 1, sa_prim = flags & 2;
   const int jd = M.jd, kd = M.kd, js = M.js, je = M.je, ks = M.ks, ke = M.ke;
   const LUGeom g = lu_geom(M);
-  const LUArr B = lu_arr(M, g.off_b, g.nrec);
   const F4* H2 = reinterpret_cast<const F4*>(reinterpret_cast<const D2*>(M.lu) + g.off_h2);
+  const u32x4_t* D = reinterpret_cast<const u32x4_t*>(reinterpret_cast<const D2*>(M.lu) + g.off_dh2);
   long long n2 = (long long)jd * kd;
   int bad = 0;
   for (long long i = blockIdx.x * 256ll + threadIdx.x; i < n2; i += 256ll * gridDim.x) {
@@ -2186,9 +2362,9 @@ __global__ __launch_bounds__(256) void k_lu_finish(const DevMesh* __restrict__ M
     if (jin && kin) {
       double dq[4];
       if constexpr (sizeof(T) == 8) {
-        const long long e = lu_entry(M, g, j, k, -1);
-        D2 a = *B.at(0, e), b = *B.at(1, e);
-        dq[0] = a.x; dq[1] = a.y; dq[2] = b.x; dq[3] = b.y;
+        const int kk = k - ks, r = kk % LU_R;
+        const u32x4_t* e = D + ((long long)(kk / LU_R) * g.TD + (j - js + 1) + r) * LU64_OUT + 2 * r;
+        dq[0] = word_pair(e[0]); dq[2] = word_pair(e[1]); dq[1] = word_pair(e[64]); dq[3] = word_pair(e[65]);
       } else {
         const long long e = lu_entry32(M, g, j, k, -1);
         const F4 a = H2[e], b = H2[e + 1];   // (value, tag) words
@@ -2725,36 +2901,42 @@ hipError_t launch_rbc(const DevMesh* dM, int nmi, hipStream_t st) {
   return hipGetLastError();
 }
 
-template <typename T, int RL, int D>
-static hipError_t launch_lu_t(const DevMesh* dM, const DevMesh* hM, int nmi, int fuse_update, Marks* mk,
+// every FP64 case: the ring's 12 slots (62 KB) leave room for two workgroups
+// on a CU, and three producers of five steps in flight cover the records'
+// latency at 215 ns a step
+static hipError_t launch_lu64(const DevMesh* dM, const DevMesh* hM, int nmi, int fuse_update, Marks* mk,
                               hipStream_t st) {
-  long long mx = 0;
-  int nimax = 0;
+  constexpr int S = 12, NP = 3, PD = 5;
+  long long mx = 0, np = 0;
+  int wmax = 1;
   for (int i = 0; i < nmi; ++i) {
     mx = hM[i].jd * (long long)hM[i].kd > mx ? hM[i].jd * (long long)hM[i].kd : mx;
-    nimax = hM[i].je - hM[i].js + 1 > nimax ? hM[i].je - hM[i].js + 1 : nimax;
+    const LUGeom g = lu_geom(hM[i].je - hM[i].js + 1, hM[i].ke - hM[i].ks + 1);
+    const long long n = lu64_prep_tiles(g) + (2ll * (g.ni + 2) + 255) / 256;
+    np = n > np ? n : np;
+    wmax = g.W > wmax ? g.W : wmax;
   }
-  size_t lds = lu_lds_bytes<T>(nimax);
+  constexpr size_t lds = lu64_lds(S);
   static bool attr_set = false;
   if (!attr_set) {
-    (void)hipFuncSetAttribute((const void*)k_lu_sweep<T, 1, RL, D>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              160 * 1024);
-    (void)hipFuncSetAttribute((const void*)k_lu_sweep<T, -1, RL, D>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              160 * 1024);
+    (void)hipFuncSetAttribute((const void*)k_lu_sweep64<1, S, NP, PD>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              (int)lds);
+    (void)hipFuncSetAttribute((const void*)k_lu_sweep64<-1, S, NP, PD>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              (int)lds);
     attr_set = true;
   }
-  hipLaunchKernelGGL(k_lu_prep, dim3(nblk(mx, 256), nmi), dim3(256), 0, st, dM);
+  hipLaunchKernelGGL(k_lu_prep, dim3((unsigned)np, nmi), dim3(256), 0, st, dM);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   mark(mk, OT2D_ST_LU_PREP, st);
-  hipLaunchKernelGGL((k_lu_sweep<T, 1, RL, D>), dim3(nmi), dim3(64), lds, st, dM);
+  hipLaunchKernelGGL((k_lu_sweep64<1, S, NP, PD>), dim3(wmax, nmi), dim3(64 * (2 + NP)), lds, st, dM);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_LU_FORWARD, st);
-  hipLaunchKernelGGL((k_lu_sweep<T, -1, RL, D>), dim3(nmi), dim3(64), lds, st, dM);
+  hipLaunchKernelGGL((k_lu_sweep64<-1, S, NP, PD>), dim3(wmax, nmi), dim3(64 * (2 + NP)), lds, st, dM);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_LU_BACKWARD, st);
   if (fuse_update & 4) return hipSuccess;
-  hipLaunchKernelGGL(k_lu_finish<T>, dim3(nblk(mx, 256), nmi), dim3(256), 0, st, dM, fuse_update);
+  hipLaunchKernelGGL(k_lu_finish<double>, dim3(nblk(mx, 256), nmi), dim3(256), 0, st, dM, fuse_update);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_LU_FINISH, st);
   return hipSuccess;
@@ -2796,7 +2978,7 @@ static hipError_t launch_lu32(const DevMesh* dM, const DevMesh* hM, int nmi, int
   for (int i = 0; i < nmi; ++i) {
     mx = hM[i].jd * (long long)hM[i].kd > mx ? hM[i].jd * (long long)hM[i].kd : mx;
     int nk = hM[i].ke - hM[i].ks + 1, ni = hM[i].je - hM[i].js + 1;
-    const LUGeom gg = lu_geom(ni, nk, hM[i].lu_rl);
+    const LUGeom gg = lu_geom(ni, nk);
     const long long nprep = (long long)gg.W * (LU32_R / 8) * ((gg.TA + LP_STEPS - 1) / LP_STEPS);   // prep tiles
     nc = nprep > nc ? nprep : nc;
     wmax = gg.W > wmax ? gg.W : wmax;
@@ -2832,36 +3014,16 @@ hipError_t launch_lu_finish(const DevMesh* dM, const DevMesh* hM, int nmi, int f
   return hipGetLastError();
 }
 
-// rows per lane rl = ceil(rows / 64) of the case (all instances share it)
 hipError_t launch_lu(const DevMesh* dM, const DevMesh* hM, int nmi, int fuse_update, int fp32, Marks* mk,
                      hipStream_t st, int sweep) {
-  const int rl = hM[0].lu_rl;
-  if (fp32) {
-    return launch_lu32(dM, hM, nmi, fuse_update, mk, st, sweep);
-  } else {
-    // prefetch depth D chosen so the record ring fits the register file
-    switch (rl) {
-      case 1: return launch_lu_t<double, 1, 3>(dM, hM, nmi, fuse_update, mk, st);
-      case 2: return launch_lu_t<double, 2, 2>(dM, hM, nmi, fuse_update, mk, st);
-      case 3: return launch_lu_t<double, 3, 1>(dM, hM, nmi, fuse_update, mk, st);
-      case 4: return launch_lu_t<double, 4, 1>(dM, hM, nmi, fuse_update, mk, st);
-      // tall meshes (Cartesian backgrounds of overset cases); the FP32 sweep
-      // has no such bound
-      case 5: return launch_lu_t<double, 5, 1>(dM, hM, nmi, fuse_update, mk, st);
-      case 6: return launch_lu_t<double, 6, 1>(dM, hM, nmi, fuse_update, mk, st);
-      case 7: return launch_lu_t<double, 7, 1>(dM, hM, nmi, fuse_update, mk, st);
-      case 8: return launch_lu_t<double, 8, 1>(dM, hM, nmi, fuse_update, mk, st);
-    }
-  }
-  return hipErrorInvalidValue;
+  if (fp32) return launch_lu32(dM, hM, nmi, fuse_update, mk, st, sweep);
+  return launch_lu64(dM, hM, nmi, fuse_update, mk, st);
 }
 
-size_t lu_lds_need(int ni, int fp32) {
-  return fp32 ? lu_lds_bytes<float>(ni) : lu_lds_bytes<double>(ni);
-}
+int lu_max_ni(int fp32) { return fp32 ? 3150 : 1575; }
 
 size_t lu_workspace_bytes(int jd, int kd, int rl) {
-  return 16 * (size_t)lu_geom(jd - 2, kd - 2, rl).total;
+  return 16 * (size_t)lu_total(jd - 2, kd - 2, rl);
 }
 
 hipError_t launch_update_monitor(const DevMesh* dM, const DevMesh* hM, int nmi, hipStream_t st, int take_turmu) {
