@@ -107,215 +107,205 @@ typedef __attribute__((address_space(1))) double gdouble;
 __device__ __forceinline__ gdouble* gptr(double* p) { return (gdouble*)p; }
 __device__ __forceinline__ const gdouble* gptr(const double* p) { return (const gdouble*)p; }
 
-// Stage one grid line of four coefficient arrays into LDS (element t at
-// p[i0 + t*st]) with a 64-lane workgroup.  Each lane issues its loads for
-// eight elements of all four arrays before its first LDS write, so a line
-// of up to 512 elements arrives in one memory round trip rather than one
-// per element and array.
-__device__ __forceinline__ void stage_line4(const double* a, const double* b, const double* c, const double* s,
-                                            long long i0, long long st, int n, double* la, double* lb, double* lc,
-                                            double* ls) {
-  for (int t0 = 0; t0 < n; t0 += 512) {
-    double ra[8], rb[8], rc[8], rs[8];
+// ------------------------------------------------- turbulence line solves
+// Tridiagonal line of n cells, a x(i-1) + b x(i) + c x(i+1) = s, solved in
+// parts of M cells, one lane per part (the turbulence models' line solves:
+// lsolvej / lsolvek and their two-equation forms).  The last cell of every
+// part is its separator.  Each lane eliminates its inner cells against the
+// separators on both sides, x(i) = S(i) + L(i) XL + R(i) XR; the separators'
+// own tridiagonal system (one row per part) is solved by parallel cyclic
+// reduction across the parts; the inner cells follow in parallel.  The
+// dependent chain is 2 M + log2(n / M) steps instead of n / 2 for an
+// elimination from both ends by two lanes, which bound these solves.
+// Parts depend on n alone, so every mapping of lines to workgroups gives the
+// same bits.  Quotients are corrected by one residual step (num - den q)
+// and sums use fused operations; against 80-bit solutions of 19200
+// diagonally dominant lines of 24 to 1000 cells the median relative error is
+// 0.9-2.4e-16 (from both ends 1.0-2.9e-16, one-sided 1.0-2.8e-16).
+// Cells past the line's end are identity rows; a of the first cell and c of
+// the last are zero.
+__host__ __device__ inline int part_cells(int n) { return n <= 512 ? 8 : (n <= 768 ? 12 : 16); }   // at most 64 parts
+
+__device__ __forceinline__ double quot(double num, double den, double r) {   // num / den, r = 1 / den
+  const double q = num * r;
+  return __builtin_fma(__builtin_fma(-den, q, num), r, q);
+}
+
+// inner cells 0 .. M-2: s, a, c become S, L, R
+template <int M>
+__device__ __forceinline__ void part_eliminate(double (&a)[M], const double (&b)[M], double (&c)[M], double (&s)[M]) {
+  {
+    const double r = 1. / b[0];
+    s[0] = quot(s[0], b[0], r);
+    a[0] = -quot(a[0], b[0], r);
+    c[0] = quot(c[0], b[0], r);
+  }
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int t = t0 + (int)threadIdx.x + 64 * u;
-      const long long i = i0 + (long long)(t < n ? t : n - 1) * st;
-      ra[u] = a[i]; rb[u] = b[i]; rc[u] = c[i]; rs[u] = s[i];
-    }
+  for (int i = 1; i < M - 1; ++i) {
+    const double ai = a[i], den = __builtin_fma(-ai, c[i - 1], b[i]);
+    const double r = 1. / den;
+    c[i] = quot(c[i], den, r);
+    s[i] = quot(__builtin_fma(-ai, s[i - 1], s[i]), den, r);
+    a[i] = -quot(ai * a[i - 1], den, r);
+  }
+  c[M - 2] = -c[M - 2];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int t = t0 + (int)threadIdx.x + 64 * u;
-      if (t < n) { la[t] = ra[u]; lb[t] = rb[u]; lc[t] = rc[u]; ls[t] = rs[u]; }
-    }
+  for (int i = M - 3; i >= 0; --i) {
+    const double ci = c[i];
+    s[i] = __builtin_fma(-ci, s[i + 1], s[i]);
+    a[i] = __builtin_fma(-ci, a[i + 1], a[i]);
+    c[i] = -ci * c[i + 1];
   }
 }
 
-// Thomas recurrence of one tridiagonal line held in LDS, run by one thread
-// with the reference's arithmetic (lsolvej / lsolvek and their two-equation
-// forms):
-//   forward   bb = 1/(b - a c'),  s' = (s - a s') bb,  c' = c bb
-//   backward  s' = s' - c' s'_next
-// s' and c' go to os and oc (os may be ls itself).  The recurrence runs in
-// chunks of THOMAS_CH cells whose LDS reads are issued a chunk ahead into
-// registers, so the dependent chain does not wait on LDS.  Chunk reads past
-// the line's end are clamped to its last cell and never used.  Cell t of the
-// line sits at index t*ST of each array (ST > 1: several lines interleaved,
-// one per lane).
-constexpr int THOMAS_CH = 8;
-template <int ST = 1>
-__device__ __forceinline__ void thomas_lds(const double* la, const double* lb, const double* lc, const double* ls,
-                                           double* os, double* oc, int n) {
-  constexpr int CH = THOMAS_CH;
-  double bb = 1. / lb[0];
-  double sp = ls[0] * bb, cp = lc[0] * bb;
-  os[0] = sp; oc[0] = cp;
-  double pa[CH], pb[CH], pc[CH], ps[CH], qa[CH], qb[CH], qc[CH], qs[CH];
-  auto ld = [&](double (&xa)[CH], double (&xb)[CH], double (&xc)[CH], double (&xs)[CH], int t) {
-#pragma unroll
-    for (int u = 0; u < CH; ++u) {
-      const int i = (t + u < n ? t + u : n - 1) * ST;
-      xa[u] = la[i]; xb[u] = lb[i]; xc[u] = lc[i]; xs[u] = ls[i];
-    }
-  };
-  auto run = [&](const double (&xa)[CH], const double (&xb)[CH], const double (&xc)[CH], const double (&xs)[CH],
-                 int t, int cnt) {
-#pragma unroll
-    for (int u = 0; u < CH; ++u) {
-      if (u < cnt) {
-        const double ai = xa[u];
-        bb = 1. / (xb[u] - ai * cp);
-        sp = (xs[u] - ai * sp) * bb;
-        cp = xc[u] * bb;
-        os[(t + u) * ST] = sp; oc[(t + u) * ST] = cp;
-      }
-    }
-  };
-  int t = 1;
-  ld(pa, pb, pc, ps, t);
-  for (; t + 2 * CH <= n; t += 2 * CH) {
-    ld(qa, qb, qc, qs, t + CH);
-    run(pa, pb, pc, ps, t, CH);
-    ld(pa, pb, pc, ps, t + 2 * CH);
-    run(qa, qb, qc, qs, t + CH, CH);
-  }
-  ld(qa, qb, qc, qs, t + CH);
-  run(pa, pb, pc, ps, t, n - t);
-  run(qa, qb, qc, qs, t + CH, n - t - CH);
-  // back substitution over cells n-2 .. 0, chunks of cells t-CH+1 .. t
-  double sn = sp;
-  double ys[CH], yc[CH], zs[CH], zc[CH];
-  auto ldb = [&](double (&xs)[CH], double (&xc)[CH], int t) {
-#pragma unroll
-    for (int u = 0; u < CH; ++u) {
-      const int i = (t - u >= 0 ? t - u : 0) * ST;
-      xs[u] = os[i]; xc[u] = oc[i];
-    }
-  };
-  auto runb = [&](const double (&xs)[CH], const double (&xc)[CH], int t, int cnt) {
-#pragma unroll
-    for (int u = 0; u < CH; ++u) {
-      if (u < cnt) {
-        sn = xs[u] - xc[u] * sn;
-        os[(t - u) * ST] = sn;
-      }
-    }
-  };
-  int b = n - 2;
-  ldb(ys, yc, b);
-  for (; b - 2 * CH + 1 >= 0; b -= 2 * CH) {
-    ldb(zs, zc, b - CH);
-    runb(ys, yc, b, CH);
-    ldb(ys, yc, b - 2 * CH);
-    runb(zs, zc, b - CH, CH);
-  }
-  ldb(zs, zc, b - CH);
-  runb(ys, yc, b, b + 1);
-  runb(zs, zc, b - CH, b - CH + 1);
+// the separator's row A X(p-1) + X(p) + C X(p+1) = D from the part's inner
+// cells and the next part's first cell (S, L, R)
+struct SepRow { double A, C, D; };
+template <int M>
+__device__ __forceinline__ SepRow part_separator(const double (&a)[M], const double (&b)[M], const double (&c)[M],
+                                                 const double (&s)[M], double Sn, double Ln, double Rn) {
+  const double am = a[M - 1], cm = c[M - 1];
+  const double den = __builtin_fma(am, c[M - 2], __builtin_fma(cm, Ln, b[M - 1]));
+  const double r = 1. / den;
+  SepRow o;
+  o.A = quot(am * a[M - 2], den, r);
+  o.C = quot(cm * Rn, den, r);
+  o.D = quot(__builtin_fma(-am, s[M - 2], __builtin_fma(-cm, Sn, s[M - 1])), den, r);
+  return o;
 }
 
-// Two-ended elimination of a tridiagonal line (the turbulence models' line
-// solves): with 32-cell tiles, ntile = ceil(n/32) and nr = floor(ntile/2)
-// (0 for ntile = 1), the right part is the last 32*nr cells and the left
-// part the first m = n - 32*nr:
-//   left  (t = 0 .. m-1, up):   bb = 1/(b - a c'),  s' = (s - a s') bb,  c' = c bb
-//   right (t = n-1 .. m, down): bb = 1/(b - c a'),  s' = (s - c s') bb,  a' = a bb
-// (the first cell of each side: bb = 1/b); at the meeting cells each side
-// takes x = (s' - c' s'_other) / (1 - c' c'_other) and substitutes back
-// towards its end, x = s' - c' x_next.  nr = 0 is the one-sided recurrence.
-constexpr int SAJ_TILE = 32;
-__device__ __forceinline__ void sa_split(int n, int& nr, int& m) {
-  const int ntile = (n + SAJ_TILE - 1) / SAJ_TILE;
-  nr = ntile >= 2 ? ntile / 2 : 0;
-  m = n - SAJ_TILE * nr;
+// one step of the cyclic reduction from the rows at distance d on both sides
+// (zero rows past the ends)
+__device__ __forceinline__ SepRow sep_reduce(const SepRow& x, const SepRow& m, const SepRow& p) {
+  const double den = __builtin_fma(-x.C, p.A, __builtin_fma(-x.A, m.C, 1.));
+  const double r = 1. / den;
+  SepRow o;
+  o.A = -quot(x.A * m.A, den, r);
+  o.C = -quot(x.C * p.C, den, r);
+  o.D = quot(__builtin_fma(-x.C, p.D, __builtin_fma(-x.A, m.D, x.D)), den, r);
+  return o;
 }
 
-// The two-ended elimination of one line in LDS, run by two lanes of one
-// wave, h = 0 (left) and h = 1 (right), lane numbers XM apart (nr > 0), or
-// by the h = 0 lane alone (nr = 0).  Cell t of the line sits at index t*ST.
-// s' and the solution go to os (which may be ls), c' / a' to oc.
-template <int ST, int XM>
-__device__ __forceinline__ void thomas2_lds(const double* la, const double* lb, const double* lc, const double* ls,
-                                            double* os, double* oc, int n, int h) {
-  constexpr int CH = THOMAS_CH;
-  int nr, m;
-  sa_split(n, nr, m);
-  const int cnt = h ? n - m : m;
-  const int i0 = (h ? n - 1 : 0) * ST, st = (h ? -1 : 1) * ST;   // index of step u: i0 + st*u
-  const double* lo = h ? lc : la;
-  const double* hi = h ? la : lc;
-  double bb = 1. / lb[i0];
-  double sp = ls[i0] * bb, cp = hi[i0] * bb;
-  os[i0] = sp; oc[i0] = cp;
-  double pa[CH], pb[CH], pc[CH], ps[CH], qa[CH], qb[CH], qc[CH], qs[CH];
-  auto ld = [&](double (&xa)[CH], double (&xb)[CH], double (&xc)[CH], double (&xs)[CH], int u0) {
+// x of the part's cells from its separators
+template <int M>
+__device__ __forceinline__ void part_expand(const double (&a)[M], const double (&c)[M], double (&s)[M], double XL,
+                                            double XR) {
 #pragma unroll
-    for (int u = 0; u < CH; ++u) {
-      const int i = i0 + st * (u0 + u < cnt ? u0 + u : cnt - 1);
-      xa[u] = lo[i]; xb[u] = lb[i]; xc[u] = hi[i]; xs[u] = ls[i];
-    }
-  };
-  auto run = [&](const double (&xa)[CH], const double (&xb)[CH], const double (&xc)[CH], const double (&xs)[CH],
-                 int u0, int k) {
+  for (int i = 0; i < M - 1; ++i) s[i] = __builtin_fma(c[i], XR, __builtin_fma(a[i], XL, s[i]));
+  s[M - 1] = XR;
+}
+
+// One line of contiguous cells by one wave (lane = part): the four arrays
+// come in coalesced and pass through LDS (`buf`, PART_BUF doubles) to the
+// lanes' parts, then y = x * b goes back the same way into s.
+constexpr int PART_BUF = 64 * 18;
+template <int M>
+__device__ __forceinline__ void part_line_wave(const gdouble* ga, const gdouble* gb, const gdouble* gc, gdouble* gs,
+                                               int n, double* buf) {
+  constexpr int LD = M + 2;   // a lane's cells in LDS: 16-byte reads, no bank conflicts
+  typedef double d2_t __attribute__((ext_vector_type(2)));
+  const int l = threadIdx.x & 63;
+  const int P = (n + M - 1) / M;
+  double v[4][M];
 #pragma unroll
-    for (int u = 0; u < CH; ++u) {
-      if (u < k) {
-        const double ai = xa[u];
-        bb = 1. / (xb[u] - ai * cp);
-        sp = (xs[u] - ai * sp) * bb;
-        cp = xc[u] * bb;
-        const int i = i0 + st * (u0 + u);
-        os[i] = sp; oc[i] = cp;
-      }
-    }
-  };
-  int u = 1;
-  ld(pa, pb, pc, ps, u);
-  for (; u + 2 * CH <= cnt; u += 2 * CH) {
-    ld(qa, qb, qc, qs, u + CH);
-    run(pa, pb, pc, ps, u, CH);
-    ld(pa, pb, pc, ps, u + 2 * CH);
-    run(qa, qb, qc, qs, u + CH, CH);
+  for (int u = 0; u < M; ++u) {
+    const int e = l + 64 * u, ec = e < n ? e : n - 1;
+    v[0][u] = ga[ec]; v[1][u] = gb[ec]; v[2][u] = gc[ec]; v[3][u] = gs[ec];
   }
-  ld(qa, qb, qc, qs, u + CH);
-  run(pa, pb, pc, ps, u, cnt - u);
-  run(qa, qb, qc, qs, u + CH, cnt - u - CH);
-  // the meeting cells
-  double sn = sp;
-  if (nr > 0) {
-    const double so = __shfl_xor(sp, XM), co = __shfl_xor(cp, XM);
-    sn = (sp - cp * so) / (1. - cp * co);
-  }
-  os[i0 + st * (cnt - 1)] = sn;
-  // back substitution towards this side's end, chunks of CH steps
-  double ys[CH], yc[CH], zs[CH], zc[CH];
-  auto ldb = [&](double (&xs)[CH], double (&xc)[CH], int u1) {
 #pragma unroll
-    for (int v = 0; v < CH; ++v) {
-      const int i = i0 + st * (u1 - v >= 0 ? u1 - v : 0);
-      xs[v] = os[i]; xc[v] = oc[i];
-    }
-  };
-  auto runb = [&](const double (&xs)[CH], const double (&xc)[CH], int u1, int k) {
-#pragma unroll
-    for (int v = 0; v < CH; ++v) {
-      if (v < k) {
-        sn = xs[v] - xc[v] * sn;
-        os[i0 + st * (u1 - v)] = sn;
-      }
-    }
-  };
-  int b = cnt - 2;
-  ldb(ys, yc, b);
-  for (; b - 2 * CH + 1 >= 0; b -= 2 * CH) {
-    ldb(zs, zc, b - CH);
-    runb(ys, yc, b, CH);
-    ldb(ys, yc, b - 2 * CH);
-    runb(zs, zc, b - CH, CH);
+  for (int u = 0; u < M; ++u) {
+    const int e = l + 64 * u;
+    if (e >= n) { v[0][u] = 0.; v[1][u] = 1.; v[3][u] = 0.; }
+    if (e == 0) v[0][u] = 0.;
+    if (e >= n - 1) v[2][u] = 0.;
   }
-  ldb(zs, zc, b - CH);
-  runb(ys, yc, b, b + 1);
-  runb(zs, zc, b - CH, b - CH + 1);
+  // one wave's LDS operations run in order: no barrier
+  auto transpose = [&](double (&x)[M]) {
+#pragma unroll
+    for (int u = 0; u < M; ++u) {
+      const int e = l + 64 * u;
+      buf[e / M * LD + e % M] = x[u];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+    for (int u = 0; u < M; u += 2) {
+      const d2_t t = *reinterpret_cast<const d2_t*>(buf + l * LD + u);
+      x[u] = t.x; x[u + 1] = t.y;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  };
+#pragma unroll
+  for (int q = 0; q < 4; ++q) transpose(v[q]);
+  double (&a)[M] = v[0], (&b)[M] = v[1], (&c)[M] = v[2], (&s)[M] = v[3];
+  part_eliminate<M>(a, b, c, s);
+  auto down = [&](double x, int d) { const double y = __shfl_down(x, d); return l + d < 64 ? y : 0.; };
+  auto up = [&](double x, int d) { const double y = __shfl_up(x, d); return l >= d ? y : 0.; };
+  SepRow w = part_separator<M>(a, b, c, s, down(s[0], 1), down(a[0], 1), down(c[0], 1));
+  for (int d = 1; d < P; d <<= 1) {
+    const SepRow m = {up(w.A, d), up(w.C, d), up(w.D, d)}, p = {down(w.A, d), down(w.C, d), down(w.D, d)};
+    w = sep_reduce(w, m, p);
+  }
+  part_expand<M>(a, c, s, up(w.D, 1), w.D);
+#pragma unroll
+  for (int u = 0; u < M; ++u) s[u] = (0. + s[u] - 0.) * b[u];
+#pragma unroll
+  for (int u = 0; u < M; u += 2) *reinterpret_cast<d2_t*>(buf + l * LD + u) = d2_t{s[u], s[u + 1]};
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+  for (int u = 0; u < M; ++u) {
+    const int e = l + 64 * u;
+    if (e < n) gs[e] = buf[e / M * LD + e % M];
+  }
+}
+__device__ __forceinline__ void part_line(const gdouble* a, const gdouble* b, const gdouble* c, gdouble* s, int n,
+                                          double* buf) {
+  switch (part_cells(n)) {
+    case 8: part_line_wave<8>(a, b, c, s, n, buf); break;
+    case 12: part_line_wave<12>(a, b, c, s, n, buf); break;
+    default: part_line_wave<16>(a, b, c, s, n, buf); break;
+  }
+}
+
+// TC adjacent columns of n <= 512 rows by one workgroup: thread (column c =
+// tid % TC, part p = tid / TC) holds rows 8p .. 8p+7 of its column, so every
+// load of a wave is whole row segments of TC cells.  The separators' rows
+// pass between the parts through LDS (`ex`, two buffers of 3 x threads).
+// On return s holds x.  Every thread of the workgroup calls it.
+constexpr int PCOL_M = 8;
+template <int TC>
+__device__ __forceinline__ void part_columns(double (&a)[PCOL_M], const double (&b)[PCOL_M], double (&c)[PCOL_M],
+                                             double (&s)[PCOL_M], int P, double* ex) {
+  constexpr int M = PCOL_M;
+  const int nt = blockDim.x, tid = threadIdx.x, p = tid / TC;
+  part_eliminate<M>(a, b, c, s);
+  double* e0 = ex;
+  double* e1 = ex + 3 * nt;
+  auto post = [&](double x, double y, double z) { e0[tid] = x; e0[nt + tid] = y; e0[2 * nt + tid] = z; };
+  auto at = [&](int q) -> SepRow {   // the row of part q of this column
+    const int o = tid + (q - p) * TC;
+    const bool in = q >= 0 && q < P;
+    const int oc = in ? o : tid;
+    const double x = e0[oc], y = e0[nt + oc], z = e0[2 * nt + oc];
+    return {in ? x : 0., in ? y : 0., in ? z : 0.};
+  };
+  auto swap = [&]() { double* t = e0; e0 = e1; e1 = t; };
+  post(s[0], a[0], c[0]);
+  __syncthreads();
+  const SepRow nx = at(p + 1);
+  swap();
+  SepRow w = part_separator<M>(a, b, c, s, nx.A, nx.C, nx.D);
+  for (int d = 1; d < P; d <<= 1) {
+    post(w.A, w.C, w.D);
+    __syncthreads();
+    const SepRow m = at(p - d), q = at(p + d);
+    swap();
+    w = sep_reduce(w, m, q);
+  }
+  e0[tid] = w.D;
+  __syncthreads();
+  const double XL = p > 0 ? e0[tid - TC] : 0.;
+  swap();
+  part_expand<M>(a, c, s, XL, w.D);
 }
 
 constexpr int RES_TJ = 32;
@@ -453,7 +443,7 @@ hipError_t launch_rbc(const DevMesh* dM, int nmi, hipStream_t st);
 constexpr int LU32_SWEEP_VARIANTS = 3;   // FP32 sweep instantiations (ring steps, producers, prefetch)
 struct LaunchCfg {
   int sweep = 0;     // 0: 12 ring steps, 3 producers; 1: 18, 3; 2: 12, 4 (with deeper prefetch)
-  int sa_lane = -1;  // SA line solves: -1 by the number of lines, 0 one wave per line, 1 one lane per line
+  int sa_lane = -1;  // SA k solves: columns per workgroup, 0: 16, 1: 8, -1 by the number of columns
 };
 // fuse_update: 1 the q update and monitor in k_lu_finish (Euler), | 2
 // k_lu_finish also leaves the SA model's laminar viscosity and velocities

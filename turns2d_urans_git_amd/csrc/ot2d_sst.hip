@@ -11,10 +11,9 @@
 //   k_sst_rhs                    komegarhslhs (464-903) in gather form: each
 //                                interior cell assembles its rows of the four
 //                                tridiagonal systems, scaled by the pseudo time step
-//   k_sst_solve_j / _k           lsolvej2 / lsolvek2 (1435-1518), one wave per
-//                                line and equation; the k solve applies the update
-//                                with its clip (146-172)
-//   k_sst_turm                   findturm after the update
+//   k_sst_solve_j / _k           lsolvej2 / lsolvek2 (1435-1518), lines solved in
+//                                parts; the k solve applies the update with its
+//                                clip (146-172) and findturm after it
 //
 // The reference reads F1, F2 and strain on the halo ring without writing
 // them there (blend and kwvortic fill the interior only; findturm and
@@ -386,80 +385,80 @@ __global__ __launch_bounds__(256) void k_sst_rhs(const DevMesh* __restrict__ Ms)
   }
 }
 
-// lsolvej2 / lsolvek2 of one line held in LDS, eliminated from both ends
-// (lanes 0 and 1; the reference's one-sided recurrence for lines of up to
-// 32 cells); on return ls holds the solution
-__device__ __forceinline__ void kw_line_solve(const double* la, const double* lb, const double* lc, double* ls,
-                                              double* lcp, int n) {
-  int nr, m;
-  sa_split(n, nr, m);
-  if (threadIdx.x >= (nr > 0 ? 2u : 1u)) return;
-  thomas2_lds<1, 1>(la, lb, lc, ls, ls, lcp, n, (int)threadIdx.x);
-}
-
-// lsolvej2 for k row blockIdx.x / 2, equation blockIdx.x % 2, then
-// sjmat = sjmat * bjmat (src/komegasst.f:133-140)
+// lsolvej2 for k row blockIdx.x / 2, equation blockIdx.x % 2, in parts by one
+// wave, then sjmat = sjmat * bjmat (src/komegasst.f:133-140).  301x90: 5.2 us
+// (two lanes per line 25), 385x97 with 401x401: 8.6 (54)
 __global__ __launch_bounds__(64) void k_sst_solve_j(const DevMesh* __restrict__ Ms) {
-  __shared__ double la[SA_LINE_MAX], lb[SA_LINE_MAX], lc[SA_LINE_MAX], ls[SA_LINE_MAX], lcp[SA_LINE_MAX];
+  __shared__ __attribute__((aligned(16))) double buf[PART_BUF];
   const DevMesh& M = Ms[blockIdx.y];
   if (*M.status) return;
   const int eq = blockIdx.x & 1;
   const int k = M.ks + (blockIdx.x >> 1);
   if (k > M.ke) return;
-  const int n = M.je - M.js + 1;
   const long long i0 = cell(M, M.js, k);
-  double* __restrict__ s = M.kw_s[eq];
-  const double* __restrict__ a = M.kw_a[eq];
-  const double* __restrict__ b = M.kw_b[eq];
-  const double* __restrict__ c = M.kw_c[eq];
-  stage_line4(a, b, c, s, i0, 1, n, la, lb, lc, ls);
-  __syncthreads();
-  kw_line_solve(la, lb, lc, ls, lcp, n);
-  __syncthreads();
-  for (int t = threadIdx.x; t < n; t += 64) s[i0 + t] = ls[t] * lb[t];
+  part_line(gptr(M.kw_a[eq]) + i0, gptr(M.kw_b[eq]) + i0, gptr(M.kw_c[eq]) + i0, gptr(M.kw_s[eq]) + i0,
+            M.je - M.js + 1, buf);
 }
 
-// lsolvek2 for j column blockIdx.x / 2, equation blockIdx.x % 2, then the
-// update of that equation with its clip (src/komegasst.f:146-172)
-__global__ __launch_bounds__(64) void k_sst_solve_k(const DevMesh* __restrict__ Ms) {
-  __shared__ double la[SA_LINE_MAX], lb[SA_LINE_MAX], lc[SA_LINE_MAX], ls[SA_LINE_MAX], lcp[SA_LINE_MAX];
+// lsolvek2 of both equations for TC adjacent j columns (blockIdx.x), one half
+// of the threads per equation, their update with its clip
+// (src/komegasst.f:146-172) and findturm for the interior after it (the halo
+// ring follows the final komegabc in k_sst_bc).  301x90: 10.6 us, 385x97
+// with 401x401: 24.6 us (one wave per line and equation from both ends, and
+// findturm in a pass of its own: 25 and 75 us).
+template <int TC>
+__global__ __launch_bounds__(512) void k_sst_solve_k(const DevMesh* __restrict__ Ms) {
+  extern __shared__ __attribute__((aligned(16))) double sst_ex[];
+  constexpr int PM = PCOL_M;
   const DevMesh& M = Ms[blockIdx.y];
   if (*M.status) return;
-  const int eq = blockIdx.x & 1;
-  const int j = M.js + (blockIdx.x >> 1);
-  if (j > M.je) return;
-  const int n = M.ke - M.ks + 1;
-  const long long i0 = cell(M, j, M.ks), st = M.jd;
-  const double* __restrict__ s = M.kw_s[eq];
-  const double* __restrict__ a = M.kw_ak[eq];
-  const double* __restrict__ b = M.kw_b[eq];
-  const double* __restrict__ c = M.kw_ck[eq];
-  stage_line4(a, b, c, s, i0, st, n, la, lb, lc, ls);
-  __syncthreads();
-  kw_line_solve(la, lb, lc, ls, lcp, n);
-  __syncthreads();
-  double* qn = M.q[4 + eq];
-  double* sn = M.s[4 + eq];
-  for (int t = threadIdx.x; t < n; t += 64) {
-    long long i = i0 + t * st;
-    double ds = 1. * ls[t];
-    sn[i] = ds;
-    double q = qn[i] + ds * (double)imk(M.iblank[i], 0);
-    qn[i] = dmax(q, 1e-20 * rho_of(M, i));
+  const int j0 = M.js + (int)blockIdx.x * TC;
+  if (j0 > M.je) return;
+  // thread (column, equation, part): both equations of a column exchange
+  // through the same calls, as 2*TC columns
+  const int n = M.ke - M.ks + 1, P = (n + PM - 1) / PM, tid = (int)threadIdx.x;
+  const int eq = (tid / TC) & 1;
+  const int j = j0 + tid % TC, k0 = (tid / (2 * TC)) * PM;
+  const bool col = j <= M.je;
+  const long long st = M.jd, i0 = cell(M, col ? j : M.je, M.ks);
+  const gdouble *ga = gptr(eq ? M.kw_ak[1] : M.kw_ak[0]), *gb = gptr(eq ? M.kw_b[1] : M.kw_b[0]),
+                *gc = gptr(eq ? M.kw_ck[1] : M.kw_ck[0]), *gs = gptr(eq ? M.kw_s[1] : M.kw_s[0]);
+  const gdouble *gq = gptr(eq ? M.q[5] : M.q[4]), *g1 = gptr(M.q[0]), *gj = gptr(M.q[M.nq - 1]);
+  double a[PM], b[PM], c[PM], s[PM], q[PM], q1[PM], qj[PM];
+  int ib[PM];
+#pragma unroll
+  for (int u = 0; u < PM; ++u) {
+    const long long i = i0 + (long long)(k0 + u < n ? k0 + u : n - 1) * st;
+    a[u] = ga[i]; b[u] = gb[i]; c[u] = gc[i]; s[u] = gs[i];
   }
-}
-
-// findturm for the interior after the update (the halo ring follows the
-// final komegabc in k_sst_bc)
-__global__ __launch_bounds__(256) void k_sst_turm(const DevMesh* __restrict__ Ms) {
-  const DevMesh& M = Ms[blockIdx.y];
-  if (*M.status) return;
-  const int js = M.js, je = M.je, ks = M.ks, ke = M.ke;
-  const int nj = je - js + 1, nk = ke - ks + 1;
-  long long ncell = (long long)nj * nk;
-  for (long long w = blockIdx.x * 256ll + threadIdx.x; w < ncell; w += 256ll * gridDim.x) {
-    const long long i = cell(M, js + (int)(w % nj), ks + (int)(w / nj));
-    M.turmu[i] = findturm(rho_of(M, i), M.q[4][i], M.q[5][i], M.kw_x[i]);
+#pragma unroll
+  for (int u = 0; u < PM; ++u) {
+    const int k = k0 + u;
+    if (k >= n) { a[u] = 0.; b[u] = 1.; s[u] = 0.; }
+    if (k == 0) a[u] = 0.;
+    if (k >= n - 1) c[u] = 0.;
+  }
+  // the update's operands, ahead of the solve
+#pragma unroll
+  for (int u = 0; u < PM; ++u) {
+    const long long i = i0 + (long long)(k0 + u < n ? k0 + u : n - 1) * st;
+    q[u] = gq[i]; q1[u] = g1[i]; qj[u] = gj[i]; ib[u] = M.iblank[i];
+  }
+  part_columns<2 * TC>(a, b, c, s, P, sst_ex);
+  double* qn = eq ? M.q[5] : M.q[4];
+  double* sn = eq ? M.s[5] : M.s[4];
+#pragma unroll
+  for (int u = 0; u < PM; ++u) {
+    const double ds = 1. * s[u];
+    const double rho = q1[u] * qj[u];
+    q[u] = dmax(q[u] + ds * (double)imk(ib[u], 0), 1e-20 * rho);
+    // findturm takes the other equation's value from its lane
+    const double qo = __shfl_xor(q[u], TC);
+    if (!col || k0 + u >= n) continue;
+    const long long i = i0 + (long long)(k0 + u) * st;
+    sn[i] = ds;
+    qn[i] = q[u];
+    if (eq == 0) M.turmu[i] = findturm(rho, q[u], qo, M.kw_x[i]);
   }
 }
 
@@ -467,6 +466,9 @@ static inline int nblk3(long long n, int per) {
   long long b = (n + per - 1) / per;
   return (int)(b < 1 ? 1 : (b > 4096 ? 4096 : b));
 }
+
+// parts of the longest column up to which 8 columns fit 512 threads (beyond: 4)
+constexpr int SSTK_NP8 = 32;
 
 // komegasst for every instance (src/komegasst.f:2-187)
 hipError_t launch_sst(const DevMesh* dM, const DevMesh* hM, int nmi, Marks* mk, hipStream_t st) {
@@ -491,12 +493,18 @@ hipError_t launch_sst(const DevMesh* dM, const DevMesh* hM, int nmi, Marks* mk, 
   hipLaunchKernelGGL(k_sst_solve_j, dim3(2 * mk_, nmi), dim3(64), 0, st, dM);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_SA_SOLVE_J, st);
-  hipLaunchKernelGGL(k_sst_solve_k, dim3(2 * mj, nmi), dim3(64), 0, st, dM);
+  {
+    const int np = (mk_ + PCOL_M - 1) / PCOL_M;   // parts of the longest column
+    auto solve_k = [&](auto kern, int tc) {
+      const int nt = (2 * np * tc + 63) / 64 * 64;
+      hipLaunchKernelGGL(kern, dim3((mj + tc - 1) / tc, nmi), dim3(nt), sizeof(double) * 6 * nt, st, dM);
+    };
+    if (np <= SSTK_NP8) solve_k(k_sst_solve_k<8>, 8);
+    else solve_k(k_sst_solve_k<4>, 4);
+  }
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_SA_SOLVE_K, st);
   hipLaunchKernelGGL(k_sst_bc, dim3(nmi), dim3(BC_THREADS), 0, st, dM, 1);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
-  hipLaunchKernelGGL(k_sst_turm, dim3(nblk3(mx, 256), nmi), dim3(256), 0, st, dM);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_SA_EDDY, st);
   return hipSuccess;

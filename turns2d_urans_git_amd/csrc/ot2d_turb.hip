@@ -12,17 +12,15 @@
 //                                      k_sa_rhs      convection, diffusion, source and the
 //                                                    two scalar tridiagonal systems, in
 //                                                    gather form (one thread per cell)
-//                                      k_sa_solve_j  tridiagonal solve along j from both ends
-//                                                    (two lanes per k row)
-//                                      k_sa_solve_kt tridiagonal solves along k, 16 or 8 adjacent
-//                                                    j columns per workgroup (k_sa_solve_k: one
-//                                                    column, for lines over 256 cells),
-//                                                    nu-tilde update and eddy viscosity
+//                                      k_sa_solve_j  tridiagonal solve along j, one wave per row
+//                                      k_sa_solve_k  tridiagonal solve along k, 8 or 16 adjacent
+//                                                    j columns per workgroup, nu-tilde update and
+//                                                    eddy viscosity
 //
 // Operand order follows the reference expressions (built with
 // -ffp-contract=off), so results agree with the reference to the rounding of
-// the device's sqrt/div/pow; the line solves of lines over 32 cells run from
-// both ends (thomas2_lds), which changes their rounding only.
+// the device's sqrt/div/pow; the line solves run in parts (part_line,
+// part_columns), which changes their rounding only.
 #include "ot2d_dev.h"
 
 namespace ot2d {
@@ -709,601 +707,75 @@ __global__ __launch_bounds__(256) void k_sa_rhs(const DevMesh* __restrict__ Ms) 
   }
 }
 
-// The two scalar tridiagonal solves of vmu_sa are sequential recurrences
-// along each grid line, both eliminated from the line's two ends at once
-// (thomas2_lds), which halves the dependent chain; lines of up to 32 cells
-// keep the reference's one-sided recurrence (lsolvej / lsolvek).  One wave
-// owns one line: all lanes stage the line's coefficients in LDS (stage_line4:
-// every load in flight at once, coalesced along j, gathered along k), two
-// lanes run the two sides out of LDS (reads a chunk ahead of the dependent
-// chain), and all lanes write the results.  The wave, tile and lane kernels
-// of a direction evaluate the same operations in the same order, so every
-// mapping gives bit-identical results; against the one-sided recurrence the
-// results differ in rounding only.
-// lsolvej (src/samodel2d.f:1306-1344), eliminated from both ends, and s1,
-// sjmat*bjmat of vmu_sa (src/samodel2d.f:148-152) for the k row blockIdx.x
+// The two scalar tridiagonal solves of vmu_sa (lsolvej, lsolvek), each line
+// solved in parts (part_line, part_columns).
+// lsolvej (src/samodel2d.f:1306-1344) and s1, sjmat*bjmat of vmu_sa
+// (src/samodel2d.f:148-152) for the k row blockIdx.x, one wave.
+// Bound by one memory round trip and the parts' chain at one case (513x129:
+// 5.5 us; by two lanes from both ends out of LDS 37 us), by HBM in a batch
+// (60 cases, 3.9 M cells, 40 bytes a cell: 36 us; one lane per line side, 99 us).
 __global__ __launch_bounds__(64) void k_sa_solve_j(const DevMesh* __restrict__ Ms) {
-  __shared__ double la[SA_LINE_MAX], lb[SA_LINE_MAX], lc[SA_LINE_MAX], ls[SA_LINE_MAX];
-  __shared__ double lcp[SA_LINE_MAX], lsp[SA_LINE_MAX];
+  __shared__ __attribute__((aligned(16))) double buf[PART_BUF];
   const DevMesh& M = Ms[blockIdx.y];
   if (*M.status) return;
-  const int js = M.js, je = M.je;
   const int k = M.ks + blockIdx.x;
   if (k > M.ke) return;
-  const int n = je - js + 1;
-  const long long i0 = cell(M, js, k);
-  double* __restrict__ s = M.sa_sj;
-  const double* __restrict__ c = M.sa_cj;
-  const double* __restrict__ a = M.sa_aj;
-  const double* __restrict__ b = M.sa_bb;
-  stage_line4(a, b, c, s, i0, 1, n, la, lb, lc, ls);
-  __syncthreads();
-  int nr, m;
-  sa_split(n, nr, m);
-  if (threadIdx.x < (nr > 0 ? 2u : 1u)) thomas2_lds<1, 1>(la, lb, lc, ls, lsp, lcp, n, (int)threadIdx.x);
-  __syncthreads();
-  // sjmat = (s1 - s2) * bjmat with s2 = 0
-  for (int t = threadIdx.x; t < n; t += 64) s[i0 + t] = (0. + lsp[t] - 0.) * lb[t];
+  const long long i0 = cell(M, M.js, k);
+  part_line(gptr(M.sa_aj) + i0, gptr(M.sa_bb) + i0, gptr(M.sa_cj) + i0, gptr(M.sa_sj) + i0, M.je - M.js + 1, buf);
 }
 
 // lsolvek (src/samodel2d.f:1347-1385), s2 and the nu-tilde update with its
 // clip (src/samodel2d.f:157-188), then the interior eddy viscosity (c_turm)
-// for the j column blockIdx.x
-__global__ __launch_bounds__(64) void k_sa_solve_k(const DevMesh* __restrict__ Ms, int ovl) {
-  __shared__ double la[SA_LINE_MAX], lb[SA_LINE_MAX], lc[SA_LINE_MAX], ls[SA_LINE_MAX];
-  __shared__ double lcp[SA_LINE_MAX], lsp[SA_LINE_MAX];
+// for TC adjacent j columns: 16 make whole 128-byte row segments for batches
+// (60 cases 113 us, 8 columns 137; lane per line and an update pass of its
+// own 125), 8 twice the workgroups for few columns (513x129: 8.9 us, 16
+// columns 9.6; two lanes per column from both ends 17.4).
+constexpr int SAK_NT = 512;
+template <int TC>
+__global__ __launch_bounds__(SAK_NT) void k_sa_solve_k(const DevMesh* __restrict__ Ms, int ovl) {
+  extern __shared__ __attribute__((aligned(16))) double sak_ex[];
+  constexpr int PM = PCOL_M;
   const DevMesh& M = Ms[blockIdx.y];
   if (*M.status) return;
-  const int ks = M.ks, ke = M.ke;
-  const int j = M.js + blockIdx.x;
-  if (j > M.je) return;
-  const int n = ke - ks + 1;
-  const long long i0 = cell(M, j, ks);
-  const long long st = M.jd;
-  const double* __restrict__ s = M.sa_sj;
-  const double* __restrict__ c = M.sa_ck;
-  const double* __restrict__ a = M.sa_ak;
-  const double* __restrict__ b = M.sa_bb;
-  stage_line4(a, b, c, s, i0, st, n, la, lb, lc, ls);
-  __syncthreads();
-  int nr, m;
-  sa_split(n, nr, m);
-  if (threadIdx.x < (nr > 0 ? 2u : 1u)) thomas2_lds<1, 1>(la, lb, lc, ls, lsp, lcp, n, (int)threadIdx.x);
-  __syncthreads();
-  const double vnulim = 1.0e-20, relfac = 1.0;
-  for (int t = threadIdx.x; t < n; t += 64) {
-    long long i = i0 + t * st;
-    double dq = relfac * (0. + lsp[t]);
-    double q5 = M.q[4][i];
-    q5 = fmax((q5 + dq * (double)imx(M.iblank[i], 0)), vnulim);
-    M.q[4][i] = q5;
-    c_turm_cell(M, i, ovl);
-  }
-}
-
-// lsolvek, the nu-tilde update and c_turm for TJ adjacent j columns
-// (blockIdx.x) at once, for lines of up to nmax cells: the workgroup (32*TJ
-// threads) stages the TJ k lines as rows of TJ consecutive cells (each row one
-// TJ*8-byte run, where the one-line kernel gathers one element per cache
-// line; TJ = 16 makes each run a whole 128-byte line), lanes 0..TJ-1 of wave
-// 0 run the TJ recurrences out of LDS (column c at stride TJ), and all
-// threads apply the update and the eddy viscosity, a few cells each with
-// their loads issued together.  Columns past je stage a harmless b = 1 row
-// and are never written.  LDS: five arrays of nmax*TJ doubles (dynamic).
-constexpr int SAK_TJ = 8, SAK_NMAX = 256;
-constexpr int SAK_TJ16 = 16, SAK_NMAX16 = 192;   // 16 columns for lines of up to 192 cells
-template <int TJ>
-__global__ __launch_bounds__(32 * TJ) void k_sa_solve_kt(const DevMesh* __restrict__ Ms, int ovl, int nmax) {
-  extern __shared__ __attribute__((aligned(16))) double sak_lds[];
-  double* const la = sak_lds;
-  double* const lb = la + (size_t)nmax * TJ;
-  double* const lc = lb + (size_t)nmax * TJ;
-  double* const ls = lc + (size_t)nmax * TJ;
-  double* const lcp = ls + (size_t)nmax * TJ;
-  const DevMesh& M = Ms[blockIdx.y];
-  if (*M.status) return;
-  const int ks = M.ks, ke = M.ke;
-  const int j0 = M.js + (int)blockIdx.x * TJ;
+  const int j0 = M.js + (int)blockIdx.x * TC;
   if (j0 > M.je) return;
-  const int n = ke - ks + 1;
-  const int ne = n * TJ;
-  constexpr int NT = 32 * TJ;   // threads
-  const int tid = (int)threadIdx.x;
-  const double* __restrict__ s = M.sa_sj;
-  const double* __restrict__ c = M.sa_ck;
-  const double* __restrict__ a = M.sa_ak;
-  const double* __restrict__ b = M.sa_bb;
-  // element e = k*TJ + col of the tile; 4 elements per thread in flight at once
-  constexpr int U = 4;
-  for (int e0 = 0; e0 < ne; e0 += NT * U) {
-    double ra[U], rb[U], rc[U], rs[U];
+  const int n = M.ke - M.ks + 1, P = (n + PM - 1) / PM;
+  const int j = j0 + (int)threadIdx.x % TC, k0 = ((int)threadIdx.x / TC) * PM;
+  const bool col = j <= M.je;
+  const long long st = M.jd, i0 = cell(M, col ? j : M.je, M.ks);
+  const gdouble *ga = gptr(M.sa_ak), *gb = gptr(M.sa_bb), *gc = gptr(M.sa_ck), *gs = gptr(M.sa_sj);
+  double a[PM], b[PM], c[PM], s[PM];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int e = e0 + tid + NT * u;
-      const int j = j0 + (e & (TJ - 1));
-      const int k = ks + (e < ne ? e : ne - 1) / TJ;
-      const long long i = cell(M, j <= M.je ? j : M.je, k);
-      ra[u] = a[i]; rb[u] = b[i]; rc[u] = c[i]; rs[u] = s[i];
-    }
+  for (int u = 0; u < PM; ++u) {
+    const long long i = i0 + (long long)(k0 + u < n ? k0 + u : n - 1) * st;
+    a[u] = ga[i]; b[u] = gb[i]; c[u] = gc[i]; s[u] = gs[i];
+  }
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int e = e0 + tid + NT * u;
-      if (e < ne) {
-        const bool in = j0 + (e & (TJ - 1)) <= M.je;
-        la[e] = in ? ra[u] : 0.0; lb[e] = in ? rb[u] : 1.0; lc[e] = in ? rc[u] : 0.0; ls[e] = in ? rs[u] : 0.0;
-      }
-    }
+  for (int u = 0; u < PM; ++u) {
+    const int k = k0 + u;
+    if (k >= n) { a[u] = 0.; b[u] = 1.; s[u] = 0.; }
+    if (k == 0) a[u] = 0.;
+    if (k >= n - 1) c[u] = 0.;
   }
-  __syncthreads();
-  {
-    // column tid & 31 of the tile, side tid >> 5 (lanes 0..TJ-1 and 32..32+TJ-1 of wave 0)
-    int nr, m;
-    sa_split(n, nr, m);
-    const int cl = tid & 31, sd = tid >> 5;
-    if (cl < TJ && (sd == 0 || (sd == 1 && nr > 0)))
-      thomas2_lds<TJ, 32>(la + cl, lb + cl, lc + cl, ls + cl, ls + cl, lcp + cl, n, sd);
-  }
-  __syncthreads();
-  // the update and c_turm, U cells per thread with all their loads issued
-  // before the first store
+  // the update's operands, ahead of the solve
   const double vnulim = 1.0e-20, relfac = 1.0;
-  for (int e0 = 0; e0 < ne; e0 += NT * U) {
-    long long ii[U];
-    bool ok[U];
-    double q5[U], q1[U], qj[U], vm[U], ib[U];
+  const gdouble *g5 = gptr(M.q[4]), *g1 = gptr(M.q[0]), *gj = gptr(M.q[M.nq - 1]), *gv = gptr(M.sa_vmul);
+  double q5[PM], q1[PM], qj[PM], vm[PM];
+  int ib[PM];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int e = e0 + tid + NT * u;
-      const int j = j0 + (e & (TJ - 1));
-      ok[u] = e < ne && j <= M.je;
-      ii[u] = cell(M, j <= M.je ? j : M.je, ks + (e < ne ? e : ne - 1) / TJ);
-      q5[u] = M.q[4][ii[u]]; q1[u] = M.q[0][ii[u]]; qj[u] = M.q[M.nq - 1][ii[u]]; vm[u] = M.sa_vmul[ii[u]];
-      ib[u] = (double)imx(M.iblank[ii[u]], 0);
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (!ok[u]) continue;
-      const int e = e0 + tid + NT * u;
-      double dq = relfac * (0. + ls[e]);
-      const double v = fmax((q5[u] + dq * ib[u]), vnulim);
-      M.q[4][ii[u]] = v;
-      put_turm(M, ii[u], q1[u], qj[u], vm[u], v, ovl);
-    }
+  for (int u = 0; u < PM; ++u) {
+    const long long i = i0 + (long long)(k0 + u < n ? k0 + u : n - 1) * st;
+    q5[u] = g5[i]; q1[u] = g1[i]; qj[u] = gj[i]; vm[u] = gv[i]; ib[u] = M.iblank[i];
   }
-}
-
-// Line solves for many lines at once: one lane per line (along j: one lane
-// per side of a line), the same arithmetic as the one-wave kernels.
-// k_sa_lines_j: lines along j (one per k row), 32 rows per workgroup, lane
-// l = 32h + r of wave 0 running side h of row r's two-ended elimination
-// (h = 0 the left part from j = js, h = 1 the right part from j = je).
-// Each side is cut into 32-cell tiles, counted from its own end; tile x of
-// side 1 is stored reversed (position p holds cell n-1-32x-p), so both
-// sides walk positions upwards in the elimination and downwards in the
-// back substitution.  Waves 1..SAJ_MW move the tiles (row-contiguous
-// segments) between global memory and two LDS slots: while wave 0 works on
-// tile x in one slot, the movers write tile x-1's results back from the
-// other slot and refill it with tile x+1, whose loads they issued SAJ_D
-// tiles earlier, so the recurrences do not wait on memory.  The elimination
-// leaves s' and c' (a' on the right) in place, the back substitution writes
-// s = (s1 - s2) * bjmat.
-constexpr int SA_TJ = SAJ_TILE, SAJ_MW = 4, SAJ_D = 2;
-constexpr int SAJ_THREADS = 64 * (1 + SAJ_MW);
-constexpr int SAJ_PER = 64 * SA_TJ / (64 * SAJ_MW);   // elements per mover lane and array
-// total lines (both directions, all instances) above which the solves run one lane per line
-constexpr long long SA_LANE_LINES = 4096;
-
-__global__ __launch_bounds__(SAJ_THREADS) void k_sa_lines_j(const DevMesh* __restrict__ Ms) {
-  __shared__ double ta[2][64][SA_TJ + 1], tb[2][64][SA_TJ + 1], tc[2][64][SA_TJ + 1], ts[2][64][SA_TJ + 1];
-  const DevMesh& M = Ms[blockIdx.y];
-  if (*M.status) return;
-  const int js = M.js, je = M.je, ks = M.ks, ke = M.ke;
-  const int k0 = ks + 32 * blockIdx.x;
-  if (k0 > ke) return;
-  const int nrow = ke - k0 + 1 < 32 ? ke - k0 + 1 : 32;
-  const int n = je - js + 1;
-  int nr, m;
-  sa_split(n, nr, m);
-  const int nl = (m + SA_TJ - 1) / SA_TJ;   // tiles of the left side (nl >= nr)
-  const int wave = threadIdx.x >> 6, l = threadIdx.x & 63, ml = (int)threadIdx.x - 64;
-  const int h = l >> 5, rr = l & 31;         // the solver lane's side and row
-  // tiles of side h, and the last position of its last tile
-  const int ntl = h ? nr : nl;
-  const int lastp = h ? SA_TJ - 1 : m - 1 - SA_TJ * (nl - 1);
-  gdouble* __restrict__ sS = gptr(M.sa_sj);
-  gdouble* __restrict__ sC = gptr(M.sa_cj);
-  const gdouble* __restrict__ sA = gptr(M.sa_aj);
-  const gdouble* __restrict__ sB = gptr(M.sa_bb);
-  // element p of mover lane ml in a tile: e = ml + 256 p, slot row e / SA_TJ
-  // (side and row as for the solver lanes), position e % SA_TJ; the global
-  // index is clamped into the grid, so every load is unconditional and no
-  // loaded value merges across a branch
-  auto gidx = [&](int x, int p, int& r, int& cc, bool& ok) {
-    const int e = ml + 64 * SAJ_MW * p;
-    r = e / SA_TJ; cc = e % SA_TJ;
-    const int hh = r >> 5, rw = r & 31;
-    const int t = hh ? n - 1 - SA_TJ * x - cc : SA_TJ * x + cc;   // cell of the line
-    ok = rw < nrow && (hh ? x < nr : t < m);
-    const int tc = t < 0 ? 0 : (t < n ? t : n - 1);
-    return cell(M, js + tc, k0 + (rw < nrow ? rw : 0));
-  };
-  double ra[SAJ_D][SAJ_PER], rb[SAJ_D][SAJ_PER], rc[SAJ_D][SAJ_PER], rs[SAJ_D][SAJ_PER];
-
-  // ---- elimination from both ends
-  auto fetch_f = [&](int t, double (&a)[SAJ_PER], double (&b)[SAJ_PER], double (&c)[SAJ_PER], double (&s)[SAJ_PER]) {
+  part_columns<TC>(a, b, c, s, P, sak_ex);
 #pragma unroll
-    for (int p = 0; p < SAJ_PER; ++p) {
-      int r, cc; bool ok;
-      const long long i = gidx(t, p, r, cc, ok);
-      (void)ok;
-      a[p] = sA[i]; b[p] = sB[i]; c[p] = sC[i]; s[p] = sS[i];
-    }
-  };
-  // elements outside a side (rows past the last, cells past the side's end
-  // in its last tile) hold copies of clamped cells: the recurrences never
-  // read them
-  auto put_f = [&](int slot, const double (&a)[SAJ_PER], const double (&b)[SAJ_PER], const double (&c)[SAJ_PER],
-                   const double (&s)[SAJ_PER]) {
-#pragma unroll
-    for (int p = 0; p < SAJ_PER; ++p) {
-      const int e = ml + 64 * SAJ_MW * p, r = e / SA_TJ, cc = e % SA_TJ;
-      ta[slot][r][cc] = a[p]; tb[slot][r][cc] = b[p]; tc[slot][r][cc] = c[p]; ts[slot][r][cc] = s[p];
-    }
-  };
-  auto back_f = [&](int t, int slot) {   // s' and c' (a') of tile t to global memory
-#pragma unroll
-    for (int p = 0; p < SAJ_PER; ++p) {
-      int r, cc; bool ok;
-      const long long i = gidx(t, p, r, cc, ok);
-      if (ok) { sS[i] = ts[slot][r][cc]; sC[i] = tc[slot][r][cc]; }
-    }
-  };
-  double cp = 0.0, sp = 0.0;
-  // side h's lower and upper coefficients: (a, c) on the left, (c, a) on the
-  // right; c' / a' goes where c was
-  auto solve_f = [&](int x, int slot) {
-    if (rr >= nrow || x >= ntl) return;
-    const int cn = x == ntl - 1 ? lastp + 1 : SA_TJ;   // positions of this tile
-    double (*LO)[SA_TJ + 1] = h ? tc[slot] : ta[slot];
-    double (*HI)[SA_TJ + 1] = h ? ta[slot] : tc[slot];
-    double (*B)[SA_TJ + 1] = tb[slot];
-    double (*Cc)[SA_TJ + 1] = tc[slot];
-    double (*S)[SA_TJ + 1] = ts[slot];
-    auto elem = [&](int cc) {
-      double ai = LO[l][cc];
-      double bb = 1. / (B[l][cc] - ai * cp);
-      sp = (S[l][cc] - ai * sp) * bb;
-      cp = HI[l][cc] * bb;
-      S[l][cc] = sp; Cc[l][cc] = cp;
-    };
-    if (x == 0) {
-      double bb = 1. / B[l][0];
-      sp = S[l][0] * bb; cp = HI[l][0] * bb;
-      S[l][0] = sp; Cc[l][0] = cp;
-#pragma unroll
-      for (int cc = 1; cc < SA_TJ; ++cc)
-        if (cc < cn) elem(cc);
-    } else if (cn == SA_TJ) {
-      // chunks of THOMAS_CH cells, each chunk's LDS reads issued before the
-      // previous chunk's recurrence
-      constexpr int CH = THOMAS_CH;
-      double xa[2][CH], xb[2][CH], xc[2][CH], xs[2][CH];
-      auto ld = [&](int q, int c0) {
-#pragma unroll
-        for (int u = 0; u < CH; ++u) {
-          xa[q][u] = LO[l][c0 + u]; xb[q][u] = B[l][c0 + u]; xc[q][u] = HI[l][c0 + u]; xs[q][u] = S[l][c0 + u];
-        }
-      };
-      ld(0, 0);
-#pragma unroll
-      for (int k = 0; k < SA_TJ / CH; ++k) {
-        if (k + 1 < SA_TJ / CH) ld((k + 1) & 1, (k + 1) * CH);
-#pragma unroll
-        for (int u = 0; u < CH; ++u) {
-          const int cc = k * CH + u;
-          const double ai = xa[k & 1][u];
-          double bb = 1. / (xb[k & 1][u] - ai * cp);
-          sp = (xs[k & 1][u] - ai * sp) * bb;
-          cp = xc[k & 1][u] * bb;
-          S[l][cc] = sp; Cc[l][cc] = cp;
-        }
-      }
-    } else {
-#pragma unroll
-      for (int cc = 0; cc < SA_TJ; ++cc)
-        if (cc < cn) elem(cc);
-    }
-  };
-  // Tile x sits in register set x % SAJ_D.  Every fetch is unconditional
-  // (tile indices past the sides are clamped to the last tile) and the
-  // movers' main loop runs whole groups of SAJ_D tiles in code of their own,
-  // so no loaded value merges across a branch and each load is waited for
-  // only where it is stored to LDS.  Solver and movers pass the same
-  // sequence of barriers: one after each pass's prologue, one per tile, and
-  // one between the passes.
-  auto clampt = [&](int t) { return t < nl ? t : nl - 1; };
-  auto step_f = [&](int t, double (&a)[SAJ_PER], double (&b)[SAJ_PER], double (&c)[SAJ_PER],
-                    double (&s)[SAJ_PER]) {
-    if (t >= 1) back_f(t - 1, (t - 1) & 1);
-    if (t + 1 < nl) put_f((t + 1) & 1, a, b, c, s);
-    fetch_f(clampt(t + 1 + SAJ_D), a, b, c, s);
-    __syncthreads();
-  };
-  if (wave == 0) {
-    __syncthreads();
-    for (int t = 0; t < nl; ++t) {
-      solve_f(t, t & 1);
-      __syncthreads();
-    }
-  } else {
-#pragma unroll
-    for (int d = 0; d < SAJ_D; ++d) fetch_f(clampt(d), ra[d], rb[d], rc[d], rs[d]);
-    put_f(0, ra[0], rb[0], rc[0], rs[0]);
-    fetch_f(clampt(SAJ_D), ra[0], rb[0], rc[0], rs[0]);
-    __syncthreads();
-    int t0 = 0;
-    for (; t0 + SAJ_D <= nl; t0 += SAJ_D) {
-#pragma unroll
-      for (int d = 0; d < SAJ_D; ++d) {
-        const int d1 = (d + 1) % SAJ_D;
-        step_f(t0 + d, ra[d1], rb[d1], rc[d1], rs[d1]);
-      }
-    }
-#pragma unroll
-    for (int d = 0; d < SAJ_D; ++d) {
-      const int d1 = (d + 1) % SAJ_D;
-      if (t0 + d < nl) step_f(t0 + d, ra[d1], rb[d1], rc[d1], rs[d1]);
-    }
-    back_f(nl - 1, (nl - 1) & 1);
-  }
-  // the meeting cells: each side's value from its own (s', c') and the other
-  // side's (lanes l and l ^ 32 hold the two sides of one row)
-  double sn = sp;
-  if (wave == 0 && nr > 0) {
-    const double so = __shfl_xor(sp, 32), co = __shfl_xor(cp, 32);
-    sn = (sp - cp * so) / (1. - cp * co);
-  }
-
-  // ---- back substitution, tiles in reverse (iteration y takes tile
-  // nl-1-y of each side); s = (0 + sn - 0) * bjmat.  Each mover lane
-  // reloads the elements it wrote itself, so program order makes them
-  // visible.
-  auto fetch_b = [&](int t, double (&b)[SAJ_PER], double (&c)[SAJ_PER], double (&s)[SAJ_PER]) {
-#pragma unroll
-    for (int p = 0; p < SAJ_PER; ++p) {
-      int r, cc; bool ok;
-      const long long i = gidx(t, p, r, cc, ok);
-      (void)ok;
-      b[p] = sB[i]; c[p] = sC[i]; s[p] = sS[i];
-    }
-  };
-  auto put_b = [&](int slot, const double (&b)[SAJ_PER], const double (&c)[SAJ_PER], const double (&s)[SAJ_PER]) {
-#pragma unroll
-    for (int p = 0; p < SAJ_PER; ++p) {
-      const int e = ml + 64 * SAJ_MW * p, r = e / SA_TJ, cc = e % SA_TJ;
-      tb[slot][r][cc] = b[p]; tc[slot][r][cc] = c[p]; ts[slot][r][cc] = s[p];
-    }
-  };
-  auto back_b = [&](int t, int slot) {
-#pragma unroll
-    for (int p = 0; p < SAJ_PER; ++p) {
-      int r, cc; bool ok;
-      const long long i = gidx(t, p, r, cc, ok);
-      if (ok) sS[i] = ts[slot][r][cc];
-    }
-  };
-  auto solve_b = [&](int x, int slot) {
-    if (rr >= nrow || x >= ntl) return;
-    double (*B)[SA_TJ + 1] = tb[slot];
-    double (*Cc)[SA_TJ + 1] = tc[slot];
-    double (*S)[SA_TJ + 1] = ts[slot];
-    auto elem = [&](int cc) {
-      sn = S[l][cc] - Cc[l][cc] * sn;
-      S[l][cc] = (0. + sn - 0.) * B[l][cc];
-    };
-    if (x == ntl - 1) {
-      // the side's meeting cell starts the substitution
-      S[l][lastp] = (0. + sn - 0.) * B[l][lastp];
-#pragma unroll
-      for (int cc = SA_TJ - 2; cc >= 0; --cc)
-        if (cc < lastp) elem(cc);
-    } else {
-      // chunks of THOMAS_CH cells from the tile's end, reads a chunk ahead
-      constexpr int CH = THOMAS_CH;
-      double xb[2][CH], xc[2][CH], xs[2][CH];
-      auto ld = [&](int q, int c1) {
-#pragma unroll
-        for (int u = 0; u < CH; ++u) {
-          xb[q][u] = B[l][c1 - u]; xc[q][u] = Cc[l][c1 - u]; xs[q][u] = S[l][c1 - u];
-        }
-      };
-      ld(0, SA_TJ - 1);
-#pragma unroll
-      for (int k = 0; k < SA_TJ / CH; ++k) {
-        if (k + 1 < SA_TJ / CH) ld((k + 1) & 1, SA_TJ - 1 - (k + 1) * CH);
-#pragma unroll
-        for (int u = 0; u < CH; ++u) {
-          const int cc = SA_TJ - 1 - k * CH - u;
-          sn = xs[k & 1][u] - xc[k & 1][u] * sn;
-          S[l][cc] = (0. + sn - 0.) * xb[k & 1][u];
-        }
-      }
-    }
-  };
-  __syncthreads();
-  // iteration y takes tile nl-1-y; register set y % SAJ_D, tiles past the
-  // sides' starts clamped to tile 0
-  auto rtile = [&](int y) { return y < nl ? nl - 1 - y : 0; };
-  auto step_b = [&](int y, double (&b)[SAJ_PER], double (&c)[SAJ_PER], double (&s)[SAJ_PER]) {
-    if (y >= 1) back_b(nl - y, (y - 1) & 1);
-    if (y + 1 < nl) put_b((y + 1) & 1, b, c, s);
-    fetch_b(rtile(y + 1 + SAJ_D), b, c, s);
-    __syncthreads();
-  };
-  if (wave == 0) {
-    __syncthreads();
-    for (int y = 0; y < nl; ++y) {
-      solve_b(nl - 1 - y, y & 1);
-      __syncthreads();
-    }
-  } else {
-#pragma unroll
-    for (int d = 0; d < SAJ_D; ++d) fetch_b(rtile(d), rb[d], rc[d], rs[d]);
-    put_b(0, rb[0], rc[0], rs[0]);
-    fetch_b(rtile(SAJ_D), rb[0], rc[0], rs[0]);
-    __syncthreads();
-    int y0 = 0;
-    for (; y0 + SAJ_D <= nl; y0 += SAJ_D) {
-#pragma unroll
-      for (int d = 0; d < SAJ_D; ++d) {
-        const int d1 = (d + 1) % SAJ_D;
-        step_b(y0 + d, rb[d1], rc[d1], rs[d1]);
-      }
-    }
-#pragma unroll
-    for (int d = 0; d < SAJ_D; ++d) {
-      const int d1 = (d + 1) % SAJ_D;
-      if (y0 + d < nl) step_b(y0 + d, rb[d1], rc[d1], rs[d1]);
-    }
-    back_b(0, (nl - 1) & 1);
-  }
-}
-
-// k_sa_lines<0>: lines along k (one per j column), one lane per side of a
-// line: 32 columns per workgroup, lane l = 32h + c walking side h of column
-// c's two-ended elimination (h = 0 up from ks, h = 1 down from ke; the same
-// operations as thomas2_lds), with the coefficients of its next SA_PK cells
-// loaded ahead into registers.  Lanes on consecutive columns, so every step
-// reads one contiguous row segment; the nu-tilde update follows in
-// k_sa_update.
-constexpr int SA_PK = 16;
-
-template <int JL>
-__global__ __launch_bounds__(64) void k_sa_lines(const DevMesh* __restrict__ Ms) {
-  static_assert(JL == 0, "lines along j run in k_sa_lines_j");
-  const DevMesh& M = Ms[blockIdx.y];
-  if (*M.status) return;
-  const int js = M.js, je = M.je, ks = M.ks, ke = M.ke;
-  if (js + 32 * (int)blockIdx.x > je) return;
-  const int h = (int)threadIdx.x >> 5;
-  const int line = js + 32 * blockIdx.x + (threadIdx.x & 31);
-  const bool lane_ok = line <= je;
-  const int ll = lane_ok ? line : je;
-  const int n = ke - ks + 1;
-  int nr, m;
-  sa_split(n, nr, m);
-  // this lane's side: cnt cells, step u at base + u*step (both in elements);
-  // a side with no cells (h = 1, nr = 0) walks the left side's cells and
-  // stores nothing
-  const bool side_ok = h == 0 || nr > 0;
-  const bool st_ok = lane_ok && side_ok;
-  const int hs = side_ok ? h : 0;
-  const int cnt = hs ? n - m : m;
-  const long long st = M.jd;
-  const long long base = cell(M, ll, ks) + (hs ? (long long)(n - 1) * st : 0);
-  const long long step = hs ? -st : st;
-  // global (not generic) pointers: the compiler then counts each load's
-  // completion exactly and the loads ahead stay in flight
-  gdouble* __restrict__ sS = gptr(M.sa_sj);
-  gdouble* __restrict__ sC = gptr(M.sa_ck);
-  const gdouble* __restrict__ sA = gptr(M.sa_ak);
-  const gdouble* __restrict__ sB = gptr(M.sa_bb);
-  // lower and upper coefficients of the side: (a, c) going up, (c, a) down;
-  // c' / a' goes where c was
-  const gdouble* __restrict__ sLo = hs ? (const gdouble*)sC : sA;
-  const gdouble* __restrict__ sHi = hs ? sA : (const gdouble*)sC;
-  // Loads ahead are unconditional (steps clamped to the side) and the
-  // unrolled loops run whole chunks, the remainder separately.  Slot d of a
-  // prefetch array holds the step congruent to d modulo SA_PK.
-  auto at = [&](int u) { return base + (long long)(u < cnt ? u : cnt - 1) * step; };
-  double pa[SA_PK], pb[SA_PK], pc[SA_PK], ps[SA_PK];
-#pragma unroll
-  for (int d = 0; d < SA_PK; ++d) {
-    const long long i = at(d);
-    pa[d] = sLo[i]; pb[d] = sB[i]; pc[d] = sHi[i]; ps[d] = sS[i];
-  }
-  double cp, sp;
-  {
-    // first cell of the side (its lower coefficient is not used)
-    const double b = pb[0], c = pc[0], s = ps[0];
-    const long long i = at(SA_PK);
-    pa[0] = sLo[i]; pb[0] = sB[i]; pc[0] = sHi[i]; ps[0] = sS[i];
-    double bb = 1. / b;
-    sp = s * bb; cp = c * bb;
-    if (st_ok) { sS[base] = sp; sC[base] = cp; }
-  }
-  auto fwd = [&](int u, int d) {
-    const double a = pa[d], b = pb[d], c = pc[d], s = ps[d];
-    const long long i = at(u + SA_PK);
-    pa[d] = sLo[i]; pb[d] = sB[i]; pc[d] = sHi[i]; ps[d] = sS[i];
-    double bb = 1. / (b - a * cp);
-    sp = (s - a * sp) * bb;
-    cp = c * bb;
-    if (st_ok) { const long long o = base + (long long)u * step; sS[o] = sp; sC[o] = cp; }
-  };
-  int tb = 1;
-  for (; tb + SA_PK <= cnt; tb += SA_PK) {
-#pragma unroll
-    for (int e = 0; e < SA_PK; ++e) fwd(tb + e, (1 + e) % SA_PK);
-  }
-#pragma unroll
-  for (int e = 0; e < SA_PK; ++e)
-    if (tb + e < cnt) fwd(tb + e, (1 + e) % SA_PK);
-  // the meeting cells (lanes l and l ^ 32 hold the two sides of a column)
-  double sn = sp;
-  if (nr > 0) {
-    const double so = __shfl_xor(sp, 32), co = __shfl_xor(cp, 32);
-    sn = (sp - cp * so) / (1. - cp * co);
-  }
-  // back substitution towards the side's start (the values this lane just
-  // wrote), the next cells loaded ahead; slot d holds back-step v congruent
-  // to d (back-step v is step cnt-1-v); dq = s2 goes back into sjmat
-  auto atb = [&](int v) { return base + (long long)(v < cnt ? cnt - 1 - v : 0) * step; };
-  double qs[SA_PK], qc[SA_PK];
-#pragma unroll
-  for (int d = 0; d < SA_PK; ++d) {
-    const long long i = atb(d);
-    qs[d] = sS[i]; qc[d] = sC[i];
-  }
-  {
-    const long long i = atb(SA_PK);
-    qs[0] = sS[i]; qc[0] = sC[i];
-    if (st_ok) sS[base + (long long)(cnt - 1) * step] = sn;
-  }
-  auto bwd = [&](int v, int d) {
-    const double s = qs[d], c = qc[d];
-    const long long i = atb(v + SA_PK);
-    qs[d] = sS[i]; qc[d] = sC[i];
-    sn = s - c * sn;
-    if (st_ok) sS[base + (long long)(cnt - 1 - v) * step] = sn;
-  };
-  int ub = 1;
-  for (; ub + SA_PK <= cnt; ub += SA_PK) {
-#pragma unroll
-    for (int e = 0; e < SA_PK; ++e) bwd(ub + e, (1 + e) % SA_PK);
-  }
-#pragma unroll
-  for (int e = 0; e < SA_PK; ++e)
-    if (ub + e < cnt) bwd(ub + e, (1 + e) % SA_PK);
-}
-
-// nu-tilde update with its clip (src/samodel2d.f:157-188) and the interior
-// eddy viscosity after the lane-per-line k solve: a pointwise pass over the
-// interior cells, so its loads stream at full bandwidth instead of waiting
-// on each line's recurrence
-__global__ __launch_bounds__(256) void k_sa_update(const DevMesh* __restrict__ Ms, int ovl) {
-  const DevMesh& M = Ms[blockIdx.y];
-  if (*M.status) return;
-  const int nj = M.je - M.js + 1, nk = M.ke - M.ks + 1;
-  const long long ncell = (long long)nj * nk;
-  const double vnulim = 1.0e-20, relfac = 1.0;
-  for (long long w = blockIdx.x * 256ll + threadIdx.x; w < ncell; w += 256ll * gridDim.x) {
-    const int j = M.js + (int)(w % nj), k = M.ks + (int)(w / nj);
-    const long long i = cell(M, j, k);
-    const double dq = M.sa_sj[i];
-    const double v = fmax((M.q[4][i] + relfac * (0. + dq) * (double)imx(M.iblank[i], 0)), vnulim);
+  for (int u = 0; u < PM; ++u) {
+    if (!col || k0 + u >= n) continue;
+    const long long i = i0 + (long long)(k0 + u) * st;
+    const double dq = relfac * (0. + s[u]);
+    const double v = fmax((q5[u] + dq * (double)imx(ib[u], 0)), vnulim);
     M.q[4][i] = v;
-    put_turm(M, i, M.q[0][i], M.q[M.nq - 1][i], M.sa_vmul[i], v, ovl);
+    put_turm(M, i, q1[u], qj[u], vm[u], v, ovl);
   }
 }
 
@@ -1370,6 +842,12 @@ hipError_t launch_sa_prim(const DevMesh* dM, const DevMesh* hM, int nmi, hipStre
   return hipGetLastError();
 }
 
+// columns (all instances) above which the k solves take 16 columns per
+// workgroup instead of 8: at 2048 columns, 8 fill the chip with 256
+// workgroups (figures at k_sa_solve_k).  Columns of more than 256 cells
+// (parts x 16 columns over 512 threads) always take 8.
+constexpr long long SAK_WIDE_COLS = 2048;
+
 // turbc over every instance: one launch per phase of the segments
 static hipError_t launch_turbc(const DevMesh* dM, const DevMesh* hM, int nmi, hipStream_t st) {
   int nbc = 1, nph = 1;
@@ -1405,44 +883,19 @@ hipError_t launch_sa(const DevMesh* dM, const DevMesh* hM, int nmi, Marks* mk, h
   hipLaunchKernelGGL(k_sa_rhs, dim3(nblk2(mx, 256), nmi), dim3(256), 0, st, dM);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_SA_RHS, st);
-  // few lines (one case): one wave per line keeps each recurrence's chain
-  // short in latency; many lines (batches): one lane per line
-  long long lines = 0;
-  for (int i = 0; i < nmi; ++i) lines += (hM[i].ke - hM[i].ks + 1) + (hM[i].je - hM[i].js + 1);
-  const bool per_lane = sa_lane < 0 ? lines > SA_LANE_LINES : sa_lane == 1;
-  if (per_lane) hipLaunchKernelGGL(k_sa_lines_j, dim3((mk_ + 31) / 32, nmi), dim3(SAJ_THREADS), 0, st, dM);
-  else hipLaunchKernelGGL(k_sa_solve_j, dim3(mk_, nmi), dim3(64), 0, st, dM);
+  hipLaunchKernelGGL(k_sa_solve_j, dim3(mk_, nmi), dim3(64), 0, st, dM);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_SA_SOLVE_J, st);
-  if (per_lane) {
-    hipLaunchKernelGGL(k_sa_lines<0>, dim3((mj + 31) / 32, nmi), dim3(64), 0, st, dM);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_sa_update, dim3(nblk2(mx, 256), nmi), dim3(256), 0, st, dM, ovl);
-  } else {
-    if (mk_ <= SAK_NMAX16) {
-      const size_t lds = (size_t)5 * mk_ * SAK_TJ16 * sizeof(double);
-      static bool attr = false;
-      if (!attr) {
-        (void)hipFuncSetAttribute((const void*)k_sa_solve_kt<SAK_TJ16>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  (int)(5 * SAK_NMAX16 * SAK_TJ16 * sizeof(double)));
-        attr = true;
-      }
-      hipLaunchKernelGGL(k_sa_solve_kt<SAK_TJ16>, dim3((mj + SAK_TJ16 - 1) / SAK_TJ16, nmi), dim3(32 * SAK_TJ16), lds,
-                         st, dM, ovl, mk_);
-    } else if (mk_ <= SAK_NMAX) {
-      const size_t lds = (size_t)5 * mk_ * SAK_TJ * sizeof(double);
-      static bool attr = false;
-      if (!attr) {
-        (void)hipFuncSetAttribute((const void*)k_sa_solve_kt<SAK_TJ>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  (int)(5 * SAK_NMAX * SAK_TJ * sizeof(double)));
-        attr = true;
-      }
-      hipLaunchKernelGGL(k_sa_solve_kt<SAK_TJ>, dim3((mj + SAK_TJ - 1) / SAK_TJ, nmi), dim3(32 * SAK_TJ), lds, st,
-                         dM, ovl, mk_);
-    } else {
-      hipLaunchKernelGGL(k_sa_solve_k, dim3(mj, nmi), dim3(64), 0, st, dM, ovl);
-    }
-  }
+  const int np = (mk_ + PCOL_M - 1) / PCOL_M;   // parts of the longest column
+  long long cols = 0;
+  for (int i = 0; i < nmi; ++i) cols += hM[i].je - hM[i].js + 1;
+  const bool wide = np * 16 <= SAK_NT && (sa_lane < 0 ? cols > SAK_WIDE_COLS : sa_lane == 0);
+  auto solve_k = [&](auto kern, int tc) {
+    const int nt = (np * tc + 63) / 64 * 64;
+    hipLaunchKernelGGL(kern, dim3((mj + tc - 1) / tc, nmi), dim3(nt), sizeof(double) * 6 * nt, st, dM, ovl);
+  };
+  if (wide) solve_k(k_sa_solve_k<16>, 16);
+  else solve_k(k_sa_solve_k<8>, 8);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_SA_SOLVE_K, st);
   hipLaunchKernelGGL(k_turbc_eddy, dim3(nmi), dim3(BC_THREADS), 0, st, dM, ovl);
