@@ -375,7 +375,9 @@ __device__ inline void norm_tile(const DevMesh& M, const ResTile& T, int j, int 
       if (a > rmax) { rmax = a; key = (double)(((long long)(k - 1) * 4 + n) * jd + (j - 1)); }
     }
   }
-  red[0][tid] = rs; red[1][tid] = rr1; red[2][tid] = rmax; red[3][tid] = valid && rmax > 0.0 ? key : 1e300;
+  if (tid < RES_THREADS) {   // threads past the tile's cells pass the barriers only
+    red[0][tid] = rs; red[1][tid] = rr1; red[2][tid] = rmax; red[3][tid] = valid && rmax > 0.0 ? key : 1e300;
+  }
   __syncthreads();
   for (int off = RES_THREADS / 2; off > 0; off >>= 1) {
     if (tid < off) {

@@ -713,16 +713,25 @@ __device__ __forceinline__ void face_states_weno(const double* sf0, int stv, int
 // of the tile's faces computed once into LDS, plus the residual-norm partials
 // of step (src/step.f:60-93).  Writes s(:,:,1:4) of the tile's interior cells.
 // H: halo cells the tile loads on each side (2 for MUSCL, 3 for WENO5)
-template <int H>
-__global__ __launch_bounds__(RES_THREADS) void k_residual(const DevMesh* __restrict__ Ms,
-                                                          const ResTile* __restrict__ tiles, int do_norms) {
+// The tile's 264 xi and 288 eta faces are one list, each face the same code
+// with its direction's LDS strides, so NT threads take them in
+// ceil(552 / NT) passes: one (NT = 576) where few tiles leave a CU one
+// workgroup and the passes' latency counts, three (NT = 256) where tiles fill
+// the chip and idle lanes of the last pass cost issue slots.  513x129 (256
+// tiles): 10 us (576), 13 (256), 15.5 with a pass or two per direction before;
+// 385x97 with 401x401, WENO5 (1206 tiles): 38 / 41 / 47; 60 cases (15200
+// tiles): 333 (576), 270 (256), 301 before.  FP64 issue binds the last
+// (800 operations a face).
+template <int H, int NT>
+__global__ __launch_bounds__(NT) void k_residual(const DevMesh* __restrict__ Ms, const ResTile* __restrict__ tiles,
+                                                 int do_norms) {
   constexpr int TJ = RES_TJ, TK = RES_TK, LJ = TJ + 2 * H, LK = TK + 2 * H;
-  __shared__ double sf[4][LK][LJ];   // primitives rho, u, v, p
-  __shared__ int sib[LK][LJ];
-  __shared__ double sxv[TK + 1][TJ + 1], syv[TK + 1][TJ + 1];
-  __shared__ double sF[4][TK][TJ + 1];  // j-face fluxes
-  __shared__ double sG[4][TK + 1][TJ];  // k-face fluxes
-  __shared__ double red[4][RES_THREADS];
+  constexpr int NXI = TK * (TJ + 1), NETA = (TK + 1) * TJ;
+  __shared__ double sf[4][LK * LJ];   // primitives rho, u, v, p; then the norms' reduction
+  __shared__ int sib[LK * LJ];
+  __shared__ double sxv[(TK + 1) * (TJ + 1)], syv[(TK + 1) * (TJ + 1)];
+  __shared__ double sF[4][NXI + NETA];  // fluxes: xi faces [TK][TJ+1], then eta faces [TK+1][TJ]
+  static_assert(4 * LK * LJ >= 4 * RES_THREADS, "the reduction fits the primitives' array");
   const ResTile T = tiles[blockIdx.x];
   const DevMesh& M = Ms[T.mesh];
   const DevConst& C = M.c;
@@ -731,7 +740,7 @@ __global__ __launch_bounds__(RES_THREADS) void k_residual(const DevMesh* __restr
   const int j0 = T.j0, k0 = T.k0;
   QV v = qview(M);
   // ---- load primitives of the tile + H-cell halo (corners unused)
-  for (int w = tid; w < LK * LJ; w += RES_THREADS) {
+  for (int w = tid; w < LK * LJ; w += NT) {
     int r = w / LJ, cc = w % LJ;
     int j = j0 - H + cc, k = k0 - H + r;
     bool row_in = (r >= H && r < H + TK), col_in = (cc >= H && cc < H + TJ);
@@ -742,91 +751,74 @@ __global__ __launch_bounds__(RES_THREADS) void k_residual(const DevMesh* __restr
     double q1 = v.q1[i], q2 = v.q2[i], q3 = v.q3[i], q4 = v.q4[i], qj = v.qj[i];
     double rhoi = 1.0 / q1;
     double ppp = C.gm1 * (q4 - 0.5 * (sq(q2) + sq(q3)) / q1);
-    sf[0][r][cc] = q1 * qj;
-    sf[1][r][cc] = q2 * rhoi;
-    sf[2][r][cc] = q3 * rhoi;
-    sf[3][r][cc] = ppp * qj;
+    sf[0][w] = q1 * qj;
+    sf[1][w] = q2 * rhoi;
+    sf[2][w] = q3 * rhoi;
+    sf[3][w] = ppp * qj;
     int ib = M.iblank[i];
-    sib[r][cc] = ib < 0 ? -ib : ib;
+    sib[w] = ib < 0 ? -ib : ib;
   }
-  for (int w = tid; w < (TK + 1) * (TJ + 1); w += RES_THREADS) {
+  for (int w = tid; w < (TK + 1) * (TJ + 1); w += NT) {
     int r = w / (TJ + 1), cc = w % (TJ + 1);
     int jv = j0 - 1 + cc, kv = k0 - 1 + r;
     jv = jv > M.jmax ? M.jmax : jv;
     kv = kv > M.kmax ? M.kmax : kv;
     long long iv = vert(M, jv, kv);
-    sxv[r][cc] = M.xv[iv];
-    syv[r][cc] = M.yv[iv];
+    sxv[w] = M.xv[iv];
+    syv[w] = M.yv[iv];
   }
   __syncthreads();
   const double th = C.th, qt = C.qt;
-  // ---- xi (j-direction) faces: face fi between cells fi and fi+1, rows k0..k0+TK-1
-  for (int w = tid; w < TK * (TJ + 1); w += RES_THREADS) {
-    int r = w / (TJ + 1), cc = w % (TJ + 1);
-    int fi = j0 - 1 + cc, k = k0 + r;
-    if (fi > M.je || k > M.ke) continue;
+  // ---- faces: xi face (r, cc) between cells i = j0-1+cc and i+1 of row
+  // k0+r, eta face between cells i = k0-1+r and i+1 of column j0+cc
+  for (int w = tid; w < NXI + NETA; w += NT) {
+    const bool eta = w >= NXI;
+    const int we = w - NXI;
+    const int r = eta ? we / TJ : w / (TJ + 1), cc = eta ? we % TJ : w % (TJ + 1);
+    const int i = eta ? k0 - 1 + r : j0 - 1 + cc;   // line cell on the face's low side
+    const int t = eta ? j0 + cc : k0 + r;           // the line
+    if (i > (eta ? M.ke : M.je) || t > (eta ? M.je : M.ke)) continue;
+    // LDS index of cell i and the line's stride
+    const int o = eta ? (r + H - 1) * LJ + cc + H : (r + H) * LJ + cc + H - 1, st = eta ? LJ : 1;
     double l[4], rr[4], f[4];
-    // LDS column of cell fi: fi - (j0 - H)
     if (H == 3 && C.ilim == 4)
-      face_states_weno(&sf[0][r + H][0], LK * LJ, 1, &sib[r + H][0], 1, fi - (j0 - H), fi, jd, qt, l, rr);
+      face_states_weno(&sf[0][o], LK * LJ, st, &sib[o], st, 0, i, eta ? kd : jd, qt, l, rr);
     else
-      face_states(&sf[0][r + H][0], LK * LJ, 1, &sib[r + H][0], 1, fi - (j0 - H), fi, jd, th, qt, M.epsj, l, rr);
-    // face vector at vertex column jv = fi, rows kv-1..kv with kv = k
-    double xa = syv[r + 1][cc] - syv[r][cc];
-    double ya = -(sxv[r + 1][cc] - sxv[r][cc]);
+      face_states(&sf[0][o], LK * LJ, st, &sib[o], st, 0, i, eta ? kd : jd, th, qt, eta ? M.epsk : M.epsj, l, rr);
+    // face vector between vertices b and a: column i, rows t-1 .. t (xi);
+    // row i, columns t-1 .. t (eta)
+    const int vb = r * (TJ + 1) + cc, va = vb + (eta ? 1 : TJ + 1);
+    const double dx = sxv[va] - sxv[vb], dy = syv[va] - syv[vb];
+    const double xa = eta ? -dy : dy, ya = eta ? dx : -dx;
     double tj = 0.0;
-    if (C.iunst > 0) {
-      tj = swept_tj(M, vert(M, fi, k), vert(M, fi, k - 1), -1.);
-    } else if (M.has_gv) {
-      long long a = vert(M, fi, k), b = vert(M, fi, k - 1);
-      tj = -0.5 * (M.ugv[a] + M.ugv[b]) * xa - 0.5 * (M.vgv[a] + M.vgv[b]) * ya;
+    if (C.iunst > 0 || M.has_gv) {
+      const long long a = eta ? vert(M, t, i) : vert(M, i, t), b = eta ? vert(M, t - 1, i) : vert(M, i, t - 1);
+      if (C.iunst > 0) tj = swept_tj(M, a, b, eta ? 1. : -1.);
+      else tj = -0.5 * (M.ugv[a] + M.ugv[b]) * xa - 0.5 * (M.vgv[a] + M.vgv[b]) * ya;
     }
     roe_face(C, l, rr, xa, ya, tj, f);
 #pragma unroll
-    for (int n = 0; n < 4; ++n) sF[n][r][cc] = f[n];
-  }
-  // ---- eta (k-direction) faces: face fk between cells fk and fk+1, columns j0..j0+TJ-1
-  for (int w = tid; w < (TK + 1) * TJ; w += RES_THREADS) {
-    int r = w / TJ, cc = w % TJ;
-    int fk = k0 - 1 + r, j = j0 + cc;
-    if (fk > M.ke || j > M.je) continue;
-    double l[4], rr[4], f[4];
-    if (H == 3 && C.ilim == 4)
-      face_states_weno(&sf[0][0][cc + H], LK * LJ, LJ, &sib[0][cc + H], LJ, fk - (k0 - H), fk, kd, qt, l, rr);
-    else
-      face_states(&sf[0][0][cc + H], LK * LJ, LJ, &sib[0][cc + H], LJ, fk - (k0 - H), fk, kd, th, qt, M.epsk, l, rr);
-    // vertex row kv = fk, columns jv-1..jv with jv = j
-    double xa = -(syv[r][cc + 1] - syv[r][cc]);
-    double ya = (sxv[r][cc + 1] - sxv[r][cc]);
-    double tj = 0.0;
-    if (C.iunst > 0) {
-      tj = swept_tj(M, vert(M, j, fk), vert(M, j - 1, fk), 1.);
-    } else if (M.has_gv) {
-      long long a = vert(M, j, fk), b = vert(M, j - 1, fk);
-      tj = -0.5 * (M.ugv[a] + M.ugv[b]) * xa - 0.5 * (M.vgv[a] + M.vgv[b]) * ya;
-    }
-    roe_face(C, l, rr, xa, ya, tj, f);
-#pragma unroll
-    for (int n = 0; n < 4; ++n) sG[n][r][cc] = f[n];
+    for (int n = 0; n < 4; ++n) sF[n][w] = f[n];
   }
   __syncthreads();
-  // ---- flux balance
+  // ---- flux balance, one cell per thread of the first RES_THREADS
   int cx = tid % TJ, ry = tid / TJ;
   int j = j0 + cx, k = k0 + ry;
   double sv[4] = {0.0, 0.0, 0.0, 0.0};
-  bool valid = (j <= M.je && k <= M.ke);
+  bool valid = (tid < RES_THREADS && j <= M.je && k <= M.ke);
   if (valid) {
     long long i = cell(M, j, k);
+    const int x = ry * (TJ + 1) + cx, e = NXI + ry * TJ + cx;
 #pragma unroll
     for (int n = 0; n < 4; ++n) {
-      sv[n] = 0.0 - (sF[n][ry][cx + 1] - sF[n][ry][cx]);
-      sv[n] = sv[n] - (sG[n][ry + 1][cx] - sG[n][ry][cx]);
+      sv[n] = 0.0 - (sF[n][x + 1] - sF[n][x]);
+      sv[n] = sv[n] - (sF[n][e + TJ] - sF[n][e]);
       M.s[n][i] = sv[n];
     }
     // the reference clears all of s at step start (src/step.f:41)
     for (int n = 4; n < M.nv; ++n) M.s[n][i] = 0.0;
   }
-  if (do_norms) norm_tile(M, T, j, k, valid, sv, &red[0][0]);
+  if (do_norms) norm_tile(M, T, j, k, valid, sv, &sf[0][0]);
 }
 
 // second stage, one block per instance: the tile partials in a fixed order
@@ -2844,12 +2836,22 @@ hipError_t launch_bc(const DevMesh* dM, const DevMesh* hM, int nmi, int zero_s, 
   return hipSuccess;
 }
 
+// tiles up to which one thread takes at most one face (576 threads); figures
+// at k_residual
+constexpr int RES_WIDE_TILES = 2048;
+
 hipError_t launch_residual(const DevMesh* dM, const ResTile* tiles, int ntiles, int do_norms, int weno,
                            hipStream_t st) {
-  if (weno)
-    hipLaunchKernelGGL(k_residual<3>, dim3(ntiles), dim3(RES_THREADS), 0, st, dM, tiles, do_norms);
-  else
-    hipLaunchKernelGGL(k_residual<2>, dim3(ntiles), dim3(RES_THREADS), 0, st, dM, tiles, do_norms);
+  auto launch = [&](auto kern, int nt) {
+    hipLaunchKernelGGL(kern, dim3(ntiles), dim3(nt), 0, st, dM, tiles, do_norms);
+  };
+  if (ntiles <= RES_WIDE_TILES) {
+    if (weno) launch(k_residual<3, 576>, 576);
+    else launch(k_residual<2, 576>, 576);
+  } else {
+    if (weno) launch(k_residual<3, 256>, 256);
+    else launch(k_residual<2, 256>, 256);
+  }
   return hipGetLastError();
 }
 
