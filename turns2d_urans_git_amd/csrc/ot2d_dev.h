@@ -47,6 +47,26 @@ struct DevConst {
   double dtps[OT2D_MAX_ITN]; // dtpseudo(itn), the dual time of sub-iteration itn
 };
 
+// A pointer into device memory held in a record: subscripts go through the
+// global address space.  A plain pointer loaded from a record is generic to
+// the compiler: its accesses become flat instructions, which count against
+// the LDS counter as well and whose completions are only known together, so
+// loads issued ahead do not stay in flight.
+template <typename T>
+struct GPtr {
+  typedef __attribute__((address_space(1))) T G;
+  T* p;
+  __host__ __device__ GPtr& operator=(T* q) { p = q; return *this; }
+  __host__ __device__ operator T*() const { return p; }
+  template <typename I>
+  __device__ __forceinline__ G& operator[](I i) const { return ((G*)p)[i]; }
+  __device__ __forceinline__ G& operator*() const { return *(G*)p; }
+  template <typename I>
+  __device__ __forceinline__ GPtr operator+(I i) const { GPtr r; r.p = p + i; return r; }
+};
+typedef GPtr<double> gd_t;
+typedef GPtr<const double> gcd_t;
+
 struct DevMesh {
   int jd, kd, jmax, kmax;
   int js, je, ks, ke;        // jbeg, jend, kbeg, kend (1-based)
@@ -57,38 +77,38 @@ struct DevMesh {
   int res_block0, res_nblocks;  // this instance's slice of the norm partials
   double epsj, epsk;         // Koren limiter epsilons (src/eulerrhs.f:51-52)
   DevBC bc[OT2D_MAXBC_DEV];
-  double* q[OT2D_MAXQ];      // q(:,:,nsp,n) planes, n = 1..nq  (index n-1)
-  double* s[OT2D_MAXQ];      // s(:,:,nsp,n) planes
-  double *x, *y, *xx, *xy, *yx, *yy, *ug, *vg, *turmu, *tscale, *bt;
-  double* turmu_n;           // SA beside ilu2d: the new eddy viscosity until the update takes it
-  double *xv, *yv, *ugv, *vgv;  // vertex arrays (jmax,kmax) of this instance
-  const double *xv0, *yv0;      // instance-1 vertices (time-spectral rotation)
-  double *xold, *yold, *xole, *yole;  // vertices one and two time steps back (moving grids), or null
-  int* iblank;
+  GPtr<double> q[OT2D_MAXQ];  // q(:,:,nsp,n) planes, n = 1..nq  (index n-1)
+  GPtr<double> s[OT2D_MAXQ];  // s(:,:,nsp,n) planes
+  GPtr<double> x, y, xx, xy, yx, yy, ug, vg, turmu, tscale, bt;
+  GPtr<double> turmu_n;  // SA beside ilu2d: the new eddy viscosity until the update takes it
+  GPtr<double> xv, yv, ugv, vgv;  // vertex arrays (jmax,kmax) of this instance
+  GPtr<const double> xv0, yv0;  // instance-1 vertices (time-spectral rotation)
+  GPtr<double> xold, yold, xole, yole;  // vertices one and two time steps back (moving grids), or null
+  GPtr<int> iblank;
   int bodyflag;              // mesh has a wall segment (type 5)
   // SA workspace (jd,kd) planes: laminar viscosity, u, v, wall distance and
   // the rows of the two tridiagonal systems (src/samodel2d.f:22-30)
-  double *sa_vmul, *sa_u, *sa_v, *sa_sn, *sa_sj, *sa_aj, *sa_cj, *sa_ak, *sa_ck, *sa_bb;
+  GPtr<double> sa_vmul, sa_u, sa_v, sa_sn, sa_sj, sa_aj, sa_cj, sa_ak, sa_ck, sa_bb;
   // SST workspace (src/komegasst.f:20-41): F1, F2*rho*strain/Re, production,
   // cross diffusion, and per equation (k, omega) the rows of the j and k
   // tridiagonal systems sharing one diagonal
-  double *kw_f1, *kw_x, *kw_prod, *kw_cd;
-  double *kw_s[2], *kw_a[2], *kw_b[2], *kw_c[2], *kw_ak[2], *kw_ck[2];
-  double* lu;                // LU-SGS sweep records (workspace)
+  GPtr<double> kw_f1, kw_x, kw_prod, kw_cd;
+  GPtr<double> kw_s[2], kw_a[2], kw_b[2], kw_c[2], kw_ak[2], kw_ck[2];
+  GPtr<double> lu;  // LU-SGS sweep records (workspace)
   int lu_fp32;               // sweep arithmetic: 1 FP32, 0 FP64
   // per-case bookkeeping (shared by all instances of a case)
-  int* status;               // 0 ok, 1 mstop, 2 norm
-  int* istep0;               // device copy of istep0
-  int* istep;                // time steps of this run (the driver's istep; time-accurate steps)
-  double* ta;                // time-accurate levels: qtn, qtnm1, qnewt (nv planes each), or null
-  double* partials;          // norm partials of this instance's tiles (res_nblocks * 4 doubles)
-  double* norms;             // rsum, resrho, resmax, jmax, kmax, nmax
-  int* stepc;                // steps started in the current ot2d_iterate call
-  double* hist;              // residual history rsum[step][slot] (may be null)
+  GPtr<int> status;  // 0 ok, 1 mstop, 2 norm
+  GPtr<int> istep0;  // device copy of istep0
+  GPtr<int> istep;  // time steps of this run (the driver's istep; time-accurate steps)
+  GPtr<double> ta;  // time-accurate levels: qtn, qtnm1, qnewt (nv planes each), or null
+  GPtr<double> partials;  // norm partials of this instance's tiles (res_nblocks * 4 doubles)
+  GPtr<double> norms;  // rsum, resrho, resmax, jmax, kmax, nmax
+  GPtr<int> stepc;  // steps started in the current ot2d_iterate call
+  GPtr<double> hist;  // residual history rsum[step][slot] (may be null)
   int hist_cap, hist_stride, hist_slot;
-  double* tspec;             // time instant of this instance
-  const double* Ds;          // spectral derivative matrix (nspec x nspec)
-  double* qall[OT2D_MAXQ];   // q planes of instance 0 (TS coupling base)
+  GPtr<double> tspec;  // time instant of this instance
+  GPtr<const double> Ds;  // spectral derivative matrix (nspec x nspec)
+  GPtr<double> qall[OT2D_MAXQ];  // q planes of instance 0 (TS coupling base)
   long long inst_stride;     // elements between instances within a plane set
   DevConst c;
 };
@@ -100,12 +120,9 @@ struct ResTile {
   int blk;    // tile index within the instance (norm partial slot)
 };
 
-// Pointers into device memory as the global address space: loads through
-// them are global (not flat) instructions, whose completions the compiler
-// counts exactly, so loads issued ahead of their use stay in flight.
+// plain global-address-space pointers, for the arguments of line solves
 typedef __attribute__((address_space(1))) double gdouble;
-__device__ __forceinline__ gdouble* gptr(double* p) { return (gdouble*)p; }
-__device__ __forceinline__ const gdouble* gptr(const double* p) { return (const gdouble*)p; }
+__device__ __forceinline__ gdouble* gptr(const gd_t& p) { return (gdouble*)p.p; }
 
 // ------------------------------------------------- turbulence line solves
 // Tridiagonal line of n cells, a x(i-1) + b x(i) + c x(i+1) = s, solved in
@@ -390,7 +407,7 @@ __device__ inline void norm_tile(const DevMesh& M, const ResTile& T, int j, int 
     __syncthreads();
   }
   if (tid == 0) {
-    double* P = M.partials + 4ll * T.blk;
+    const gd_t P = M.partials + 4ll * T.blk;
     P[0] = red[0][0]; P[1] = red[1][0]; P[2] = red[2][0]; P[3] = red[3][0];
   }
 }

@@ -141,9 +141,9 @@ __global__ __launch_bounds__(256) void k_stqol(const DevMesh* __restrict__ Ms) {
   const bool bdf3 = ntac == 3 && istep > 2;
   for (long long i = blockIdx.x * 256ll + threadIdx.x; i < n2; i += 256ll * gridDim.x)
     for (int n = 0; n < nv; ++n) {
-      double* qtn = M.ta + (long long)n * n2;
-      double* qtnm1 = M.ta + (long long)(nv + n) * n2;
-      double* qnewt = M.ta + (long long)(2 * nv + n) * n2;
+      const gd_t qtn = M.ta + (long long)n * n2;
+      const gd_t qtnm1 = M.ta + (long long)(nv + n) * n2;
+      const gd_t qnewt = M.ta + (long long)(2 * nv + n) * n2;
       const double q = M.q[n][i], a = qtn[i], b = qtnm1[i];
       double w = q;
       if (bdf2) w = w + (q - a) / 3.;
@@ -166,7 +166,7 @@ __global__ __launch_bounds__(256) void k_newton(const DevMesh* __restrict__ Ms) 
   for (long long w = blockIdx.x * 256ll + threadIdx.x; w < ncell; w += 256ll * gridDim.x) {
     const long long i = cell(M, M.js + (int)(w % nj), M.ks + (int)(w / nj));
     for (int n = 0; n < M.nv; ++n) {
-      const double* qnewt = M.ta + (long long)(2 * M.nv + n) * n2;
+      const gd_t qnewt = M.ta + (long long)(2 * M.nv + n) * n2;
       M.s[n][i] = M.s[n][i] - (M.q[n][i] - qnewt[i]) * tac;
     }
   }
@@ -181,7 +181,7 @@ __global__ __launch_bounds__(256) void k_copy_doubles(double* __restrict__ dst, 
 
 // ======================================================================= BCs
 struct QV {
-  double *q1, *q2, *q3, *q4, *qj;
+  gd_t q1, q2, q3, q4, qj;
 };
 __device__ inline QV qview(const DevMesh& M) {
   QV v;
@@ -247,7 +247,7 @@ __device__ inline void trkl_cell(const DevMesh& M, const QV& v, long long i, lon
   double gm1 = C.gm1, gamma = C.gamma, Mp = C.Mp;
   double foso = 1.0;
   double qext[4], qbar[4], delq[4], delw[4];
-  double* qs[4] = {v.q1, v.q2, v.q3, v.q4};
+  const gd_t qs[4] = {v.q1, v.q2, v.q3, v.q4};
 #pragma unroll
   for (int n = 0; n < 4; ++n) qext[n] = (1. + foso) * qs[n][i1] * v.qj[i1] - foso * qs[n][i2] * v.qj[i2];
   qbar[0] = 0.5 * (qext[0] + C.rinf);
@@ -338,7 +338,7 @@ __device__ void bc_segment(const DevMesh& M, const DevBC& b, int istep0) {
     }
     case 10: {
       double foso = 0.0;
-      double* qs[4] = {v.q1, v.q2, v.q3, v.q4};
+      const gd_t qs[4] = {v.q1, v.q2, v.q3, v.q4};
       if (iadir == 1) {
         int j = (idir == 1) ? je : js;  // one layer
         int j1 = j + iadd, j2 = j1 + iadd;
@@ -837,7 +837,7 @@ __global__ __launch_bounds__(RES_THREADS) void k_norms_final(const DevMesh* __re
   const int jd = M.jd, kd = M.kd;
   {
     double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 1e300;
-    const double* P = M.partials;
+    const gd_t P = M.partials;
     for (int b = tid; b < M.res_nblocks; b += RES_THREADS) {
       a0 = a0 + P[4 * b + 0];
       a1 = a1 + P[4 * b + 1];
@@ -870,7 +870,7 @@ __global__ __launch_bounds__(RES_THREADS) void k_norms_final(const DevMesh* __re
       nm = (int)(rest % 4) + 1;
       km = (int)(rest / 4) + 1;
     }
-    double* N = M.norms;
+    const gd_t N = M.norms;
     N[0] = rsum; N[1] = resrho; N[2] = resmax; N[3] = jm; N[4] = km; N[5] = nm;
     if (M.hist && M.stepc) {
       int sc = *M.stepc;
@@ -933,8 +933,8 @@ __global__ __launch_bounds__(256) void k_tsrhs(const DevMesh* __restrict__ Ms) {
 // (rbcwake 1576-1633), extrapolation (2029-2094), symmetry (2160-2222),
 // periodic (270-357).
 __device__ void rbc_segment(const DevMesh& M, const DevBC& b) {
-  double* qj = M.q[M.nq - 1];
-  double* ss[4] = {M.s[0], M.s[1], M.s[2], M.s[3]};
+  const gd_t qj = M.q[M.nq - 1];
+  const gd_t ss[4] = {M.s[0], M.s[1], M.s[2], M.s[3]};
   int js = b.js, je = b.je, ks = b.ks, ke = b.ke, idir = b.idir;
   int iadd = idir >= 0 ? 1 : -1, iadir = idir >= 0 ? idir : -idir;
   int t = threadIdx.x, nt = blockDim.x;
@@ -1223,9 +1223,12 @@ __device__ __forceinline__ LUGeom lu_geom(const DevMesh& M) {
 typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
 typedef double f64x2_t __attribute__((ext_vector_type(2)));
-struct D2 { double x, y; };
-struct F4 { float x, y, z, w; };
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
 struct F2 { float x, y; };
+// the workspace as 16-byte units of the global address space
+typedef __attribute__((address_space(1))) f64x2_t gf64x2;
+typedef __attribute__((address_space(1))) f32x4_t gf32x4;
+typedef __attribute__((address_space(1))) u32x4_t gu32x4;
 
 // buffer descriptor built from wave-uniform values (keeps it in SGPRs, so
 // buffer accesses need no waterfall loop)
@@ -1265,7 +1268,7 @@ __global__ __launch_bounds__(256) void k_lu_prep(const DevMesh* __restrict__ Ms)
   const double eps2 = C.epse * 2.;
   const double epsv = 1. + eps2;
   const LUGeom g = lu_geom(M);
-  D2* lu = reinterpret_cast<D2*>(M.lu);
+  gf64x2* lu = (gf64x2*)M.lu.p;
   const int tiles_t = (g.TD + LU64_PSTEPS - 1) / LU64_PSTEPS, tiles = lu64_prep_tiles(g);
   const bool top_in = g.nk % LU_R != 0;   // the halo row k = ke+1 is the last block's last row
   int c, kk, w = 0, t = -1;
@@ -1313,29 +1316,29 @@ __global__ __launch_bounds__(256) void k_lu_prep(const DevMesh* __restrict__ Ms)
   nb_k(q, L, eps2, +1, kf);
   nb_k(q, L, eps2, -1, kb);
   if (t >= 0) {
-    D2* rec = lu + ((long long)w * g.TD + t) * LU64_STEP + (kk - LU_R * w);
-    rec[0 * LU_R] = D2{jb.chk, jb.spec};
-    rec[1 * LU_R] = D2{kb.chk, kb.spec};
-    rec[2 * LU_R] = D2{L.uu, L.vv};
-    rec[3 * LU_R] = D2{L.uv2, L.ge};
-    rec[4 * LU_R] = D2{q.xx, q.xy};
-    rec[5 * LU_R] = D2{q.yx, q.yy};
-    rec[6 * LU_R] = D2{L.qx, L.qy};
-    rec[7 * LU_R] = interior ? D2{ts * 0.5, L.d} : D2{0.0, 1.0};
-    rec[8 * LU_R] = D2{jf.chk, jf.spec};
-    rec[9 * LU_R] = D2{kf.chk, kf.spec};
-    rec[10 * LU_R] = D2{st[0], st[1]};
-    rec[11 * LU_R] = D2{st[2], st[3]};
+    gf64x2* rec = lu + ((long long)w * g.TD + t) * LU64_STEP + (kk - LU_R * w);
+    rec[0 * LU_R] = f64x2_t{jb.chk, jb.spec};
+    rec[1 * LU_R] = f64x2_t{kb.chk, kb.spec};
+    rec[2 * LU_R] = f64x2_t{L.uu, L.vv};
+    rec[3 * LU_R] = f64x2_t{L.uv2, L.ge};
+    rec[4 * LU_R] = f64x2_t{q.xx, q.xy};
+    rec[5 * LU_R] = f64x2_t{q.yx, q.yy};
+    rec[6 * LU_R] = f64x2_t{L.qx, L.qy};
+    rec[7 * LU_R] = interior ? f64x2_t{ts * 0.5, L.d} : f64x2_t{0.0, 1.0};
+    rec[8 * LU_R] = f64x2_t{jf.chk, jf.spec};
+    rec[9 * LU_R] = f64x2_t{kf.chk, kf.spec};
+    rec[10 * LU_R] = f64x2_t{st[0], st[1]};
+    rec[11 * LU_R] = f64x2_t{st[2], st[3]};
   } else {
     const LUNb& b = kk < 0 ? kf : kb;
-    D2* h = lu + (kk < 0 ? g.off_hrf : g.off_hrb) + (c - 1);
-    h[0ll * g.ni] = D2{st[0], st[1]};
-    h[1ll * g.ni] = D2{st[2], st[3]};
-    h[2ll * g.ni] = D2{L.uu, L.vv};
-    h[3ll * g.ni] = D2{L.uv2, L.ge};
-    h[4ll * g.ni] = D2{q.yx, q.yy};
-    h[5ll * g.ni] = D2{0.0, L.qy};
-    h[6ll * g.ni] = D2{b.chk, b.spec};
+    gf64x2* h = lu + (kk < 0 ? g.off_hrf : g.off_hrb) + (c - 1);
+    h[0ll * g.ni] = f64x2_t{st[0], st[1]};
+    h[1ll * g.ni] = f64x2_t{st[2], st[3]};
+    h[2ll * g.ni] = f64x2_t{L.uu, L.vv};
+    h[3ll * g.ni] = f64x2_t{L.uv2, L.ge};
+    h[4ll * g.ni] = f64x2_t{q.yx, q.yy};
+    h[5ll * g.ni] = f64x2_t{0.0, L.qy};
+    h[6ll * g.ni] = f64x2_t{b.chk, b.spec};
   }
 }
 
@@ -1447,9 +1450,9 @@ __device__ __forceinline__ void lu32_term(const LUPrepLds& S, int n, bool halo, 
 
 // matrix row `row` of P with its columns in lane pair h's order: its own
 // pair (2h, 2h+1) first, then the other pair
-__device__ __forceinline__ F4 pair_row(const double* P, int row, int h) {
+__device__ __forceinline__ f32x4_t pair_row(const double* P, int row, int h) {
   const int o = 2 * h, p = 2 - 2 * h;
-  return F4{(float)P[row * 4 + o], (float)P[row * 4 + o + 1], (float)P[row * 4 + p], (float)P[row * 4 + p + 1]};
+  return f32x4_t{(float)P[row * 4 + o], (float)P[row * 4 + o + 1], (float)P[row * 4 + p], (float)P[row * 4 + p + 1]};
 }
 
 __global__ __launch_bounds__(64 * LP_WAVES) void k_lu_prep32(const DevMesh* __restrict__ Ms) {
@@ -1459,7 +1462,7 @@ __global__ __launch_bounds__(64 * LP_WAVES) void k_lu_prep32(const DevMesh* __re
   const double eps2 = M.c.epse * 2.;
   const double epsv = 1. + eps2;
   const LUGeom g = lu_geom(M);
-  D2* lu = reinterpret_cast<D2*>(M.lu);
+  gf32x4* lu = (gf32x4*)M.lu.p;
   constexpr int RG = LU32_R / 8;   // 8-row groups per block
   const int nthr = 64 * LP_WAVES;
   // tile of this workgroup: block w, rows 8*lb .. 8*lb+7, steps T0 .. T0+LP_STEPS-1
@@ -1507,8 +1510,8 @@ __global__ __launch_bounds__(64 * LP_WAVES) void k_lu_prep32(const DevMesh* __re
   lu32_term(S, n0 + 1, j == je, 1, -1, -f, eps2, gm1, QA, cb);
   lu32_term(S, n0 + LP_RJ, k == ke, 0, -1, -f, eps2, gm1, QB, cb);
   const long long rec = (long long)w * g.TA + t;
-  F4* rf = reinterpret_cast<F4*>(lu + g.off_f32 + rec * 288);
-  F4* rb = reinterpret_cast<F4*>(lu + g.off_b32 + rec * 256);
+  gf32x4* rf = lu + g.off_f32 + rec * 288;
+  gf32x4* rb = lu + g.off_b32 + rec * 256;
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     const int l = 2 * r + h;
@@ -1522,9 +1525,9 @@ __global__ __launch_bounds__(64 * LP_WAVES) void k_lu_prep32(const DevMesh* __re
     rb[3 * 64 + l] = pair_row(QB, 2 * h + 1, h);
   }
   // u of lanes 2r, 2r+1 and cB of the cell (both lanes' pairs, one unit)
-  rf[256 + r] = F4{(float)u[0], (float)u[1], (float)u[2], (float)u[3]};
-  reinterpret_cast<F4*>(lu + g.off_cb)[((long long)w * g.TW + t) * 32 + r] =
-      F4{(float)cb[0], (float)cb[1], (float)cb[2], (float)cb[3]};
+  rf[256 + r] = f32x4_t{(float)u[0], (float)u[1], (float)u[2], (float)u[3]};
+  (lu + g.off_cb)[((long long)w * g.TW + t) * 32 + r] =
+      f32x4_t{(float)cb[0], (float)cb[1], (float)cb[2], (float)cb[3]};
 }
 
 // Bounded waits.  Every wait of the FP32 sweeps gives up after LU32_WAIT
@@ -1626,7 +1629,7 @@ __global__ __launch_bounds__(64 * (2 + NP)) void k_lu_sweep32(const DevMesh* __r
   int2* tags = reinterpret_cast<int2*>(ring + (size_t)S * NV * 64);  // [S]: records, fill
   const DevMesh& M = Ms[blockIdx.y];
   const LUGeom g = lu_geom(M);
-  D2* lu = reinterpret_cast<D2*>(M.lu);
+  f64x2_t* lu = reinterpret_cast<f64x2_t*>(M.lu.p);
   if (threadIdx.x == 0) {
     consumed = 0;
     abort_flag = 0;
@@ -1998,7 +2001,7 @@ __global__ __launch_bounds__(64 * (2 + NP)) void k_lu_sweep64(const DevMesh* __r
   unsigned* stage = reinterpret_cast<unsigned*>(ring + (size_t)S * LU64_SLOT + (S * 8 + 15) / 16);   // [16][8]
   const DevMesh& M = Ms[blockIdx.y];
   const LUGeom g = lu_geom(M);
-  D2* lu = reinterpret_cast<D2*>(M.lu);
+  f64x2_t* lu = reinterpret_cast<f64x2_t*>(M.lu.p);
   if (threadIdx.x == 0) {
     consumed = 0;
     abort_flag = 0;
@@ -2052,17 +2055,17 @@ __global__ __launch_bounds__(64 * (2 + NP)) void k_lu_sweep64(const DevMesh* __r
     const int wn = w - DIR;
     gu64* const mail = (gu64*)(lu + (DIR > 0 ? g.off_dh : g.off_dh2));
     // operators: planes at unit `ob` + `oc` x column + `op` x plane
-    const D2* ob;
+    const gf64x2* ob;
     long long oc;
     int o_uv, o_ge, o_y, o_q, o_c;
     const long long hb = DIR > 0 ? g.off_hrf : g.off_hrb;
     if (from_block) {
       // edge row: row R-1 at record step c + R-1, or row 0 at step c
-      ob = lu + ((long long)wn * g.TD + (DIR > 0 ? R - 1 : 0)) * LU64_STEP + (DIR > 0 ? R - 1 : 0);
+      ob = (gf64x2*)lu + ((long long)wn * g.TD + (DIR > 0 ? R - 1 : 0)) * LU64_STEP + (DIR > 0 ? R - 1 : 0);
       oc = LU64_STEP;
       o_uv = 2 * R; o_ge = 3 * R; o_y = 5 * R; o_q = 6 * R; o_c = (DIR > 0 ? 9 : 1) * R;
     } else {
-      ob = lu + hb - 1;   // column c at entry c-1
+      ob = (gf64x2*)lu + hb - 1;   // column c at entry c-1
       oc = 1;
       o_uv = 2 * g.ni; o_ge = 3 * g.ni; o_y = 4 * g.ni; o_q = 5 * g.ni; o_c = 6 * g.ni;
     }
@@ -2071,8 +2074,8 @@ __global__ __launch_bounds__(64 * (2 + NP)) void k_lu_sweep64(const DevMesh* __r
       return DIR > 0 ? ec + 1 : g.ni - ec;
     };
     auto ops = [&](int e0, LU64Op& o) {
-      const D2* p = ob + oc * col(e0 + (l & 15));
-      const D2 a = p[o_uv], b = p[o_ge], y = p[o_y], q = p[o_q], c = p[o_c];
+      const gf64x2* p = ob + oc * col(e0 + (l & 15));
+      const f64x2_t a = p[o_uv], b = p[o_ge], y = p[o_y], q = p[o_q], c = p[o_c];
       o.uu = a.x; o.vv = a.y; o.uv2 = b.x; o.ge = b.y; o.ri1 = y.x; o.ri2 = y.y; o.qq = q.y;
       o.chk = c.x; o.spec = c.y;
     };
@@ -2118,8 +2121,8 @@ __global__ __launch_bounds__(64 * (2 + NP)) void k_lu_sweep64(const DevMesh* __r
       ops(e0 + 16, nxt);
       double s[4], b[4];
       if (!from_block) {
-        const D2* p = lu + hb + (col(e0 + (l & 15)) - 1);
-        const D2 a = p[0], c = p[g.ni];
+        const gf64x2* p = (gf64x2*)lu + hb + (col(e0 + (l & 15)) - 1);
+        const f64x2_t a = p[0], c = p[g.ni];
         s[0] = a.x; s[1] = a.y; s[2] = c.x; s[3] = c.y;
         lu64_apply(gm1, cur, s, b);
         ok = deliver(e0 + 1, 0, ne, b);
@@ -2329,8 +2332,8 @@ __global__ __launch_bounds__(256) void k_lu_finish(const DevMesh* __restrict__ M
   const int fuse_update = flags & 1, sa_prim = flags & 2;
   const int jd = M.jd, kd = M.kd, js = M.js, je = M.je, ks = M.ks, ke = M.ke;
   const LUGeom g = lu_geom(M);
-  const F4* H2 = reinterpret_cast<const F4*>(reinterpret_cast<const D2*>(M.lu) + g.off_h2);
-  const u32x4_t* D = reinterpret_cast<const u32x4_t*>(reinterpret_cast<const D2*>(M.lu) + g.off_dh2);
+  const gf32x4* H2 = (gf32x4*)M.lu.p + g.off_h2;
+  const gu32x4* D = (gu32x4*)M.lu.p + g.off_dh2;
   long long n2 = (long long)jd * kd;
   int bad = 0;
   for (long long i = blockIdx.x * 256ll + threadIdx.x; i < n2; i += 256ll * gridDim.x) {
@@ -2355,11 +2358,11 @@ __global__ __launch_bounds__(256) void k_lu_finish(const DevMesh* __restrict__ M
       double dq[4];
       if constexpr (sizeof(T) == 8) {
         const int kk = k - ks, r = kk % LU_R;
-        const u32x4_t* e = D + ((long long)(kk / LU_R) * g.TD + (j - js + 1) + r) * LU64_OUT + 2 * r;
+        const gu32x4* e = D + ((long long)(kk / LU_R) * g.TD + (j - js + 1) + r) * LU64_OUT + 2 * r;
         dq[0] = word_pair(e[0]); dq[2] = word_pair(e[1]); dq[1] = word_pair(e[64]); dq[3] = word_pair(e[65]);
       } else {
         const long long e = lu_entry32(M, g, j, k, -1);
-        const F4 a = H2[e], b = H2[e + 1];   // (value, tag) words
+        const f32x4_t a = H2[e], b = H2[e + 1];   // (value, tag) words
         dq[0] = (double)a.x; dq[1] = (double)a.z; dq[2] = (double)b.x; dq[3] = (double)b.z;
       }
       for (int n = 0; n < 4; ++n) M.s[n][i] = dq[n];
@@ -2423,10 +2426,10 @@ __global__ __launch_bounds__(256) void k_init_geometry(const DevMesh* __restrict
   const int t = threadIdx.x, nt = blockDim.x;
   const int jd = M.jd, kd = M.kd, jmax = M.jmax, kmax = M.kmax;
   const long long nv2 = (long long)jmax * kmax, n2 = (long long)jd * kd;
-  double* x = M.x;
-  double* y = M.y;
-  double* xv = M.xv;
-  double* yv = M.yv;
+  const gd_t x = M.x;
+  const gd_t y = M.y;
+  const gd_t xv = M.xv;
+  const gd_t yv = M.yv;
   const double pi = 4.0 * atan(1.0);
   if (metrics_only) goto metrics;
   // find_coord_TS for instances 2..nspec (src/setup.f:348-393)
@@ -2525,7 +2528,7 @@ __global__ __launch_bounds__(256) void k_init_geometry(const DevMesh* __restrict
   }
   // ---- metfv
 metrics:
-  double* qj = M.q[M.nq - 1];
+  const gd_t qj = M.q[M.nq - 1];
   for (long long w = t; w < (long long)(jmax - 1) * (kmax - 1); w += nt) {
     int j = 2 + (int)(w % (jmax - 1)), k = 2 + (int)(w / (jmax - 1));
     long long i = cell(M, j, k);  // jc = j, kc = k with one halo
@@ -2683,11 +2686,11 @@ __global__ __launch_bounds__(256) void k_forces(const DevMesh* __restrict__ Ms, 
   const int t = threadIdx.x;
   const int k = M.ks, k2 = k + 1, k3 = k2 + 1;
   const int j1 = M.jtail1, j2 = M.jtail2;
-  const double* q1 = M.q[0];
-  const double* q2 = M.q[1];
-  const double* q3 = M.q[2];
-  const double* q4 = M.q[3];
-  const double* qj = M.q[M.nq - 1];
+  const gd_t q1 = M.q[0];
+  const gd_t q2 = M.q[1];
+  const gd_t q3 = M.q[2];
+  const gd_t q4 = M.q[3];
+  const gd_t qj = M.q[M.nq - 1];
   const double fmm = C.fmm, halfv = C.half;
   double gm1 = C.gm1, gamma = C.gamma;
   double acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // cn, cc, cmle, cpinv, cnv, ccv, cmlev, cpv

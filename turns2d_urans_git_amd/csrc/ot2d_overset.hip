@@ -39,11 +39,11 @@ __global__ __launch_bounds__(256) void k_interp_donors(const DevMesh* __restrict
   int s = 0;
   for (int dk = -1; dk <= 1; ++dk)
     for (int dj = -1; dj <= 1; ++dj) c[s++] = cell(M, D.jj + dj, D.kk + dk);
-  const double* qj = M.q[M.nq - 1];
+  const gd_t qj = M.q[M.nq - 1];
   double* out = qbc + (size_t)d * nv;
   // conserved variables (q times J) for n <= nmv, raw turbulence variables
   for (int n = 0; n < nv; ++n) {
-    const double* q = M.q[n];
+    const gd_t q = M.q[n];
     double a;
     if (n < 4) {
       a = w[0] * q[c[0]] * qj[c[0]];

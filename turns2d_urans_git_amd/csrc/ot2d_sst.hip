@@ -56,10 +56,10 @@ __device__ __forceinline__ double findturm(double rho, double q5, double q6, dou
 __global__ __launch_bounds__(BC_THREADS) void k_sst_bc(const DevMesh* __restrict__ Ms, int eddy) {
   const DevMesh& M = Ms[blockIdx.x];
   if (*M.status) return;
-  double* q5 = M.q[4];
-  double* q6 = M.q[5];
-  const double* u = M.sa_u;
-  const double* v = M.sa_v;
+  const gd_t q5 = M.q[4];
+  const gd_t q6 = M.q[5];
+  const gd_t u = M.sa_u;
+  const gd_t v = M.sa_v;
   const double rei = 1. / M.c.rey;
   const int t = threadIdx.x, nt = blockDim.x;
   for (int ib = 0; ib < M.nbc; ++ib) {
@@ -198,10 +198,10 @@ __global__ __launch_bounds__(256) void k_sst_blend(const DevMesh* __restrict__ M
   if (*M.status) return;
   const int jd = M.jd, js = M.js, je = M.je, ks = M.ks, ke = M.ke;
   const double rei = 1. / M.c.rey;
-  const double* q5 = M.q[4];
-  const double* q6 = M.q[5];
-  const double* u = M.sa_u;
-  const double* v = M.sa_v;
+  const gd_t q5 = M.q[4];
+  const gd_t q6 = M.q[5];
+  const gd_t u = M.sa_u;
+  const gd_t v = M.sa_v;
   long long n2 = (long long)jd * M.kd;
   for (long long i = blockIdx.x * 256ll + threadIdx.x; i < n2; i += 256ll * gridDim.x) {
     const int j = 1 + (int)(i % jd), k = 1 + (int)(i / jd);
@@ -253,7 +253,7 @@ __global__ __launch_bounds__(256) void k_sst_blend(const DevMesh* __restrict__ M
 
 // j-face diffusion coefficient and difference of equation n between cells
 // a and b = a+1 (src/komegasst.f:630-636, 676-682)
-__device__ __forceinline__ void kw_half(const DevMesh& M, long long a, long long b, const double* qn, double s1,
+__device__ __forceinline__ void kw_half(const DevMesh& M, long long a, long long b, const gd_t& qn, double s1,
                                         double s2, double rei, double& chp, double& dn) {
   double vnulh = 0.5 * (M.sa_vmul[a] + M.sa_vmul[b]);
   double vnuh = 0.5 * (M.turmu[a] + M.turmu[b]);
@@ -273,10 +273,10 @@ __global__ __launch_bounds__(256) void k_sst_rhs(const DevMesh* __restrict__ Ms)
   const int jd = M.jd, js = M.js, je = M.je, ks = M.ks, ke = M.ke;
   const int nj = je - js + 1, nk = ke - ks + 1;
   const double rey = C.rey, rei = 1. / rey;
-  const double* xx = M.xx;
-  const double* xy = M.xy;
-  const double* yx = M.yx;
-  const double* yy = M.yy;
+  const gd_t xx = M.xx;
+  const gd_t xy = M.xy;
+  const gd_t yx = M.yx;
+  const gd_t yy = M.yy;
   long long ncell = (long long)nj * nk;
   for (long long w = blockIdx.x * 256ll + threadIdx.x; w < ncell; w += 256ll * gridDim.x) {
     const int j = js + (int)(w % nj), k = ks + (int)(w / nj);
@@ -291,7 +291,7 @@ __global__ __launch_bounds__(256) void k_sst_rhs(const DevMesh* __restrict__ Ms)
     double sj[2], aj[2], bj[2], cj[2], ak[2], ck[2];
 #pragma unroll
     for (int n = 0; n < 2; ++n) {
-      const double* qn = M.q[4 + n];
+      const gd_t qn = M.q[4 + n];
       double s = M.s[4 + n][i];
       s = s - up * (qn[i] - qn[iw]) - um * (qn[ie] - qn[i]);
       aj[n] = 0.0 - up;
@@ -445,8 +445,8 @@ __global__ __launch_bounds__(512) void k_sst_solve_k(const DevMesh* __restrict__
     q[u] = gq[i]; q1[u] = g1[i]; qj[u] = gj[i]; ib[u] = M.iblank[i];
   }
   part_columns<2 * TC>(a, b, c, s, P, sst_ex);
-  double* qn = eq ? M.q[5] : M.q[4];
-  double* sn = eq ? M.s[5] : M.s[4];
+  const gd_t qn = eq ? M.q[5] : M.q[4];
+  const gd_t sn = eq ? M.s[5] : M.s[4];
 #pragma unroll
   for (int u = 0; u < PM; ++u) {
     const double ds = 1. * s[u];

@@ -246,7 +246,7 @@ __global__ __launch_bounds__(VIS_THREADS) void k_visrhs(const DevMesh* __restric
   const double c2b = 198.6 / C.tinf, c2bp = c2b + 1.;
   const int j0 = M.js + ((int)blockIdx.x % tiles_j) * VIS_TJ, k0 = M.ks + ((int)blockIdx.x / tiles_j) * VIS_TK;
   const int t = threadIdx.x;
-  const double* qj = M.q[M.nq - 1];
+  const gd_t qj = M.q[M.nq - 1];
 
   // tile and ring: primitives (src/visrhs.f:47-57), quotient primitives
   // (src/visrhs.f:108-119), metrics and 1/q(nq)
@@ -418,9 +418,9 @@ __device__ __forceinline__ void c_turm_cell(const DevMesh& M, long long i, int o
 
 // turbc (src/samodel2d.f:827-1303) for one boundary segment
 __device__ void turbc_segment(const DevMesh& M, const DevBC& b) {
-  double* q5 = M.q[4];
-  const double* u = M.sa_u;
-  const double* v = M.sa_v;
+  const gd_t q5 = M.q[4];
+  const gd_t u = M.sa_u;
+  const gd_t v = M.sa_v;
   const int t = threadIdx.x, nt = blockDim.x;
   {
     int js = b.js, je = b.je, ks = b.ks, ke = b.ke, idir = b.idir;
@@ -537,78 +537,100 @@ __global__ __launch_bounds__(BC_THREADS) void k_turbc_eddy(const DevMesh* __rest
   }
 }
 
-// convective upwind speeds of a cell (src/samodel2d.f:483-491)
-struct UpDown { double up, um, vp, vm; };
-__device__ __forceinline__ UpDown sa_updown(const DevMesh& M, long long i) {
-  double ug = M.has_gv ? M.ug[i] : 0.0, vg = M.has_gv ? M.vg[i] : 0.0;
-  double u = M.sa_u[i], v = M.sa_v[i];
-  double uu = M.xx[i] * (u - ug) + M.xy[i] * (v - vg);
-  double vv = M.yx[i] * (u - ug) + M.yy[i] * (v - vg);
-  UpDown o;
-  o.up = 0.5 * (uu + fabs(uu)); o.um = 0.5 * (uu - fabs(uu));
-  o.vp = 0.5 * (vv + fabs(vv)); o.vm = 0.5 * (vv - fabs(vv));
-  return o;
-}
-
-__device__ __forceinline__ double sa_vnul(const DevMesh& M, long long i) {
-  return M.sa_vmul[i] / M.q[0][i] / M.q[M.nq - 1][i];
-}
+// convective upwind speeds of a contravariant velocity (src/samodel2d.f:483-491)
+struct UpDown { double p, m; };
+__device__ __forceinline__ UpDown sa_updown(double uu) { return {0.5 * (uu + fabs(uu)), 0.5 * (uu - fabs(uu))}; }
 
 // diffusion half-point coefficient chp and difference dnuhp of the face
-// between cells a and b (src/samodel2d.f:575-584, 622-631)
-__device__ __forceinline__ void sa_half(const DevMesh& M, long long a, long long b, double rey, double& chp,
+// between cells with (vnul, nu-tilde) a and b (src/samodel2d.f:575-584, 622-631)
+__device__ __forceinline__ void sa_half(double va, double na, double vb, double nb, double rey, double& chp,
                                         double& dn) {
-  double vnulh = 0.5 * (sa_vnul(M, a) + sa_vnul(M, b));
-  double vnuh = 0.5 * (M.q[4][a] + M.q[4][b]);
+  double vnulh = 0.5 * (va + vb);
+  double vnuh = 0.5 * (na + nb);
   chp = (1. + SA_cb2) / SA_sigma / rey * (vnulh + vnuh);
-  dn = M.q[4][b] - M.q[4][a];
+  dn = nb - na;
 }
 
 // rhslhs (convec + diffus + source) and the pseudo-time scaling of vmu_sa
-// (src/samodel2d.f:101-131, 402-824) for every interior cell, in gather
-// form: each cell assembles its own row of the two tridiagonal systems.
-__global__ __launch_bounds__(256) void k_sa_rhs(const DevMesh* __restrict__ Ms) {
+// (src/samodel2d.f:101-131, 402-824), in gather form: each cell assembles its
+// own row of the two tridiagonal systems.  A workgroup takes a 32x8 tile:
+// what the stencil reads of a cell (nu-tilde, vnul, contravariant velocities,
+// velocities, metrics) is formed once for the tile and its one-cell ring in
+// LDS.  Bound by FP64 issue (about 1100 operations a cell, 40 divisions among
+// them).  60 cases (3.9 M cells): 178 us; with every thread gathering its
+// neighbours' planes and forming their quantities again 256 us (two
+// divisions a neighbour, 160-220 registers).  513x129: 9 us both ways.
+constexpr int SAR_N = VIS_NR;
+struct SaLds {
+  double nt[SAR_N], vn[SAR_N], U[SAR_N], V[SAR_N], u[SAR_N], v[SAR_N], xx[SAR_N], xy[SAR_N], yx[SAR_N], yy[SAR_N];
+};
+
+__global__ __launch_bounds__(VIS_THREADS, 4) void k_sa_rhs(const DevMesh* __restrict__ Ms) {
+  __shared__ SaLds L;
   const DevMesh& M = Ms[blockIdx.y];
-  if (*M.status) return;
-  const DevConst& C = M.c;
   const int js = M.js, je = M.je, ks = M.ks, ke = M.ke;
   const int nj = je - js + 1, nk = ke - ks + 1;
+  const int tiles_j = (nj + VIS_TJ - 1) / VIS_TJ;
+  if ((int)blockIdx.x >= tiles_j * ((nk + VIS_TK - 1) / VIS_TK) || *M.status) return;
+  const DevConst& C = M.c;
   const double rey = C.rey;
-  const double* q5 = M.q[4];
-  const double* xx = M.xx;
-  const double* xy = M.xy;
-  const double* yx = M.yx;
-  const double* yy = M.yy;
-  long long ncell = (long long)nj * nk;
-  for (long long w = blockIdx.x * 256ll + threadIdx.x; w < ncell; w += 256ll * gridDim.x) {
-    const int j = js + (int)(w % nj), k = ks + (int)(w / nj);
+  const int j0 = js + ((int)blockIdx.x % tiles_j) * VIS_TJ, k0 = ks + ((int)blockIdx.x / tiles_j) * VIS_TK;
+  const int t = threadIdx.x;
+  for (int n = t; n < SAR_N; n += VIS_THREADS) {
+    const int j = j0 - 1 + n % VIS_RJ, k = k0 - 1 + n / VIS_RJ;
+    if (j > je + 1 || k > ke + 1) continue;
     const long long i = cell(M, j, k);
-    const long long iw = cell(M, j - 1, k), ie = cell(M, j + 1, k), is = cell(M, j, k - 1), in = cell(M, j, k + 1);
-    UpDown c = sa_updown(M, i);
-    UpDown cw = sa_updown(M, iw), ce = sa_updown(M, ie), cs = sa_updown(M, is), cn = sa_updown(M, in);
-    double nt = q5[i];
+    const double u = M.sa_u[i], v = M.sa_v[i], xx = M.xx[i], xy = M.xy[i], yx = M.yx[i], yy = M.yy[i];
+    const double vmul = M.sa_vmul[i], q1 = M.q[0][i], qn = M.q[M.nq - 1][i], nt = M.q[4][i];
+    const double ug = M.has_gv ? M.ug[i] : 0.0, vg = M.has_gv ? M.vg[i] : 0.0;
+    L.nt[n] = nt;
+    L.vn[n] = vmul / q1 / qn;
+    L.U[n] = xx * (u - ug) + xy * (v - vg);
+    L.V[n] = yx * (u - ug) + yy * (v - vg);
+    L.u[n] = u; L.v[n] = v; L.xx[n] = xx; L.xy[n] = xy; L.yx[n] = yx; L.yy[n] = yy;
+  }
+  __syncthreads();
+  const int j = j0 + t % VIS_TJ, k = k0 + t / VIS_TJ;
+  if (j <= je && k <= ke) {
+    const long long i = cell(M, j, k);
+    const int c = (t / VIS_TJ + 1) * VIS_RJ + t % VIS_TJ + 1, w = c - 1, e = c + 1, s = c - VIS_RJ, n = c + VIS_RJ;
+    const double nt = L.nt[c], vnul = L.vn[c];
+    const double xx = L.xx[c], xy = L.xy[c], yx = L.yx[c], yy = L.yy[c];
     // ---- convec (src/samodel2d.f:493-538)
     double sj = M.s[4][i];
-    sj = sj - c.up * (nt - q5[iw]) - c.um * (q5[ie] - nt);
-    sj = sj - c.vp * (nt - q5[is]) - c.vm * (q5[in] - nt);
     double aj = 0.0, bj = 0.0, cj = 0.0, ak = 0.0, bk = 0.0, ck = 0.0;
-    if (j > js) aj = aj - (c.up > 1.0e-12 ? 1.0 : 0.0) * (cw.up + cw.um);
-    bj = bj + c.up - c.um;
-    if (j < je) cj = cj + (c.um < -1.0e-12 ? 1.0 : 0.0) * (ce.up + ce.um);
-    if (k > ks) ak = ak - (c.vp > 1.0e-12 ? 1.0 : 0.0) * (cs.vp + cs.vm);
-    bk = bk + c.vp - c.vm;
-    if (k < ke) ck = ck + (c.vm < -1.0e-12 ? 1.0 : 0.0) * (cn.vp + cn.vm);
+    const UpDown cu = sa_updown(L.U[c]), cv = sa_updown(L.V[c]);
+    sj = sj - cu.p * (nt - L.nt[w]) - cu.m * (L.nt[e] - nt);
+    sj = sj - cv.p * (nt - L.nt[s]) - cv.m * (L.nt[n] - nt);
+    if (j > js) {
+      const UpDown x = sa_updown(L.U[w]);
+      aj = aj - (cu.p > 1.0e-12 ? 1.0 : 0.0) * (x.p + x.m);
+    }
+    bj = bj + cu.p - cu.m;
+    if (j < je) {
+      const UpDown x = sa_updown(L.U[e]);
+      cj = cj + (cu.m < -1.0e-12 ? 1.0 : 0.0) * (x.p + x.m);
+    }
+    if (k > ks) {
+      const UpDown x = sa_updown(L.V[s]);
+      ak = ak - (cv.p > 1.0e-12 ? 1.0 : 0.0) * (x.p + x.m);
+    }
+    bk = bk + cv.p - cv.m;
+    if (k < ke) {
+      const UpDown x = sa_updown(L.V[n]);
+      ck = ck + (cv.m < -1.0e-12 ? 1.0 : 0.0) * (x.p + x.m);
+    }
     // ---- diffus, j direction (src/samodel2d.f:570-607)
     {
       double chpm, dnm, chpp, dnp;
-      sa_half(M, iw, i, rey, chpm, dnm);
-      sa_half(M, i, ie, rey, chpp, dnp);
-      double dmxhm = 0.5 * (xx[iw] + xx[i]), dmyhm = 0.5 * (xy[iw] + xy[i]);
-      double dmxhp = 0.5 * (xx[i] + xx[ie]), dmyhp = 0.5 * (xy[i] + xy[ie]);
-      double dxp = dmxhp * xx[i] + dmyhp * xy[i];
-      double dxm = dmxhm * xx[i] + dmyhm * xy[i];
+      sa_half(L.vn[w], L.nt[w], vnul, nt, rey, chpm, dnm);
+      sa_half(vnul, nt, L.vn[e], L.nt[e], rey, chpp, dnp);
+      double dmxhm = 0.5 * (L.xx[w] + xx), dmyhm = 0.5 * (L.xy[w] + xy);
+      double dmxhp = 0.5 * (xx + L.xx[e]), dmyhp = 0.5 * (xy + L.xy[e]);
+      double dxp = dmxhp * xx + dmyhp * xy;
+      double dxm = dmxhm * xx + dmyhm * xy;
       double c2 = SA_cb2 / SA_sigma / rey;
-      c2 = c2 * (sa_vnul(M, i) + nt);
+      c2 = c2 * (vnul + nt);
       double dcp = dxp * (chpp - c2);
       double dcm = dxm * (chpm - c2);
       double ax = fmax(dcm, 0.0), cx = fmax(dcp, 0.0);
@@ -620,14 +642,14 @@ __global__ __launch_bounds__(256) void k_sa_rhs(const DevMesh* __restrict__ Ms) 
     // ---- diffus, k direction (src/samodel2d.f:617-654)
     {
       double chpm, dnm, chpp, dnp;
-      sa_half(M, is, i, rey, chpm, dnm);
-      sa_half(M, i, in, rey, chpp, dnp);
-      double dmxhm = 0.5 * (yx[is] + yx[i]), dmyhm = 0.5 * (yy[is] + yy[i]);
-      double dmxhp = 0.5 * (yx[i] + yx[in]), dmyhp = 0.5 * (yy[i] + yy[in]);
-      double dyp = dmxhp * yx[i] + dmyhp * yy[i];
-      double dym = dmxhm * yx[i] + dmyhm * yy[i];
+      sa_half(L.vn[s], L.nt[s], vnul, nt, rey, chpm, dnm);
+      sa_half(vnul, nt, L.vn[n], L.nt[n], rey, chpp, dnp);
+      double dmxhm = 0.5 * (L.yx[s] + yx), dmyhm = 0.5 * (L.yy[s] + yy);
+      double dmxhp = 0.5 * (yx + L.yx[n]), dmyhp = 0.5 * (yy + L.yy[n]);
+      double dyp = dmxhp * yx + dmyhp * yy;
+      double dym = dmxhm * yx + dmyhm * yy;
       double c2 = SA_cb2 / SA_sigma / rey;
-      c2 = c2 * (sa_vnul(M, i) + nt);
+      c2 = c2 * (vnul + nt);
       double dcp = dyp * (chpp - c2);
       double dcm = dym * (chpm - c2);
       double ay = fmax(dcm, 0.0), cy = fmax(dcp, 0.0);
@@ -640,15 +662,14 @@ __global__ __launch_bounds__(256) void k_sa_rhs(const DevMesh* __restrict__ Ms) 
     {
       double vort = 0.0;
       if (M.bodyflag) {
-        double ux = (M.sa_u[ie] - M.sa_u[iw]) * 0.5;
-        double vx = (M.sa_v[ie] - M.sa_v[iw]) * 0.5;
-        double uy = (M.sa_u[in] - M.sa_u[is]) * 0.5;
-        double vy = (M.sa_v[in] - M.sa_v[is]) * 0.5;
-        vort = fabs(xy[i] * ux - xx[i] * vx + yy[i] * uy - yx[i] * vy);
+        double ux = (L.u[e] - L.u[w]) * 0.5;
+        double vx = (L.v[e] - L.v[w]) * 0.5;
+        double uy = (L.u[n] - L.u[s]) * 0.5;
+        double vy = (L.v[n] - L.v[s]) * 0.5;
+        vort = fabs(xy * ux - xx * vx + yy * uy - yx * vy);
       }
       const double d2min = 1.e-12, rmax = 10.0, stilim = 1.e-12, fturf = 0.0;
       const double cv1_3 = ip3(SA_cv1), cw3_6 = ip6(SA_cw3);
-      double vnul = sa_vnul(M, i);
       double chi = nt / vnul;
       double d = M.sa_sn[i];
       chi = fmax(chi, 1.e-12);
@@ -815,13 +836,19 @@ static long long max_cells(const DevMesh* hM, int nmi) {
   return mx;
 }
 
-hipError_t launch_visrhs(const DevMesh* dM, const DevMesh* hM, int nmi, hipStream_t st, int norms) {
+// 32x8 tiles of the largest instance
+static int vis_tiles(const DevMesh* hM, int nmi) {
   int tiles = 1;
   for (int i = 0; i < nmi; ++i) {
     const int nj = hM[i].je - hM[i].js + 1, nk = hM[i].ke - hM[i].ks + 1;
     const int n = ((nj + VIS_TJ - 1) / VIS_TJ) * ((nk + VIS_TK - 1) / VIS_TK);
     tiles = n > tiles ? n : tiles;
   }
+  return tiles;
+}
+
+hipError_t launch_visrhs(const DevMesh* dM, const DevMesh* hM, int nmi, hipStream_t st, int norms) {
+  const int tiles = vis_tiles(hM, nmi);
   static bool lds_set = false;
   if (!lds_set) {
     hipError_t e = hipFuncSetAttribute((const void*)k_visrhs, hipFuncAttributeMaxDynamicSharedMemorySize, (int)VIS_LDS);
@@ -880,7 +907,7 @@ hipError_t launch_sa(const DevMesh* dM, const DevMesh* hM, int nmi, Marks* mk, h
   mark(mk, OT2D_ST_SA_PRIM, st);
   if ((e = launch_turbc(dM, hM, nmi, st)) != hipSuccess) return e;
   mark(mk, OT2D_ST_SA_BC, st);
-  hipLaunchKernelGGL(k_sa_rhs, dim3(nblk2(mx, 256), nmi), dim3(256), 0, st, dM);
+  hipLaunchKernelGGL(k_sa_rhs, dim3(vis_tiles(hM, nmi), nmi), dim3(VIS_THREADS), 0, st, dM);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_SA_RHS, st);
   hipLaunchKernelGGL(k_sa_solve_j, dim3(mk_, nmi), dim3(64), 0, st, dM);
