@@ -149,32 +149,22 @@ __device__ __forceinline__ DivPrim div_prim(const DevMesh& M, long long i) {
   return div_prim_of(M.q[0][i], M.q[1][i], M.q[2][i], M.q[3][i]);
 }
 
-// cross-derivative term of the eta line at cell c from its j neighbours
-// (src/visrhs.f:106-146)
-__device__ __forceinline__ Tri eta_cross(const VisCoef& c, const DivPrim& p, const DivPrim& m) {
-  double duj = 0.5 * (p.u - m.u), dvj = 0.5 * (p.v - m.v), dej = 0.5 * (p.e - m.e);
+// cross-derivative term of a line at a cell from its neighbours across the
+// line: the eta line's from its j neighbours (src/visrhs.f:106-146), the xi
+// line's from its k neighbours (src/visrhs.f:227-268).  The coefficients of
+// the two velocity gradients change places between them.
+__device__ __forceinline__ Tri vis_cross(const VisCoef& c, const DivPrim& p, const DivPrim& m, bool eta) {
+  const double du = 0.5 * (p.u - m.u), dv = 0.5 * (p.v - m.v), de = 0.5 * (p.e - m.e);
+  const double d5 = eta ? c.d5 : c.d7, d7 = eta ? c.d7 : c.d5;
   Tri f;
-  f.f2 = c.d1 * duj + c.d5 * dvj;
-  f.f3 = c.d7 * duj + c.d2 * dvj;
+  f.f2 = c.d1 * du + d5 * dv;
+  f.f3 = d7 * du + c.d2 * dv;
   double t = 0.5 * c.d1 * 0.5 * (sqd(p.u) - sqd(m.u));
   t = t + 0.5 * c.d2 * 0.5 * (sqd(p.v) - sqd(m.v));
-  t = t + c.d5 * 0.5 * (p.u + m.u) * dvj;
-  t = t + c.d7 * 0.5 * (p.v + m.v) * duj;
-  f.f4 = t + c.d4 * dej;
-  return f;
-}
-
-// cross-derivative term of the xi line (src/visrhs.f:227-268)
-__device__ __forceinline__ Tri xi_cross(const VisCoef& c, const DivPrim& p, const DivPrim& m) {
-  double duk = 0.5 * (p.u - m.u), dvk = 0.5 * (p.v - m.v), dek = 0.5 * (p.e - m.e);
-  Tri f;
-  f.f2 = c.d1 * duk + c.d7 * dvk;
-  f.f3 = c.d5 * duk + c.d2 * dvk;
-  double t = 0.5 * c.d1 * 0.5 * (sqd(p.u) - sqd(m.u));
-  t = t + 0.5 * c.d2 * 0.5 * (sqd(p.v) - sqd(m.v));
-  t = t + c.d5 * 0.5 * (p.v + m.v) * duk;
-  t = t + c.d7 * 0.5 * (p.u + m.u) * dvk;
-  f.f4 = t + c.d4 * dek;
+  const double su = p.u + m.u, sv = p.v + m.v;
+  t = t + c.d5 * 0.5 * (eta ? su : sv) * (eta ? dv : du);
+  t = t + c.d7 * 0.5 * (eta ? sv : su) * (eta ? du : dv);
+  f.f4 = t + c.d4 * de;
   return f;
 }
 
@@ -191,18 +181,35 @@ constexpr int VIS_NR = VIS_RJ * VIS_RK;   // tile and ring, ring row 0 = k0-1, c
 constexpr int VIS_NE = VIS_TJ * VIS_RK;   // eta cells: tile columns, rows k0-1 .. k0+TK
 constexpr int VIS_NX = VIS_RJ * VIS_TK;   // xi cells: columns j0-1 .. j0+TJ, tile rows
 
+// The first phase's per-cell quantities that only the coefficients read and
+// the coefficients themselves share their memory: each thread holds its (at
+// most VIS_PER) coefficient cells in registers across a barrier.
+constexpr int VIS_PER = (VIS_NE + VIS_NX + VIS_THREADS - 1) / VIS_THREADS;
 struct VisLds {
-  double u[VIS_NR], v[VIS_NR], e[VIS_NR], vnu[VIS_NR], gkap[VIS_NR];
-  double du[VIS_NR], dv[VIS_NR], de[VIS_NR];
-  double xx[VIS_NR], xy[VIS_NR], yx[VIS_NR], yy[VIS_NR], r[VIS_NR];
-  double ec[4][VIS_NE], eg[3][VIS_NE];     // eta: c1 c2 c5 c4 and the cross term
-  double xc[4][VIS_NX], xg[3][VIS_NX];     // xi
+  double u[VIS_NR], v[VIS_NR], e[VIS_NR];
+  union {
+    struct {
+      double vnu[VIS_NR], gkap[VIS_NR], du[VIS_NR], dv[VIS_NR], de[VIS_NR];
+      double xx[VIS_NR], xy[VIS_NR], yx[VIS_NR], yy[VIS_NR], r[VIS_NR];
+    };
+    struct {
+      double ec[4][VIS_NE], eg[3][VIS_NE];     // eta: c1 c2 c5 c4 and the cross term
+      double xc[4][VIS_NX], xg[3][VIS_NX];     // xi
+    };
+    double red[4][RES_THREADS];
+  };
 };
 constexpr size_t VIS_LDS = sizeof(VisLds);
 
 __device__ __forceinline__ VisPrim lds_prim(const VisLds& L, int c) {
   VisPrim p;
   p.u = L.u[c]; p.v = L.v[c]; p.e = L.e[c]; p.vnu = L.vnu[c]; p.gkap = L.gkap[c];
+  return p;
+}
+// the face fluxes read u, v and e only
+__device__ __forceinline__ VisPrim lds_uve(const VisLds& L, int c) {
+  VisPrim p;
+  p.u = L.u[c]; p.v = L.v[c]; p.e = L.e[c]; p.vnu = 0.; p.gkap = 0.;
   return p;
 }
 __device__ __forceinline__ DivPrim lds_div(const VisLds& L, int c) {
@@ -228,13 +235,16 @@ __device__ __forceinline__ Tri lds_tri(const double (&g)[3][N], int c) {
   return f;
 }
 
+// Bound by latency at the 12 waves a CU its LDS (41 KB) and registers (168)
+// allow; FP64 issue alone is 97 us of the 60-case batch's 228 us (286 us with
+// each array in memory of its own, 77 KB and 8 waves a CU); 513x129: 9.7 us
+// both ways.
 // With norms set, the residual is complete once this kernel has added the
 // viscous terms, so each tile also takes its residual-norm partials here
 // (the tiles and thread-to-cell map are the residual's: 32x8 tiles, k-tile
 // major), instead of a separate pass over s.
-__global__ __launch_bounds__(VIS_THREADS) void k_visrhs(const DevMesh* __restrict__ Ms, int norms) {
+__global__ __launch_bounds__(VIS_THREADS, 3) void k_visrhs(const DevMesh* __restrict__ Ms, int norms) {
   static_assert(VIS_TJ == RES_TJ && VIS_TK == RES_TK, "visrhs tiles are the residual's");
-  __shared__ double red[4][RES_THREADS];
   const DevMesh& M = Ms[blockIdx.y];
   const int nj = M.je - M.js + 1, nk = M.ke - M.ks + 1;
   const int tiles_j = (nj + VIS_TJ - 1) / VIS_TJ;
@@ -266,25 +276,33 @@ __global__ __launch_bounds__(VIS_THREADS) void k_visrhs(const DevMesh* __restric
 
   // coefficients and cross terms: eta along the tile columns for rows
   // k0-1 .. k0+TK, xi along the tile rows for columns j0-1 .. j0+TJ
-  for (int n = t; n < VIS_NE + VIS_NX; n += VIS_THREADS) {
-    if (n < VIS_NE) {
-      const int a = n % VIS_TJ, b = n / VIS_TJ;
-      if (j0 + a > M.je || k0 - 1 + b > M.ke + 1) continue;
-      const int c = b * VIS_RJ + a + 1;
-      const VisCoef o = vis_coef(L.yx[c], L.yy[c], L.r[c], lds_met(L, c - 1), lds_met(L, c + 1), lds_prim(L, c), dre,
-                                 gkpr);
-      const Tri g = eta_cross(o, lds_div(L, c + 1), lds_div(L, c - 1));
-      L.ec[0][n] = o.c1; L.ec[1][n] = o.c2; L.ec[2][n] = o.c5; L.ec[3][n] = o.c4;
-      L.eg[0][n] = g.f2; L.eg[1][n] = g.f3; L.eg[2][n] = g.f4;
-    } else {
-      const int m = n - VIS_NE, a = m % VIS_RJ, b = m / VIS_RJ;
-      if (j0 - 1 + a > M.je + 1 || k0 + b > M.ke) continue;
-      const int c = (b + 1) * VIS_RJ + a;
-      const VisCoef o = vis_coef(L.xx[c], L.xy[c], L.r[c], lds_met(L, c - VIS_RJ), lds_met(L, c + VIS_RJ),
-                                 lds_prim(L, c), dre, gkpr);
-      const Tri g = xi_cross(o, lds_div(L, c + VIS_RJ), lds_div(L, c - VIS_RJ));
-      L.xc[0][m] = o.c1; L.xc[1][m] = o.c2; L.xc[2][m] = o.c5; L.xc[3][m] = o.c4;
-      L.xg[0][m] = g.f2; L.xg[1][m] = g.f3; L.xg[2][m] = g.f4;
+  double oc[VIS_PER][7];
+#pragma unroll
+  for (int u = 0; u < VIS_PER; ++u) {
+    const int n = t + VIS_THREADS * u;
+    if (n >= VIS_NE + VIS_NX) break;
+    const bool eta = n < VIS_NE;
+    const int m = n - VIS_NE;
+    const int a = eta ? n % VIS_TJ : m % VIS_RJ, b = eta ? n / VIS_TJ : m / VIS_RJ;
+    if (eta ? (j0 + a > M.je || k0 - 1 + b > M.ke + 1) : (j0 - 1 + a > M.je + 1 || k0 + b > M.ke)) continue;
+    // the cell, and the step to its neighbours across the line
+    const int c = eta ? b * VIS_RJ + a + 1 : (b + 1) * VIS_RJ + a, d = eta ? 1 : VIS_RJ;
+    const VisCoef o = vis_coef(eta ? L.yx[c] : L.xx[c], eta ? L.yy[c] : L.xy[c], L.r[c], lds_met(L, c - d),
+                               lds_met(L, c + d), lds_prim(L, c), dre, gkpr);
+    const Tri g = vis_cross(o, lds_div(L, c + d), lds_div(L, c - d), eta);
+    oc[u][0] = o.c1; oc[u][1] = o.c2; oc[u][2] = o.c5; oc[u][3] = o.c4;
+    oc[u][4] = g.f2; oc[u][5] = g.f3; oc[u][6] = g.f4;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < VIS_PER; ++u) {
+    const int n = t + VIS_THREADS * u;
+    if (n >= VIS_NE + VIS_NX) break;
+    const int m = n - VIS_NE;
+#pragma unroll
+    for (int q = 0; q < 7; ++q) {
+      if (n < VIS_NE) (q < 4 ? L.ec[q & 3] : L.eg[q - 4])[n] = oc[u][q];
+      else (q < 4 ? L.xc[q & 3] : L.xg[q - 4])[m] = oc[u][q];
     }
   }
   __syncthreads();
@@ -299,13 +317,13 @@ __global__ __launch_bounds__(VIS_THREADS) void k_visrhs(const DevMesh* __restric
     const long long i = cell(M, j, k);
     double s2 = M.s[1][i], s3 = M.s[2][i], s4 = M.s[3][i];
     const int c = (b + 1) * VIS_RJ + a + 1;
-    const VisPrim p1 = lds_prim(L, c);
+    const VisPrim p1 = lds_uve(L, c);
     // ---- eta part (j = const line): faces k-1|k, k|k+1, cross terms
     {
       const int e = (b + 1) * VIS_TJ + a;
       const VisCoef c0 = lds_coef(L.ec, e - VIS_TJ), c1 = lds_coef(L.ec, e), c2 = lds_coef(L.ec, e + VIS_TJ);
-      const Tri fm = vis_face(lds_prim(L, c - VIS_RJ), c0, p1, c1);   // face k-1
-      const Tri fp = vis_face(p1, c1, lds_prim(L, c + VIS_RJ), c2);   // face k
+      const Tri fm = vis_face(lds_uve(L, c - VIS_RJ), c0, p1, c1);   // face k-1
+      const Tri fp = vis_face(p1, c1, lds_uve(L, c + VIS_RJ), c2);   // face k
       const Tri gm = lds_tri(L.eg, e - VIS_TJ), gc = lds_tri(L.eg, e);
       if (k < M.ke) {
         const Tri gp = lds_tri(L.eg, e + VIS_TJ);
@@ -319,7 +337,7 @@ __global__ __launch_bounds__(VIS_THREADS) void k_visrhs(const DevMesh* __restric
         } else {  // row k-2 lies below the tile's ring
           const VisPrim pq = vis_prim(M, cell(M, j, k - 2), c2b, c2bp, prtr);
           const VisCoef cq = eta_coef(M, j, k - 2, pq, dre, gkpr);
-          gq = eta_cross(cq, div_prim(M, cell(M, j + 1, k - 2)), div_prim(M, cell(M, j - 1, k - 2)));
+          gq = vis_cross(cq, div_prim(M, cell(M, j + 1, k - 2)), div_prim(M, cell(M, j - 1, k - 2)), true);
         }
         s2 = s2 + (fp.f2 - fm.f2) + 0.5 * (gq.f2 - 4. * gm.f2 + 3 * gc.f2);
         s3 = s3 + (fp.f3 - fm.f3) + 0.5 * (gq.f3 - 4. * gm.f3 + 3 * gc.f3);
@@ -330,8 +348,8 @@ __global__ __launch_bounds__(VIS_THREADS) void k_visrhs(const DevMesh* __restric
     {
       const int x = b * VIS_RJ + a + 1;
       const VisCoef c0 = lds_coef(L.xc, x - 1), c1 = lds_coef(L.xc, x), c2 = lds_coef(L.xc, x + 1);
-      const Tri fm = vis_face(lds_prim(L, c - 1), c0, p1, c1);
-      const Tri fp = vis_face(p1, c1, lds_prim(L, c + 1), c2);
+      const Tri fm = vis_face(lds_uve(L, c - 1), c0, p1, c1);
+      const Tri fp = vis_face(p1, c1, lds_uve(L, c + 1), c2);
       const Tri gm = lds_tri(L.xg, x - 1), gc = lds_tri(L.xg, x);
       if (j < M.je) {
         const Tri gp = lds_tri(L.xg, x + 1);
@@ -345,7 +363,7 @@ __global__ __launch_bounds__(VIS_THREADS) void k_visrhs(const DevMesh* __restric
         } else {  // column j-2 lies left of the tile's ring
           const VisPrim pq = vis_prim(M, cell(M, j - 2, k), c2b, c2bp, prtr);
           const VisCoef cq = xi_coef(M, j - 2, k, pq, dre, gkpr);
-          gq = xi_cross(cq, div_prim(M, cell(M, j - 2, k + 1)), div_prim(M, cell(M, j - 2, k - 1)));
+          gq = vis_cross(cq, div_prim(M, cell(M, j - 2, k + 1)), div_prim(M, cell(M, j - 2, k - 1)), false);
         }
         s2 = s2 + (fp.f2 - fm.f2) + 0.5 * (gq.f2 - 4. * gm.f2 + 3 * gc.f2);
         s3 = s3 + (fp.f3 - fm.f3) + 0.5 * (gq.f3 - 4. * gm.f3 + 3 * gc.f3);
@@ -359,7 +377,8 @@ __global__ __launch_bounds__(VIS_THREADS) void k_visrhs(const DevMesh* __restric
   }
   if (norms) {
     const ResTile T{(int)blockIdx.y, j0, k0, (int)blockIdx.x};
-    norm_tile(M, T, j, k, valid, sv, &red[0][0]);
+    __syncthreads();   // the reduction takes the coefficients' memory
+    norm_tile(M, T, j, k, valid, sv, &L.red[0][0]);
   }
 }
 
