@@ -329,9 +329,31 @@ constexpr int RES_TJ = 32;
 constexpr int RES_TK = 8;
 constexpr int RES_THREADS = RES_TJ * RES_TK;
 
-// boundary-condition kernels run one workgroup per instance, its segments
-// one after another
-constexpr int BC_THREADS = 256;
+// The turbulence models' boundary conditions and those of the residual run
+// one workgroup per instance.  The segments of a phase touch disjoint cells:
+// f(segment, t, nt) runs for as many of them side by side as there are waves,
+// each on a group of whole waves (t, nt: the thread's number in its group and
+// the group's size); the phases follow one another with a barrier between.
+constexpr int BC_THREADS = 256, BC_ALL_THREADS = 1024;
+template <typename F>
+__device__ __forceinline__ void for_phases(const DevMesh& M, F f) {
+  const int nw = (int)(blockDim.x >> 6);
+  for (int ph = 0; ph < M.nbc_phase; ++ph) {
+    int m = 0;   // segments of this phase
+    for (int ib = 0; ib < M.nbc; ++ib) m += M.bc[ib].phase == ph;
+    for (int g0 = 0; g0 < m; g0 += nw) {
+      const int groups = m - g0 < nw ? m - g0 : nw, nt = 64 * (nw / groups);
+      const int mine = __builtin_amdgcn_readfirstlane((int)threadIdx.x / nt);
+      if (mine < groups) {
+        int q = g0 + mine, ib = 0;
+        for (;; ++ib)
+          if (M.bc[ib].phase == ph && q-- == 0) break;
+        f(M.bc[ib], (int)threadIdx.x - mine * nt, nt);
+      }
+    }
+    __syncthreads();
+  }
+}
 
 // oat of the time-accuracy order (src/time.f:22-25): the reference's istep
 // counts the time steps of the run

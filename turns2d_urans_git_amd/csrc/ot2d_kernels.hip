@@ -824,7 +824,7 @@ __global__ __launch_bounds__(NT) void k_residual(const DevMesh* __restrict__ Ms,
 // second stage, one block per instance: the tile partials in a fixed order
 // (strided per-thread sums, then an LDS tree), the norms, the history slot
 // and the "norm" status (src/step.f:104-110)
-__device__ void rbc_segment(const DevMesh& M, const DevBC& b);
+__device__ void rbc_segment(const DevMesh& M, const DevBC& b, int t, int nt);
 
 // with rbc = 1 the residual boundary conditions of the instance follow in
 // the same workgroup (rbc, src/step.f:133-136), unless the norm stopped it
@@ -882,10 +882,7 @@ __global__ __launch_bounds__(RES_THREADS) void k_norms_final(const DevMesh* __re
   if (!rbc) return;
   __syncthreads();
   if (stop_s) return;
-  for (int ib = 0; ib < M.nbc; ++ib) {
-    rbc_segment(M, M.bc[ib]);
-    __syncthreads();
-  }
+  for_phases(M, [&](const DevBC& b, int t, int nt) { rbc_segment(M, b, t, nt); });
 }
 
 // residual norms over the final residual when viscous / time-spectral terms
@@ -932,12 +929,11 @@ __global__ __launch_bounds__(256) void k_tsrhs(const DevMesh* __restrict__ Ms) {
 // rbc (src/bc.f:88-177): zero for wall/far-field types, wake copy
 // (rbcwake 1576-1633), extrapolation (2029-2094), symmetry (2160-2222),
 // periodic (270-357).
-__device__ void rbc_segment(const DevMesh& M, const DevBC& b) {
+__device__ void rbc_segment(const DevMesh& M, const DevBC& b, int t, int nt) {
   const gd_t qj = M.q[M.nq - 1];
   const gd_t ss[4] = {M.s[0], M.s[1], M.s[2], M.s[3]};
   int js = b.js, je = b.je, ks = b.ks, ke = b.ke, idir = b.idir;
   int iadd = idir >= 0 ? 1 : -1, iadir = idir >= 0 ? idir : -idir;
-  int t = threadIdx.x, nt = blockDim.x;
   int ty = b.type;
   int nj = je - js + 1, nk = ke - ks + 1;
   if (ty == 3 || ty == 4 || ty == 5 || ty == 46 || ty == 47) {
@@ -1006,10 +1002,7 @@ __device__ void rbc_segment(const DevMesh& M, const DevBC& b) {
 __global__ __launch_bounds__(BC_THREADS) void k_rbc(const DevMesh* __restrict__ Ms) {
   const DevMesh& M = Ms[blockIdx.x];
   if (*M.status) return;
-  for (int ib = 0; ib < M.nbc; ++ib) {
-    rbc_segment(M, M.bc[ib]);
-    __syncthreads();
-  }
+  for_phases(M, [&](const DevBC& b, int t, int nt) { rbc_segment(M, b, t, nt); });
 }
 
 // ==================================================================== LU-SGS

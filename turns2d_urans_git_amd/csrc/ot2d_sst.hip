@@ -2,9 +2,9 @@
 // itrans = 0).
 //
 //   k_sa_prim (shared with SA)   laminar viscosity, u, v (all cells)
-//   k_sst_bc                     komegabc (src/komegasst.f:906-1434), segments in
-//                                order, one block per instance; with eddy=1 the
-//                                eddy viscosity of the halo ring follows
+//   k_sst_bc                     komegabc (src/komegasst.f:906-1434), one workgroup
+//                                per instance; with eddy=1 the eddy viscosity of
+//                                the halo ring follows
 //   k_sst_blend                  kwvortic, turbstress, crossdiff, blend
 //                                (src/komegasst.f:270-461) per interior cell and
 //                                findturm (190-215) for every cell
@@ -52,18 +52,14 @@ __device__ __forceinline__ double findturm(double rho, double q5, double q6, dou
 }
 }  // namespace
 
-// komegabc for one instance, segments in the reference's order
-__global__ __launch_bounds__(BC_THREADS) void k_sst_bc(const DevMesh* __restrict__ Ms, int eddy) {
-  const DevMesh& M = Ms[blockIdx.x];
-  if (*M.status) return;
+// komegabc (src/komegasst.f:906-1434) for one segment
+__device__ void sst_bc_segment(const DevMesh& M, const DevBC& b, int t, int nt) {
   const gd_t q5 = M.q[4];
   const gd_t q6 = M.q[5];
   const gd_t u = M.sa_u;
   const gd_t v = M.sa_v;
   const double rei = 1. / M.c.rey;
-  const int t = threadIdx.x, nt = blockDim.x;
-  for (int ib = 0; ib < M.nbc; ++ib) {
-    const DevBC& b = M.bc[ib];
+  {
     int js = b.js, je = b.je, ks = b.ks, ke = b.ke, idir = b.idir;
     int iadd = idir >= 0 ? 1 : -1, iadir = idir >= 0 ? idir : -idir;
     int ty = b.type;
@@ -173,20 +169,27 @@ __global__ __launch_bounds__(BC_THREADS) void k_sst_bc(const DevMesh* __restrict
         }
       }
     }
-    __syncthreads();
   }
+}
+
+// komegabc of an instance by one workgroup, the segments of a phase side by
+// side (they touch disjoint cells), the phases in order
+__global__ __launch_bounds__(BC_ALL_THREADS) void k_sst_bc(const DevMesh* __restrict__ Ms, int eddy) {
+  const DevMesh& M = Ms[blockIdx.x];
+  if (*M.status) return;
+  for_phases(M, [&](const DevBC& b, int t, int nt) { sst_bc_segment(M, b, t, nt); });
   if (!eddy) return;
   // findturm on the halo ring (F2 = strain = 0 there)
   const int jd = M.jd, kd = M.kd;
   int nring = 2 * jd + 2 * (kd - 2);
-  for (int w = t; w < nring; w += nt) {
+  for (int w = threadIdx.x; w < nring; w += BC_ALL_THREADS) {
     int j, k;
     if (w < jd) { j = w + 1; k = 1; }
     else if (w < 2 * jd) { j = w - jd + 1; k = kd; }
     else if (w < 2 * jd + kd - 2) { j = 1; k = w - 2 * jd + 2; }
     else { j = jd; k = w - 2 * jd - (kd - 2) + 2; }
     long long i = cell(M, j, k);
-    M.turmu[i] = findturm(rho_of(M, i), q5[i], q6[i], M.kw_x[i]);
+    M.turmu[i] = findturm(rho_of(M, i), M.q[4][i], M.q[5][i], M.kw_x[i]);
   }
 }
 
@@ -482,7 +485,7 @@ hipError_t launch_sst(const DevMesh* dM, const DevMesh* hM, int nmi, Marks* mk, 
   hipError_t e;
   if ((e = launch_sa_prim(dM, hM, nmi, st)) != hipSuccess) return e;
   mark(mk, OT2D_ST_SA_PRIM, st);
-  hipLaunchKernelGGL(k_sst_bc, dim3(nmi), dim3(BC_THREADS), 0, st, dM, 0);
+  hipLaunchKernelGGL(k_sst_bc, dim3(nmi), dim3(BC_ALL_THREADS), 0, st, dM, 0);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_SA_BC, st);
   hipLaunchKernelGGL(k_sst_blend, dim3(nblk3(mx, 256), nmi), dim3(256), 0, st, dM);
@@ -504,7 +507,7 @@ hipError_t launch_sst(const DevMesh* dM, const DevMesh* hM, int nmi, Marks* mk, 
   }
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_SA_SOLVE_K, st);
-  hipLaunchKernelGGL(k_sst_bc, dim3(nmi), dim3(BC_THREADS), 0, st, dM, 1);
+  hipLaunchKernelGGL(k_sst_bc, dim3(nmi), dim3(BC_ALL_THREADS), 0, st, dM, 1);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_SA_EDDY, st);
   return hipSuccess;

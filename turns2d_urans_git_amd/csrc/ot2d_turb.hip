@@ -5,9 +5,8 @@
 //                                                    cross terms once into LDS, then each
 //                                                    cell's thin-layer fluxes from there
 //   vmu_sa (src/samodel2d.f:2-197)     k_sa_prim     laminar viscosity, u, v (all cells)
-//                                      k_turbc       SA boundary conditions (1 block / segment,
-//                                                    one launch per phase of the segments)
-//                                      k_turbc_eddy  the final SA boundary conditions and the
+//                                      k_turbc       SA boundary conditions (one workgroup per
+//                                                    instance); the final ones with the
 //                                                    eddy viscosity of the halo ring
 //                                      k_sa_rhs      convection, diffusion, source and the
 //                                                    two scalar tridiagonal systems, in
@@ -436,11 +435,10 @@ __device__ __forceinline__ void c_turm_cell(const DevMesh& M, long long i, int o
 }
 
 // turbc (src/samodel2d.f:827-1303) for one boundary segment
-__device__ void turbc_segment(const DevMesh& M, const DevBC& b) {
+__device__ void turbc_segment(const DevMesh& M, const DevBC& b, int t, int nt) {
   const gd_t q5 = M.q[4];
   const gd_t u = M.sa_u;
   const gd_t v = M.sa_v;
-  const int t = threadIdx.x, nt = blockDim.x;
   {
     int js = b.js, je = b.je, ks = b.ks, ke = b.ke, idir = b.idir;
     int iadd = idir >= 0 ? 1 : -1, iadir = idir >= 0 ? idir : -idir;
@@ -523,30 +521,17 @@ __device__ void turbc_segment(const DevMesh& M, const DevBC& b) {
   }
 }
 
-// the segments of one phase of every instance, one workgroup per segment
-// (segments of a phase touch disjoint cells; phases run in the reference's
-// segment order)
-__global__ __launch_bounds__(BC_THREADS) void k_turbc(const DevMesh* __restrict__ Ms, int phase) {
-  const DevMesh& M = Ms[blockIdx.y];
-  if (*M.status) return;
-  const int ib = blockIdx.x;
-  if (ib >= M.nbc || M.bc[ib].phase != phase) return;
-  turbc_segment(M, M.bc[ib]);
-}
-
-// the final turbc and the eddy viscosity of the halo ring after it
-// (c_turm), one workgroup per instance: every segment in order (one launch
-// here costs less than a launch per phase and one for the ring)
-__global__ __launch_bounds__(BC_THREADS) void k_turbc_eddy(const DevMesh* __restrict__ Ms, int ovl) {
+// turbc of an instance by one workgroup (the segments of a phase side by
+// side).  With eddy set (the final turbc) the eddy viscosity of the halo ring
+// follows (c_turm)
+__global__ __launch_bounds__(BC_ALL_THREADS) void k_turbc(const DevMesh* __restrict__ Ms, int eddy, int ovl) {
   const DevMesh& M = Ms[blockIdx.x];
   if (*M.status) return;
-  for (int ib = 0; ib < M.nbc; ++ib) {
-    turbc_segment(M, M.bc[ib]);
-    __syncthreads();
-  }
+  for_phases(M, [&](const DevBC& b, int t, int nt) { turbc_segment(M, b, t, nt); });
+  if (!eddy) return;
   const int jd = M.jd, kd = M.kd;
   const int nring = 2 * jd + 2 * (kd - 2);
-  for (int w = threadIdx.x; w < nring; w += blockDim.x) {
+  for (int w = threadIdx.x; w < nring; w += BC_ALL_THREADS) {
     int j, k;
     if (w < jd) { j = w + 1; k = 1; }
     else if (w < 2 * jd) { j = w - jd + 1; k = kd; }
@@ -894,21 +879,6 @@ hipError_t launch_sa_prim(const DevMesh* dM, const DevMesh* hM, int nmi, hipStre
 // (parts x 16 columns over 512 threads) always take 8.
 constexpr long long SAK_WIDE_COLS = 2048;
 
-// turbc over every instance: one launch per phase of the segments
-static hipError_t launch_turbc(const DevMesh* dM, const DevMesh* hM, int nmi, hipStream_t st) {
-  int nbc = 1, nph = 1;
-  for (int i = 0; i < nmi; ++i) {
-    nbc = hM[i].nbc > nbc ? hM[i].nbc : nbc;
-    nph = hM[i].nbc_phase > nph ? hM[i].nbc_phase : nph;
-  }
-  for (int ph = 0; ph < nph; ++ph) {
-    hipLaunchKernelGGL(k_turbc, dim3(nbc, nmi), dim3(BC_THREADS), 0, st, dM, ph);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-  }
-  return hipSuccess;
-}
-
 // vmu_sa for every instance (src/samodel2d.f:2-197, itrans = 0)
 hipError_t launch_sa(const DevMesh* dM, const DevMesh* hM, int nmi, Marks* mk, hipStream_t st, int sa_lane,
                      int prim_done, int ovl) {
@@ -924,7 +894,8 @@ hipError_t launch_sa(const DevMesh* dM, const DevMesh* hM, int nmi, Marks* mk, h
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
   mark(mk, OT2D_ST_SA_PRIM, st);
-  if ((e = launch_turbc(dM, hM, nmi, st)) != hipSuccess) return e;
+  hipLaunchKernelGGL(k_turbc, dim3(nmi), dim3(BC_ALL_THREADS), 0, st, dM, 0, ovl);
+  if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_SA_BC, st);
   hipLaunchKernelGGL(k_sa_rhs, dim3(vis_tiles(hM, nmi), nmi), dim3(VIS_THREADS), 0, st, dM);
   if ((e = hipGetLastError()) != hipSuccess) return e;
@@ -944,7 +915,7 @@ hipError_t launch_sa(const DevMesh* dM, const DevMesh* hM, int nmi, Marks* mk, h
   else solve_k(k_sa_solve_k<8>, 8);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_SA_SOLVE_K, st);
-  hipLaunchKernelGGL(k_turbc_eddy, dim3(nmi), dim3(BC_THREADS), 0, st, dM, ovl);
+  hipLaunchKernelGGL(k_turbc, dim3(nmi), dim3(BC_ALL_THREADS), 0, st, dM, 1, ovl);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_SA_EDDY, st);
   return hipSuccess;
