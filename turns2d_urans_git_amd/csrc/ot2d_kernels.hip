@@ -1401,18 +1401,22 @@ __device__ __forceinline__ void nb_matrix(const LUNb& n, double gm1, double m[16
 
 // Prep tiles.  A workgroup of LP_WAVES waves covers 8 rows of a block and
 // LP_WAVES*8 consecutive sweep steps; row r at step t is cell jr = t - r,
-// so its entries lie in a parallelogram of cells whose bounding box, with
-// the one-cell ring the neighbour terms reach, is LP_RJ x LP_RK cells.  The
-// per-cell quantities of ilu2d (src/lhs.f:524-564) are formed once per cell
-// of that box in LDS; each cell then assembles its operators from itself and
-// its four neighbours there.
+// so its entries lie in a parallelogram of cells.  The per-cell quantities of
+// ilu2d (src/lhs.f:524-564) are formed once per cell of it and of the one-cell
+// ring the neighbour terms reach in LDS, LP_C sweep steps of LP_K rows: cell
+// (row r, step t) at (r + 1) * LP_C + t + 1, its j neighbours one step, its k
+// neighbours a row and a step away.  Each cell then assembles its operators
+// from itself and its four neighbours there.
+// Bound by memory: 304 bytes written a cell, 112 read, the ring's again.  The
+// skewed ring is 340 cells for 256 where the bounding box of the parallelogram
+// was 410, and its 51 KiB (was 67) leave room for three workgroups a CU: 60
+// cases (3.9 M cells) 408 -> 360 us, 20 of them 136 -> 121, 513x129 11.1 -> 10.7.
 constexpr int LP_WAVES = 4, LP_STEPS = 8 * LP_WAVES;
-constexpr int LP_RJ = LP_STEPS + 7 + 2, LP_RK = 8 + 2, LP_N = LP_RJ * LP_RK;
+constexpr int LP_C = LP_STEPS + 2, LP_K = 8 + 2, LP_N = LP_C * LP_K;
 
 struct LUPrepLds {
-  double uu[LP_N], vv[LP_N], uv2[LP_N], ge[LP_N], qx[LP_N], qy[LP_N], cx[LP_N], cy[LP_N], vn[LP_N], d[LP_N],
-      qqx[LP_N], qqy[LP_N];
-  double xx[LP_N], xy[LP_N], yx[LP_N], yy[LP_N], ts[LP_N];
+  double uu[LP_N], vv[LP_N], ge[LP_N], qx[LP_N], qy[LP_N], cx[LP_N], cy[LP_N], vn[LP_N], qqx[LP_N], qqy[LP_N];
+  double xx[LP_N], xy[LP_N], yx[LP_N], yy[LP_N], f[LP_N];   // f = sv * d
   double sh[4][LP_N];   // s * tscale * d (src/step.f:141-148, src/lhs.f:568-598)
 };
 constexpr size_t LP_LDS = sizeof(LUPrepLds);
@@ -1425,7 +1429,7 @@ __device__ __forceinline__ void lu32_term(const LUPrepLds& S, int n, bool halo, 
   CellLoad cn;
   cn.xx = S.xx[n]; cn.xy = S.xy[n]; cn.yx = S.yx[n]; cn.yy = S.yy[n];
   LUCellF64 Ln;
-  Ln.uu = S.uu[n]; Ln.vv = S.vv[n]; Ln.uv2 = S.uv2[n]; Ln.ge = S.ge[n]; Ln.qx = S.qx[n]; Ln.qy = S.qy[n];
+  Ln.uu = S.uu[n]; Ln.vv = S.vv[n]; Ln.uv2 = 0.5 * (Ln.uu * Ln.uu + Ln.vv * Ln.vv); Ln.ge = S.ge[n]; Ln.qx = S.qx[n]; Ln.qy = S.qy[n];
   Ln.cx = S.cx[n]; Ln.cy = S.cy[n]; Ln.vn = S.vn[n]; Ln.qqx_s = S.qqx[n]; Ln.qqy_s = S.qqy[n];
   LUNb nb;
   if (jdir) nb_j(cn, Ln, eps2, dir, nb);
@@ -1464,21 +1468,19 @@ __global__ __launch_bounds__(64 * LP_WAVES) void k_lu_prep32(const DevMesh* __re
   const int tb = (int)blockIdx.x % tiles_t, rest = (int)blockIdx.x / tiles_t;
   const int lb = rest % RG, w = rest / RG;
   const int T0 = tb * LP_STEPS, L0 = lb * 8;
-  // box origin: cell (jr, kk) = (T0 - L0 - 8, LU32_R*w + L0 - 1) is LDS cell 0
-  const int jr0 = T0 - L0 - 8, kk0 = LU32_R * w + L0 - 1;
   extern __shared__ __attribute__((aligned(16))) double lp_raw[];
   LUPrepLds& S = *reinterpret_cast<LUPrepLds*>(lp_raw);
   for (int n = threadIdx.x; n < LP_N; n += nthr) {
-    const int jr = jr0 + n % LP_RJ, kk = kk0 + n / LP_RJ;
+    const int rr = n / LP_C - 1, jr = T0 + n % LP_C - 1 - (L0 + rr), kk = LU32_R * w + L0 + rr;
     if (jr < -1 || jr > g.ni || kk < -1 || kk > g.nk) continue;
     const long long i = cell(M, js + jr, ks + kk);
     const CellLoad c = load_cell(M, i);
     double sv[4];
     for (int q = 0; q < 4; ++q) sv[q] = M.s[q][i];
     const LUCellF64 L = lu_of(M.c, c, epsv);
-    S.uu[n] = L.uu; S.vv[n] = L.vv; S.uv2[n] = L.uv2; S.ge[n] = L.ge; S.qx[n] = L.qx; S.qy[n] = L.qy;
-    S.cx[n] = L.cx; S.cy[n] = L.cy; S.vn[n] = L.vn; S.d[n] = L.d; S.qqx[n] = L.qqx_s; S.qqy[n] = L.qqy_s;
-    S.xx[n] = c.xx; S.xy[n] = c.xy; S.yx[n] = c.yx; S.yy[n] = c.yy; S.ts[n] = c.ts;
+    S.uu[n] = L.uu; S.vv[n] = L.vv; S.ge[n] = L.ge; S.qx[n] = L.qx; S.qy[n] = L.qy;
+    S.cx[n] = L.cx; S.cy[n] = L.cy; S.vn[n] = L.vn; S.qqx[n] = L.qqx_s; S.qqy[n] = L.qqy_s;
+    S.xx[n] = c.xx; S.xy[n] = c.xy; S.yx[n] = c.yx; S.yy[n] = c.yy; S.f[n] = (c.ts * 0.5) * L.d;
     for (int q = 0; q < 4; ++q) S.sh[q][n] = sv[q] * c.ts * L.d;
   }
   __syncthreads();
@@ -1493,15 +1495,15 @@ __global__ __launch_bounds__(64 * LP_WAVES) void k_lu_prep32(const DevMesh* __re
   const int kk = LU32_R * w + r, jr = t - r;
   if (t >= g.TA || kk >= g.nk || jr < 0 || jr >= g.ni) return;
   const int j = js + jr, k = ks + kk;
-  const int n0 = (kk - kk0) * LP_RJ + (jr - jr0);
-  const double di = S.d[n0], f = (S.ts[n0] * 0.5) * di;
+  const int n0 = (r - L0 + 1) * LP_C + (t - T0) + 1;
+  const double f = S.f[n0];
   const double gm1 = M.c.gm1;
   double u[4], cb[4] = {0.0, 0.0, 0.0, 0.0}, PA[16], PB[16], QA[16], QB[16];
   for (int q = 0; q < 4; ++q) u[q] = S.sh[q][n0];
   lu32_term(S, n0 - 1, j == js, 1, +1, f, eps2, gm1, PA, u);
-  lu32_term(S, n0 - LP_RJ, k == ks, 0, +1, f, eps2, gm1, PB, u);
+  lu32_term(S, n0 - LP_C - 1, k == ks, 0, +1, f, eps2, gm1, PB, u);
   lu32_term(S, n0 + 1, j == je, 1, -1, -f, eps2, gm1, QA, cb);
-  lu32_term(S, n0 + LP_RJ, k == ke, 0, -1, -f, eps2, gm1, QB, cb);
+  lu32_term(S, n0 + LP_C + 1, k == ke, 0, -1, -f, eps2, gm1, QB, cb);
   const long long rec = (long long)w * g.TA + t;
   gf32x4* rf = lu + g.off_f32 + rec * 288;
   gf32x4* rb = lu + g.off_b32 + rec * 256;
