@@ -724,7 +724,7 @@ __device__ __forceinline__ void face_states_weno(const double* sf0, int stv, int
 // (800 operations a face).
 template <int H, int NT>
 __global__ __launch_bounds__(NT) void k_residual(const DevMesh* __restrict__ Ms, const ResTile* __restrict__ tiles,
-                                                 int do_norms) {
+                                                 int ntiles, int do_norms) {
   constexpr int TJ = RES_TJ, TK = RES_TK, LJ = TJ + 2 * H, LK = TK + 2 * H;
   constexpr int NXI = TK * (TJ + 1), NETA = (TK + 1) * TJ;
   __shared__ double sf[4][LK * LJ];   // primitives rho, u, v, p; then the norms' reduction
@@ -732,7 +732,9 @@ __global__ __launch_bounds__(NT) void k_residual(const DevMesh* __restrict__ Ms,
   __shared__ double sxv[(TK + 1) * (TJ + 1)], syv[(TK + 1) * (TJ + 1)];
   __shared__ double sF[4][NXI + NETA];  // fluxes: xi faces [TK][TJ+1], then eta faces [TK+1][TJ]
   static_assert(4 * LK * LJ >= 4 * RES_THREADS, "the reduction fits the primitives' array");
-  const ResTile T = tiles[blockIdx.x];
+  const int tile = xcd_tile(ntiles);
+  if (tile < 0) return;
+  const ResTile T = tiles[tile];
   const DevMesh& M = Ms[T.mesh];
   const DevConst& C = M.c;
   const int tid = threadIdx.x;
@@ -1410,7 +1412,7 @@ __device__ __forceinline__ void nb_matrix(const LUNb& n, double gm1, double m[16
 // Bound by memory: 304 bytes written a cell, 112 read, the ring's again.  The
 // skewed ring is 340 cells for 256 where the bounding box of the parallelogram
 // was 410, and its 51 KiB (was 67) leave room for three workgroups a CU: 60
-// cases (3.9 M cells) 408 -> 360 us, 20 of them 136 -> 121, 513x129 11.1 -> 10.7.
+// cases (3.9 M cells) 408 -> 360 us, 20 of them 136 -> 121, 513x129 11.1 -> 10.3 (with xcd_tile).
 constexpr int LP_WAVES = 4, LP_STEPS = 8 * LP_WAVES;
 constexpr int LP_C = LP_STEPS + 2, LP_K = 8 + 2, LP_N = LP_C * LP_K;
 
@@ -1464,8 +1466,9 @@ __global__ __launch_bounds__(64 * LP_WAVES) void k_lu_prep32(const DevMesh* __re
   const int nthr = 64 * LP_WAVES;
   // tile of this workgroup: block w, rows 8*lb .. 8*lb+7, steps T0 .. T0+LP_STEPS-1
   const int tiles_t = (g.TA + LP_STEPS - 1) / LP_STEPS;
-  if ((int)blockIdx.x >= g.W * RG * tiles_t) return;
-  const int tb = (int)blockIdx.x % tiles_t, rest = (int)blockIdx.x / tiles_t;
+  const int tile = xcd_tile(g.W * RG * tiles_t);
+  if (tile < 0) return;
+  const int tb = tile % tiles_t, rest = tile / tiles_t;
   const int lb = rest % RG, w = rest / RG;
   const int T0 = tb * LP_STEPS, L0 = lb * 8;
   extern __shared__ __attribute__((aligned(16))) double lp_raw[];
@@ -2841,7 +2844,7 @@ constexpr int RES_WIDE_TILES = 2048;
 hipError_t launch_residual(const DevMesh* dM, const ResTile* tiles, int ntiles, int do_norms, int weno,
                            hipStream_t st) {
   auto launch = [&](auto kern, int nt) {
-    hipLaunchKernelGGL(kern, dim3(ntiles), dim3(nt), 0, st, dM, tiles, do_norms);
+    hipLaunchKernelGGL(kern, dim3(xcd_grid(ntiles)), dim3(nt), 0, st, dM, tiles, ntiles, do_norms);
   };
   if (ntiles <= RES_WIDE_TILES) {
     if (weno) launch(k_residual<3, 576>, 576);
@@ -2988,7 +2991,7 @@ static hipError_t launch_lu32(const DevMesh* dM, const DevMesh* hM, int nmi, int
     (void)hipFuncSetAttribute((const void*)k_lu_prep32, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LP_LDS);
     attr_set = true;
   }
-  hipLaunchKernelGGL(k_lu_prep32, dim3((unsigned)nc, nmi), dim3(64 * LP_WAVES), LP_LDS, st, dM);
+  hipLaunchKernelGGL(k_lu_prep32, dim3(xcd_grid(nc), nmi), dim3(64 * LP_WAVES), LP_LDS, st, dM);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   mark(mk, OT2D_ST_LU_PREP, st);

@@ -247,13 +247,14 @@ __global__ __launch_bounds__(VIS_THREADS, 3) void k_visrhs(const DevMesh* __rest
   const DevMesh& M = Ms[blockIdx.y];
   const int nj = M.je - M.js + 1, nk = M.ke - M.ks + 1;
   const int tiles_j = (nj + VIS_TJ - 1) / VIS_TJ;
-  if ((int)blockIdx.x >= tiles_j * ((nk + VIS_TK - 1) / VIS_TK) || *M.status) return;
+  const int tile = xcd_tile(tiles_j * ((nk + VIS_TK - 1) / VIS_TK));
+  if (tile < 0 || *M.status) return;
   extern __shared__ __attribute__((aligned(16))) double vis_raw[];
   VisLds& L = *reinterpret_cast<VisLds*>(vis_raw);
   const DevConst& C = M.c;
   const double gkpr = C.gamma / C.pr, prtr = C.pr / 0.9, dre = .5 / C.rey;
   const double c2b = 198.6 / C.tinf, c2bp = c2b + 1.;
-  const int j0 = M.js + ((int)blockIdx.x % tiles_j) * VIS_TJ, k0 = M.ks + ((int)blockIdx.x / tiles_j) * VIS_TK;
+  const int j0 = M.js + (tile % tiles_j) * VIS_TJ, k0 = M.ks + (tile / tiles_j) * VIS_TK;
   const int t = threadIdx.x;
   const gd_t qj = M.q[M.nq - 1];
 
@@ -375,7 +376,7 @@ __global__ __launch_bounds__(VIS_THREADS, 3) void k_visrhs(const DevMesh* __rest
     sv[0] = M.s[0][i]; sv[1] = s2; sv[2] = s3; sv[3] = s4;
   }
   if (norms) {
-    const ResTile T{(int)blockIdx.y, j0, k0, (int)blockIdx.x};
+    const ResTile T{(int)blockIdx.y, j0, k0, tile};
     __syncthreads();   // the reduction takes the coefficients' memory
     norm_tile(M, T, j, k, valid, sv, &L.red[0][0]);
   }
@@ -575,10 +576,11 @@ __global__ __launch_bounds__(VIS_THREADS, 4) void k_sa_rhs(const DevMesh* __rest
   const int js = M.js, je = M.je, ks = M.ks, ke = M.ke;
   const int nj = je - js + 1, nk = ke - ks + 1;
   const int tiles_j = (nj + VIS_TJ - 1) / VIS_TJ;
-  if ((int)blockIdx.x >= tiles_j * ((nk + VIS_TK - 1) / VIS_TK) || *M.status) return;
+  const int tile = xcd_tile(tiles_j * ((nk + VIS_TK - 1) / VIS_TK));
+  if (tile < 0 || *M.status) return;
   const DevConst& C = M.c;
   const double rey = C.rey;
-  const int j0 = js + ((int)blockIdx.x % tiles_j) * VIS_TJ, k0 = ks + ((int)blockIdx.x / tiles_j) * VIS_TK;
+  const int j0 = js + (tile % tiles_j) * VIS_TJ, k0 = ks + (tile / tiles_j) * VIS_TK;
   const int t = threadIdx.x;
   for (int n = t; n < SAR_N; n += VIS_THREADS) {
     const int j = j0 - 1 + n % VIS_RJ, k = k0 - 1 + n / VIS_RJ;
@@ -859,7 +861,7 @@ hipError_t launch_visrhs(const DevMesh* dM, const DevMesh* hM, int nmi, hipStrea
     if (e != hipSuccess) return e;
     lds_set = true;
   }
-  hipLaunchKernelGGL(k_visrhs, dim3(tiles, nmi), dim3(VIS_THREADS), VIS_LDS, st, dM, norms);
+  hipLaunchKernelGGL(k_visrhs, dim3(xcd_grid(tiles), nmi), dim3(VIS_THREADS), VIS_LDS, st, dM, norms);
   return hipGetLastError();
 }
 
@@ -897,7 +899,7 @@ hipError_t launch_sa(const DevMesh* dM, const DevMesh* hM, int nmi, Marks* mk, h
   hipLaunchKernelGGL(k_turbc, dim3(nmi), dim3(BC_ALL_THREADS), 0, st, dM, 0, ovl);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_SA_BC, st);
-  hipLaunchKernelGGL(k_sa_rhs, dim3(vis_tiles(hM, nmi), nmi), dim3(VIS_THREADS), 0, st, dM);
+  hipLaunchKernelGGL(k_sa_rhs, dim3(xcd_grid(vis_tiles(hM, nmi)), nmi), dim3(VIS_THREADS), 0, st, dM);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_SA_RHS, st);
   hipLaunchKernelGGL(k_sa_solve_j, dim3(mk_, nmi), dim3(64), 0, st, dM);
