@@ -1175,7 +1175,7 @@ static int32_t enqueue_time_step(ot2d_case* c, Marks* mk, int part = 0) {
       // grid and metrics
       const int nmv = (c->ncase == 1 && c->nmesh > 1) ? c->nspec : v.n;
       HIPCHK(launch_pitch(v.dM, v.hM, nmv, c->stream));
-      HIPCHK(launch_init_geometry(v.dM, nmv, c->stream, 1));
+      HIPCHK(launch_metrics(v.dM, v.hM, nmv, c->stream));
       if (!c->lamin) HIPCHK(launch_sa_dist(v.dM, v.hM, nmv, c->stream));
     }
   }

@@ -470,7 +470,8 @@ inline void mark(Marks* m, int s, hipStream_t st) {
 
 // metrics_only: metfv alone on moved vertices (no cell centres, no
 // free-stream state), as the time loop of a moving grid does
-hipError_t launch_init_geometry(const DevMesh* dM, int nmi, hipStream_t st, int metrics_only = 0);
+hipError_t launch_init_geometry(const DevMesh* dM, int nmi, hipStream_t st);
+hipError_t launch_metrics(const DevMesh* dM, const DevMesh* hM, int nmi, hipStream_t st);
 // pitch (src/motion.f:546-632): the grid turns by this time step's angle
 hipError_t launch_pitch(const DevMesh* dM, const DevMesh* hM, int nmi, hipStream_t st);
 // with ncase > 0 also opens the step of every running case (istep0 and the

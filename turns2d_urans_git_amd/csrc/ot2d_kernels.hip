@@ -2418,7 +2418,38 @@ __global__ __launch_bounds__(256) void k_monitor(const DevMesh* __restrict__ Ms)
 // find_cellcenter (setup.f:111-345), metfv (setup.f:440-724),
 // find_timemetrics_TS (setup.f:727-786), qzero (init.f:209-277), qdivj
 // (init.f:180-206).  One block per instance, phases separated by barriers.
-__global__ __launch_bounds__(256) void k_init_geometry(const DevMesh* __restrict__ Ms, int metrics_only) {
+// metfv of one interior cell (src/setup.f:485-531): qj and the metrics from its four
+// vertices
+__device__ __forceinline__ void metric_cell(const DevMesh& M, int j, int k) {
+  auto xv = [&](int a, int b) { return M.xv[vert(M, a, b)]; };
+  auto yv = [&](int a, int b) { return M.yv[vert(M, a, b)]; };
+  long long i = cell(M, j, k);  // jc = j, kc = k with one halo
+  double dx1 = xv(j, k) - xv(j - 1, k - 1);
+  double dy1 = yv(j, k) - yv(j - 1, k - 1);
+  double dx2 = xv(j - 1, k) - xv(j, k - 1);
+  double dy2 = yv(j - 1, k) - yv(j, k - 1);
+  double a3 = 0.5 * (dx1 * dy2 - dx2 * dy1);
+  double J = 1. / a3;
+  double xx = 0.5 * (yv(j, k) - yv(j, k - 1) + yv(j - 1, k) - yv(j - 1, k - 1));
+  double xy = -0.5 * (xv(j, k) - xv(j, k - 1) + xv(j - 1, k) - xv(j - 1, k - 1));
+  double yx = -0.5 * (yv(j, k) - yv(j - 1, k) + yv(j, k - 1) - yv(j - 1, k - 1));
+  double yy = 0.5 * (xv(j, k) - xv(j - 1, k) + xv(j, k - 1) - xv(j - 1, k - 1));
+  M.q[M.nq - 1][i] = J;
+  M.xx[i] = J * xx; M.xy[i] = J * xy; M.yx[i] = J * yx; M.yy[i] = J * yy;
+}
+
+// metfv's interior of a grid that has turned, one thread per cell; its halo
+// follows by k_init_geometry.  193x65: 4.8 us and 11 for the halo; one
+// workgroup for both took 47.
+__global__ __launch_bounds__(256) void k_metrics(const DevMesh* __restrict__ Ms) {
+  const DevMesh& M = Ms[blockIdx.y];
+  const int nj = M.jmax - 1;
+  const long long n = (long long)nj * (M.kmax - 1);
+  for (long long w = blockIdx.x * 256ll + threadIdx.x; w < n; w += 256ll * gridDim.x)
+    metric_cell(M, 2 + (int)(w % nj), 2 + (int)(w / nj));
+}
+
+__global__ __launch_bounds__(256) void k_init_geometry(const DevMesh* __restrict__ Ms, int halo_only) {
   const DevMesh& M = Ms[blockIdx.x];
   const DevConst& C = M.c;
   const int t = threadIdx.x, nt = blockDim.x;
@@ -2429,7 +2460,8 @@ __global__ __launch_bounds__(256) void k_init_geometry(const DevMesh* __restrict
   const gd_t xv = M.xv;
   const gd_t yv = M.yv;
   const double pi = 4.0 * atan(1.0);
-  if (metrics_only) goto metrics;
+  const gd_t qj = M.q[M.nq - 1];
+  if (halo_only) goto halo;
   // find_coord_TS for instances 2..nspec (src/setup.f:348-393)
   if (M.nsp > 0 && C.timespectral) {
     double tspec = *M.tspec;
@@ -2525,25 +2557,12 @@ __global__ __launch_bounds__(256) void k_init_geometry(const DevMesh* __restrict
     __syncthreads();
   }
   // ---- metfv
-metrics:
-  const gd_t qj = M.q[M.nq - 1];
   for (long long w = t; w < (long long)(jmax - 1) * (kmax - 1); w += nt) {
     int j = 2 + (int)(w % (jmax - 1)), k = 2 + (int)(w / (jmax - 1));
-    long long i = cell(M, j, k);  // jc = j, kc = k with one halo
-    double dx1 = XV(j, k) - XV(j - 1, k - 1);
-    double dy1 = YV(j, k) - YV(j - 1, k - 1);
-    double dx2 = XV(j - 1, k) - XV(j, k - 1);
-    double dy2 = YV(j - 1, k) - YV(j, k - 1);
-    double a3 = 0.5 * (dx1 * dy2 - dx2 * dy1);
-    double J = 1. / a3;
-    qj[i] = J;
-    double xx = 0.5 * (YV(j, k) - YV(j, k - 1) + YV(j - 1, k) - YV(j - 1, k - 1));
-    double xy = -0.5 * (XV(j, k) - XV(j, k - 1) + XV(j - 1, k) - XV(j - 1, k - 1));
-    double yx = -0.5 * (YV(j, k) - YV(j - 1, k) + YV(j, k - 1) - YV(j - 1, k - 1));
-    double yy = 0.5 * (XV(j, k) - XV(j - 1, k) + XV(j, k - 1) - XV(j - 1, k - 1));
-    M.xx[i] = J * xx; M.xy[i] = J * xy; M.yx[i] = J * yx; M.yy[i] = J * yy;
+    metric_cell(M, j, k);
   }
   __syncthreads();
+halo:
 #define CPY(dst, src) { qj[dst] = qj[src]; M.xx[dst] = M.xx[src]; M.xy[dst] = M.xy[src]; \
     M.yx[dst] = M.yx[src]; M.yy[dst] = M.yy[src]; }
   for (int k = M.ks + t; k <= M.ke; k += nt) {
@@ -2585,7 +2604,7 @@ metrics:
     __syncthreads();
   }
 #undef CPY
-  if (metrics_only) return;
+  if (halo_only) return;
   // ---- find_timemetrics_TS (src/setup.f:727-786)
   if (C.timespectral) {
     double tspec = *M.tspec, rotf = C.rotf, am = C.angmax;
@@ -2778,8 +2797,18 @@ static inline int nblk(long long n, int per) {
   return (int)(b < 1 ? 1 : (b > 4096 ? 4096 : b));
 }
 
-hipError_t launch_init_geometry(const DevMesh* dM, int nmi, hipStream_t st, int metrics_only) {
-  hipLaunchKernelGGL(k_init_geometry, dim3(nmi), dim3(256), 0, st, dM, metrics_only);
+hipError_t launch_init_geometry(const DevMesh* dM, int nmi, hipStream_t st) {
+  hipLaunchKernelGGL(k_init_geometry, dim3(nmi), dim3(256), 0, st, dM, 0);
+  return hipGetLastError();
+}
+
+hipError_t launch_metrics(const DevMesh* dM, const DevMesh* hM, int nmi, hipStream_t st) {
+  long long mx = 0;
+  for (int i = 0; i < nmi; ++i) mx = hM[i].jmax * (long long)hM[i].kmax > mx ? hM[i].jmax * (long long)hM[i].kmax : mx;
+  hipLaunchKernelGGL(k_metrics, dim3(nblk(mx, 256), nmi), dim3(256), 0, st, dM);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(k_init_geometry, dim3(nmi), dim3(256), 0, st, dM, 1);
   return hipGetLastError();
 }
 
