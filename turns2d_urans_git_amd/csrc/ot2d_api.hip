@@ -1145,10 +1145,10 @@ static int32_t enqueue_turbulent_implicit(ot2d_case* c, const StepView& v, Marks
     HIPCHK(launch_update_monitor(v.dM, v.hM, v.n, c->stream, 1));
     return OT2D_OK;
   }
-  // SA: the laminar viscosity and velocities come out of k_lu_finish
-  const int sa = c->iturb == 1 ? 2 : 0;
-  HIPCHK(launch_lu(v.dM, v.hM, v.n, sa, c->p.lu_fp32, mk, c->stream, c->cfg.sweep));
-  if (c->iturb == 2) HIPCHK(launch_sst(v.dM, v.hM, v.n, mk, c->stream));
+  // the laminar viscosity and velocities come out of k_lu_finish (a pass of
+  // their own takes 5 us, they add 0.3 there)
+  HIPCHK(launch_lu(v.dM, v.hM, v.n, 2, c->p.lu_fp32, mk, c->stream, c->cfg.sweep));
+  if (c->iturb == 2) HIPCHK(launch_sst(v.dM, v.hM, v.n, mk, c->stream, 1));
   else HIPCHK(launch_sa(v.dM, v.hM, v.n, mk, c->stream, c->cfg.sa_lane, 1));
   // the q update and monitor in one pass (stage "update", marked by the caller)
   HIPCHK(launch_update_monitor(v.dM, v.hM, v.n, c->stream));

@@ -474,7 +474,7 @@ static inline int nblk3(long long n, int per) {
 constexpr int SSTK_NP8 = 32;
 
 // komegasst for every instance (src/komegasst.f:2-187)
-hipError_t launch_sst(const DevMesh* dM, const DevMesh* hM, int nmi, Marks* mk, hipStream_t st) {
+hipError_t launch_sst(const DevMesh* dM, const DevMesh* hM, int nmi, Marks* mk, hipStream_t st, int prim_done) {
   long long mx = 0;
   int mj = 1, mk_ = 1;
   for (int i = 0; i < nmi; ++i) {
@@ -483,7 +483,7 @@ hipError_t launch_sst(const DevMesh* dM, const DevMesh* hM, int nmi, Marks* mk, 
     mk_ = hM[i].ke - hM[i].ks + 1 > mk_ ? hM[i].ke - hM[i].ks + 1 : mk_;
   }
   hipError_t e;
-  if ((e = launch_sa_prim(dM, hM, nmi, st)) != hipSuccess) return e;
+  if (!prim_done && (e = launch_sa_prim(dM, hM, nmi, st)) != hipSuccess) return e;
   mark(mk, OT2D_ST_SA_PRIM, st);
   hipLaunchKernelGGL(k_sst_bc, dim3(nmi), dim3(BC_ALL_THREADS), 0, st, dM, 0);
   if ((e = hipGetLastError()) != hipSuccess) return e;
