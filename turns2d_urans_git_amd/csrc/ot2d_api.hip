@@ -88,7 +88,10 @@ struct ot2d_case {
   int* d_istep0 = nullptr;
   int* d_stepc = nullptr;
   int* d_istep = nullptr;      // time steps of this run per case (time-accurate steps)
-  int* h_small = nullptr;      // pinned host copy of d_stepc and d_status (2 * ncase ints)
+  // what a call clears and reads back, in one allocation with a pinned copy of
+  // it: d_norms, d_status, d_stepc
+  double* d_call = nullptr;
+  double* h_call = nullptr;
   double* h_hist = nullptr;    // pinned host copy of d_hist (hist_cap steps)
   int tacc = 0;                // time-accurate steps: stored levels, Newton sub-iterations, motion
   int moving = 0;              // the grid pitches every time step (iunst = 1)
@@ -384,11 +387,11 @@ static void free_case(ot2d_case* c) {
     dfree(mb.xold); dfree(mb.yold); dfree(mb.xole); dfree(mb.yole); dfree(mb.turmu_n);
   }
   dfree(c->dMa); dfree(c->dTa); dfree(c->d_istep); dfree(c->d_itnorms);
-  dfree(c->dM); dfree(c->dT); dfree(c->d_status); dfree(c->d_istep0); dfree(c->d_stepc);
-  if (c->h_small) (void)hipHostFree(c->h_small);
+  dfree(c->dM); dfree(c->dT); dfree(c->d_call); dfree(c->d_istep0);
+  if (c->h_call) (void)hipHostFree(c->h_call);
   if (c->h_hist) (void)hipHostFree(c->h_hist);
   dfree(c->d_cinst); dfree(c->d_ctol);
-  dfree(c->d_partials); dfree(c->d_norms); dfree(c->d_tspec);
+  dfree(c->d_partials); dfree(c->d_tspec);
   dfree(c->d_Ds); dfree(c->d_hist); dfree(c->d_forces);
   if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
   if (c->ev_join) (void)hipEventDestroy(c->ev_join);
@@ -646,15 +649,19 @@ static int32_t create_impl(const ot2d_params* ps, int32_t ncase, int32_t nmesh, 
   c->itnmax = p->itnmax;
   c->moving = !p->timespectral && p->iunst == 1;
   c->tacc = p->itnmax > 1 || p->ntac > 1 || c->moving;
-  A(c->d_status, ncase); A(c->d_istep0, ncase); A(c->d_stepc, ncase); A(c->d_istep, ncase);
-  if ((e = hipHostMalloc((void**)&c->h_small, sizeof(int) * 2 * (size_t)ncase, hipHostMallocDefault)) != hipSuccess) {
-    c->h_small = nullptr;
+  const size_t ncall = 6 * (size_t)nmi + (size_t)ncase;   // doubles: the norms, then two ints a case
+  A(c->d_call, ncall); A(c->d_istep0, ncase); A(c->d_istep, ncase);
+  c->d_norms = c->d_call;
+  c->d_status = reinterpret_cast<int*>(c->d_call + 6 * (size_t)nmi);
+  c->d_stepc = c->d_status + ncase;
+  if ((e = hipHostMalloc((void**)&c->h_call, sizeof(double) * ncall, hipHostMallocDefault)) != hipSuccess) {
+    c->h_call = nullptr;
     free_case(c);
     return fail(OT2D_ERR_NOMEM, "pinned host allocation failed: %s", hipGetErrorString(e));
   }
   if (c->tacc) A(c->d_itnorms, 6 * (size_t)nmi * c->itnmax);
   A(c->d_cinst, 2 * (size_t)ncase); A(c->d_ctol, ncase);
-  A(c->d_norms, 6 * nmi); A(c->d_tspec, (size_t)ns * ncase); A(c->d_Ds, ns * ns);
+  A(c->d_tspec, (size_t)ns * ncase); A(c->d_Ds, ns * ns);
   A(c->d_forces, 16);
   // spectral coefficients, src/setup.f:838-873
   {
@@ -1009,6 +1016,14 @@ static int32_t clear_status(ot2d_case* c) {
   return OT2D_OK;
 }
 
+// what a call of steps clears: the step counters and, of a single case, the
+// status (adjacent: one memset)
+static int32_t open_call(ot2d_case* c) {
+  int* from = c->batch ? c->d_stepc : c->d_status;
+  HIPCHK(hipMemsetAsync(from, 0, sizeof(int) * (size_t)(c->batch ? c->ncase : 2 * c->ncase), c->stream));
+  return OT2D_OK;
+}
+
 extern "C" int32_t ot2d_time_step(ot2d_case* c) {
   if (!c) return fail(OT2D_ERR_ARG, "null case");
   if (int32_t rc = clear_status(c)) return rc;
@@ -1233,38 +1248,23 @@ extern "C" int32_t ot2d_turbulence(ot2d_case* c) {
   return sync(c);
 }
 
-// status of a single case; for a batch, 3 if any case's sweep pipeline
-// stopped, else 0 (per-case states through ot2d_batch_status)
-static int32_t read_status(ot2d_case* c, int* st) {
-  std::vector<int> all(c->ncase);
-  HIPCHK(hipMemcpyAsync(all.data(), c->d_status, sizeof(int) * c->ncase, hipMemcpyDeviceToHost, c->stream));
+// what the device holds of a call (with its norms where they are asked for),
+// into the pinned copy by one copy and one synchronisation.  steps: done by
+// the furthest case; st: the status of a single case, for a batch 3 if any
+// case's sweep pipeline stopped, else 0 (per-case states through
+// ot2d_batch_status)
+static int32_t close_call(ot2d_case* c, bool norms, int* steps, int* st) {
+  const size_t n6 = 6 * (size_t)nmi(c), from = norms ? 0 : n6;
+  HIPCHK(hipMemcpyAsync(c->h_call + from, c->d_call + from, sizeof(double) * (n6 + (size_t)c->ncase - from),
+                        hipMemcpyDeviceToHost, c->stream));
   if (int32_t rc = sync(c)) return rc;
-  if (!c->batch) {
-    *st = all[0];
-  } else {
-    *st = 0;
-    for (int v : all)
-      if (v == 3) *st = 3;
-  }
-  return OT2D_OK;
-}
-
-// steps done by the furthest case in the current call and the status as
-// read_status gives it, with one synchronisation (both copies into the
-// case's pinned buffer)
-static int32_t read_steps_status(ot2d_case* c, int* steps, int* st) {
-  const size_t nb = sizeof(int) * (size_t)c->ncase;
-  HIPCHK(hipMemcpyAsync(c->h_small, c->d_stepc, nb, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipMemcpyAsync(c->h_small + c->ncase, c->d_status, nb, hipMemcpyDeviceToHost, c->stream));
-  if (int32_t rc = sync(c)) return rc;
+  const int* status = reinterpret_cast<const int*>(c->h_call + n6);
+  const int* stepc = status + c->ncase;
   *steps = 0;
-  for (int i = 0; i < c->ncase; ++i) *steps = c->h_small[i] > *steps ? c->h_small[i] : *steps;
-  if (!c->batch) {
-    *st = c->h_small[c->ncase];
-  } else {
-    *st = 0;
-    for (int i = 0; i < c->ncase; ++i)
-      if (c->h_small[c->ncase + i] == 3) *st = 3;
+  *st = c->batch ? 0 : status[0];
+  for (int i = 0; i < c->ncase; ++i) {
+    *steps = stepc[i] > *steps ? stepc[i] : *steps;
+    if (c->batch && status[i] == 3) *st = 3;
   }
   return OT2D_OK;
 }
@@ -1306,17 +1306,15 @@ extern "C" int32_t ot2d_step(ot2d_case* c, double* norms, int32_t* argmax) {
   {
     Fp32Order order(c);
     HIPCHK(order.error());
-    if (int32_t rc = clear_status(c)) return rc;
-    HIPCHK(hipMemsetAsync(c->d_stepc, 0, sizeof(int) * c->ncase, c->stream));
+    if (int32_t rc = open_call(c)) return rc;
     if (!recut)
       if (int32_t rc = enqueue_step(c)) return rc;
   }
   if (recut)
     if (int32_t rc = run_recut_steps(c, 1)) return rc;
-  int st = 0;
-  if (int32_t rc = read_status(c, &st)) return rc;
-  std::vector<double> nb(6 * nmi(c));
-  HIPCHK(hipMemcpy(nb.data(), c->d_norms, sizeof(double) * nb.size(), hipMemcpyDeviceToHost));
+  int st = 0, steps = 0;
+  if (int32_t rc = close_call(c, true, &steps, &st)) return rc;
+  const double* nb = c->h_call;
   for (int i = 0; i < nmi(c); ++i) {
     if (norms) { norms[3 * i] = nb[6 * i]; norms[3 * i + 1] = nb[6 * i + 1]; norms[3 * i + 2] = nb[6 * i + 2]; }
     if (argmax) {
@@ -1390,8 +1388,7 @@ extern "C" int32_t ot2d_iterate(ot2d_case* c, int32_t niter, double* hist, int32
   {
     Fp32Order order(c);
     HIPCHK(order.error());
-    if (int32_t rc = clear_status(c)) return rc;
-    HIPCHK(hipMemsetAsync(c->d_stepc, 0, sizeof(int) * c->ncase, c->stream));
+    if (int32_t rc = open_call(c)) return rc;
     if (!recut) {
       if (int32_t rc = ensure_graph(c)) return rc;
       for (int it = 0; it < niter; ++it) HIPCHK(hipGraphLaunch(c->graph, c->stream));
@@ -1404,7 +1401,7 @@ extern "C" int32_t ot2d_iterate(ot2d_case* c, int32_t niter, double* hist, int32
     HIPCHK(hipMemcpyAsync(c->h_hist, c->d_hist, sizeof(double) * (size_t)niter * per, hipMemcpyDeviceToHost,
                           c->stream));
   int st = 0, steps = 0;
-  if (int32_t rc = read_steps_status(c, &steps, &st)) return rc;
+  if (int32_t rc = close_call(c, false, &steps, &st)) return rc;
   if (hist && steps > 0) memcpy(hist, c->h_hist, sizeof(double) * (size_t)steps * per);
   c->istep0 += steps;
   if (done) *done = steps;
@@ -1482,8 +1479,7 @@ extern "C" int32_t ot2d_iterate_noalloc(ot2d_case* c, int32_t niter, double* his
   {
     Fp32Order order(c);
     HIPCHK(order.error());
-    if (int32_t rc = clear_status(c)) return rc;
-    HIPCHK(hipMemsetAsync(c->d_stepc, 0, sizeof(int) * c->ncase, c->stream));
+    if (int32_t rc = open_call(c)) return rc;
     // the captured step when one exists (an earlier ot2d_iterate made it);
     // otherwise the same kernels launched one by one (capturing a graph
     // allocates)
@@ -1649,7 +1645,7 @@ extern "C" int32_t ot2d_profile(ot2d_case* c, int32_t nsteps, double* stage_ms, 
         break;
       }
     }
-    if (rc == OT2D_OK) rc = read_steps_status(c, &steps, &st);
+    if (rc == OT2D_OK) rc = close_call(c, false, &steps, &st);
   }
   for (int i = 0; i < created; ++i) (void)hipEventDestroy(mk.ev[i]);
   (void)hipEventDestroy(ev0);
