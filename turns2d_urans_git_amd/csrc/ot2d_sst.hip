@@ -206,7 +206,7 @@ __global__ __launch_bounds__(256) void k_sst_blend(const DevMesh* __restrict__ M
   const gd_t u = M.sa_u;
   const gd_t v = M.sa_v;
   long long n2 = (long long)jd * M.kd;
-  for (long long i = blockIdx.x * 256ll + threadIdx.x; i < n2; i += 256ll * gridDim.x) {
+  for (long long i = xcd_tile(gridDim.x) * 256ll + threadIdx.x; i < n2; i += 256ll * gridDim.x) {
     const int j = 1 + (int)(i % jd), k = 1 + (int)(i / jd);
     const double rho = rho_of(M, i);
     double f1 = 0.0, X = 0.0;
@@ -281,7 +281,7 @@ __global__ __launch_bounds__(256) void k_sst_rhs(const DevMesh* __restrict__ Ms)
   const gd_t yx = M.yx;
   const gd_t yy = M.yy;
   long long ncell = (long long)nj * nk;
-  for (long long w = blockIdx.x * 256ll + threadIdx.x; w < ncell; w += 256ll * gridDim.x) {
+  for (long long w = xcd_tile(gridDim.x) * 256ll + threadIdx.x; w < ncell; w += 256ll * gridDim.x) {
     const int j = js + (int)(w % nj), k = ks + (int)(w / nj);
     const long long i = cell(M, j, k);
     const long long iw = i - 1, ie = i + 1, is = i - jd, in = i + jd;
@@ -407,7 +407,8 @@ __global__ __launch_bounds__(64) void k_sst_solve_j(const DevMesh* __restrict__ 
 // of the threads per equation, their update with its clip
 // (src/komegasst.f:146-172) and findturm for the interior after it (the halo
 // ring follows the final komegabc in k_sst_bc).  301x90: 10.6 us, 385x97
-// with 401x401: 24.6 us (one wave per line and equation from both ends, and
+// with 401x401: 20.6 us (24.6 without the runs per
+// XCD: 4 or 8 columns are a part of a cache line; one wave per line and equation from both ends, and
 // findturm in a pass of its own: 25 and 75 us).
 template <int TC>
 __global__ __launch_bounds__(512) void k_sst_solve_k(const DevMesh* __restrict__ Ms) {
@@ -415,8 +416,9 @@ __global__ __launch_bounds__(512) void k_sst_solve_k(const DevMesh* __restrict__
   constexpr int PM = PCOL_M;
   const DevMesh& M = Ms[blockIdx.y];
   if (*M.status) return;
-  const int j0 = M.js + (int)blockIdx.x * TC;
-  if (j0 > M.je) return;
+  const int group = xcd_tile((M.je - M.js + TC) / TC);
+  if (group < 0) return;
+  const int j0 = M.js + group * TC;
   // thread (column, equation, part): both equations of a column exchange
   // through the same calls, as 2*TC columns
   const int n = M.ke - M.ks + 1, P = (n + PM - 1) / PM, tid = (int)threadIdx.x;
@@ -488,9 +490,9 @@ hipError_t launch_sst(const DevMesh* dM, const DevMesh* hM, int nmi, Marks* mk, 
   hipLaunchKernelGGL(k_sst_bc, dim3(nmi), dim3(BC_ALL_THREADS), 0, st, dM, 0);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_SA_BC, st);
-  hipLaunchKernelGGL(k_sst_blend, dim3(nblk3(mx, 256), nmi), dim3(256), 0, st, dM);
+  hipLaunchKernelGGL(k_sst_blend, dim3(xcd_grid(nblk3(mx, 256)), nmi), dim3(256), 0, st, dM);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  hipLaunchKernelGGL(k_sst_rhs, dim3(nblk3(mx, 256), nmi), dim3(256), 0, st, dM);
+  hipLaunchKernelGGL(k_sst_rhs, dim3(xcd_grid(nblk3(mx, 256)), nmi), dim3(256), 0, st, dM);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_SA_RHS, st);
   hipLaunchKernelGGL(k_sst_solve_j, dim3(2 * mk_, nmi), dim3(64), 0, st, dM);
@@ -500,7 +502,7 @@ hipError_t launch_sst(const DevMesh* dM, const DevMesh* hM, int nmi, Marks* mk, 
     const int np = (mk_ + PCOL_M - 1) / PCOL_M;   // parts of the longest column
     auto solve_k = [&](auto kern, int tc) {
       const int nt = (2 * np * tc + 63) / 64 * 64;
-      hipLaunchKernelGGL(kern, dim3((mj + tc - 1) / tc, nmi), dim3(nt), sizeof(double) * 6 * nt, st, dM);
+      hipLaunchKernelGGL(kern, dim3(xcd_grid((mj + tc - 1) / tc), nmi), dim3(nt), sizeof(double) * 6 * nt, st, dM);
     };
     if (np <= SSTK_NP8) solve_k(k_sst_solve_k<8>, 8);
     else solve_k(k_sst_solve_k<4>, 4);

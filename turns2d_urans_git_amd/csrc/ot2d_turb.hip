@@ -764,8 +764,9 @@ __global__ __launch_bounds__(SAK_NT) void k_sa_solve_k(const DevMesh* __restrict
   constexpr int PM = PCOL_M;
   const DevMesh& M = Ms[blockIdx.y];
   if (*M.status) return;
-  const int j0 = M.js + (int)blockIdx.x * TC;
-  if (j0 > M.je) return;
+  const int group = xcd_tile((M.je - M.js + TC) / TC);
+  if (group < 0) return;
+  const int j0 = M.js + group * TC;
   const int n = M.ke - M.ks + 1, P = (n + PM - 1) / PM;
   const int j = j0 + (int)threadIdx.x % TC, k0 = ((int)threadIdx.x / TC) * PM;
   const bool col = j <= M.je;
@@ -911,7 +912,7 @@ hipError_t launch_sa(const DevMesh* dM, const DevMesh* hM, int nmi, Marks* mk, h
   const bool wide = np * 16 <= SAK_NT && (sa_lane < 0 ? cols > SAK_WIDE_COLS : sa_lane == 0);
   auto solve_k = [&](auto kern, int tc) {
     const int nt = (np * tc + 63) / 64 * 64;
-    hipLaunchKernelGGL(kern, dim3((mj + tc - 1) / tc, nmi), dim3(nt), sizeof(double) * 6 * nt, st, dM, ovl);
+    hipLaunchKernelGGL(kern, dim3(xcd_grid((mj + tc - 1) / tc), nmi), dim3(nt), sizeof(double) * 6 * nt, st, dM, ovl);
   };
   if (wide) solve_k(k_sa_solve_k<16>, 16);
   else solve_k(k_sa_solve_k<8>, 8);
