@@ -223,7 +223,7 @@ int32_t ot2d_batch_admit(ot2d_case* c, int32_t icase, const ot2d_params* p, cons
 
 /* ------------------------------------------------------------ launch choices
  * Launch shapes that change speed but not results: sweep (0, 1 or 2) picks
- * the FP32 LU-SGS sweep's LDS ring depth and producer count (12 slots and
+ * the FP32 LU-SGS sweep's LDS ring depth and producer count (15 slots and
  * 3 producer waves, 18 and 3, 12 and 4); sa_lane picks how
  * many adjacent columns a workgroup of the SA k solve takes (-1 by the number
  * of columns, 0 16 where columns hold up to 256 cells, 1 8).

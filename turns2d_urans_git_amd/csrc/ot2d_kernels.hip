@@ -2974,13 +2974,24 @@ static hipError_t launch_lu64(const DevMesh* dM, const DevMesh* hM, int nmi, int
   return hipSuccess;
 }
 
-// LDS ring slots of the FP32 sweeps (LU32_NV KiB each and two tag words): 14
-// slots, so two workgroups fit one CU's LDS; producer waves and the steps
-// each keeps in flight
-// the FP32 sweep's instantiations (ring steps S, producer waves NP,
+// The FP32 sweep's instantiations (ring steps S, producer waves NP,
 // deliveries in flight per producer PD): the same arithmetic in the same
-// order, so the choice (LaunchCfg::sweep, the autotuner's) changes no result
-constexpr size_t lu32_lds(int S) { return (size_t)S * LU32_NV * 1024 + 16 * ((S * 8 + 15) / 16); }
+// order, so the choice (LaunchCfg::sweep, the autotuner's) changes no result.
+// Forward + backward, us:       513x129  385x97 with 401x401  60 cases (263 blocks)
+//   S 12, NP 3, PD 5              164         234               530
+//   S 15, NP 3, PD 5              160         231               487
+//   S 18, NP 3, PD 5              162         234               490
+//   S 12, NP 4, PD 6              166         -                 505
+//   S 24 or 30, NP 3, PD 5        164         235-241           487
+// LDS of a workgroup: the ring (LU32_NV KiB and two tag words a slot), and
+// more than half a CU's, so that a CU takes one workgroup at a time.  Two that
+// share a CU while others stand idle are the last to end: 50 cases (211
+// blocks) 494 us with two of S = 15 to a CU, 409 with one; 60 cases 530 and
+// 487; 120 cases (513 blocks, two rounds of them) 871 and 832.
+constexpr size_t lu32_lds(int S) {
+  const size_t ring = (size_t)S * LU32_NV * 1024 + 16 * ((S * 8 + 15) / 16), half = 80 * 1024 + 16;
+  return ring > half ? ring : half;
+}
 
 template <int S, int NP, int PD>
 static hipError_t launch_sweeps32(const DevMesh* dM, int wmax, int nmi, Marks* mk, hipStream_t st) {
@@ -3025,7 +3036,7 @@ static hipError_t launch_lu32(const DevMesh* dM, const DevMesh* hM, int nmi, int
   if (e != hipSuccess) return e;
   mark(mk, OT2D_ST_LU_PREP, st);
   switch (sweep) {
-    case 0: e = launch_sweeps32<12, 3, 5>(dM, wmax, nmi, mk, st); break;
+    case 0: e = launch_sweeps32<15, 3, 5>(dM, wmax, nmi, mk, st); break;
     case 1: e = launch_sweeps32<18, 3, 5>(dM, wmax, nmi, mk, st); break;
     case 2: e = launch_sweeps32<12, 4, 6>(dM, wmax, nmi, mk, st); break;
     default: return hipErrorInvalidValue;
