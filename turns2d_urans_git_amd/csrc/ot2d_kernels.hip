@@ -7,14 +7,14 @@
 //   muscld_new       821-912; norms step.f:53-115
 //   timespectralrhs  src/sources.f:2-27          k_tsrhs
 //   rbc              src/bc.f:88-177             k_rbc            (1 block / instance)
-//   s*tscale, ilu2d  src/step.f:141-159,         FP64: k_lu_prep, k_lu_sweep<double,RL>
-//                    src/lhs.f:470-814            (one wave per instance, skewed rows),
+//   s*tscale, ilu2d  src/step.f:141-159,         FP64: k_lu_prep, k_lu_sweep64
+//                    src/lhs.f:470-814            (32-row workgroups),
 //                                                 k_lu_finish; FP32 operator: k_lu_prep32,
 //                                                 k_lu_sweep32 (32-row workgroups),
 //                                                 k_lu_finish<float>
 //   q update         src/step.f:205-211          fused in k_lu_finish (Euler) or
 //   monitor          src/step.f:332-392          k_update_monitor; k_monitor alone
-//   initia geometry  src/init.f:2-177, setup.f   k_init_geometry
+//   initia geometry  src/init.f:2-177, setup.f   k_init_geometry; turned grids k_metrics
 //   force2d          src/forces.f:111-398        k_forces
 //
 // Arithmetic follows the reference expressions operand for operand; the
@@ -720,7 +720,7 @@ __device__ __forceinline__ void face_states_weno(const double* sf0, int stv, int
 // the chip and idle lanes of the last pass cost issue slots.  513x129 (256
 // tiles): 10 us (576), 13 (256), 15.5 with a pass or two per direction before;
 // 385x97 with 401x401, WENO5 (1206 tiles): 38 / 41 / 47; 60 cases (15200
-// tiles): 333 (576), 270 (256), 301 before.  FP64 issue binds the last
+// tiles): 333 (576), 270 (256; 254 with xcd_tile), 301 before.  FP64 issue binds the last
 // (800 operations a face).
 template <int H, int NT>
 __global__ __launch_bounds__(NT) void k_residual(const DevMesh* __restrict__ Ms, const ResTile* __restrict__ tiles,

@@ -406,9 +406,9 @@ __global__ __launch_bounds__(64) void k_sst_solve_j(const DevMesh* __restrict__ 
 // lsolvek2 of both equations for TC adjacent j columns (blockIdx.x), one half
 // of the threads per equation, their update with its clip
 // (src/komegasst.f:146-172) and findturm for the interior after it (the halo
-// ring follows the final komegabc in k_sst_bc).  301x90: 10.6 us, 385x97
-// with 401x401: 20.6 us (24.6 without the runs per
-// XCD: 4 or 8 columns are a part of a cache line; one wave per line and equation from both ends, and
+// ring follows the final komegabc in k_sst_bc).  301x90: 10.5 us, 385x97
+// with 401x401: 18 us (25 without the runs per XCD, for 4 or 8 columns are a
+// part of a cache line; one wave per line and equation from both ends, and
 // findturm in a pass of its own: 25 and 75 us).
 template <int TC>
 __global__ __launch_bounds__(512) void k_sst_solve_k(const DevMesh* __restrict__ Ms) {

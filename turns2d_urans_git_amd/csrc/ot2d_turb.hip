@@ -235,7 +235,7 @@ __device__ __forceinline__ Tri lds_tri(const double (&g)[3][N], int c) {
 }
 
 // Bound by latency at the 12 waves a CU its LDS (41 KB) and registers (168)
-// allow; FP64 issue alone is 97 us of the 60-case batch's 228 us (286 us with
+// allow; FP64 issue alone is 97 us of the 60-case batch's 223 us (286 us with
 // each array in memory of its own, 77 KB and 8 waves a CU); 513x129: 9.7 us
 // both ways.
 // With norms set, the residual is complete once this kernel has added the
@@ -562,9 +562,9 @@ __device__ __forceinline__ void sa_half(double va, double na, double vb, double 
 // what the stencil reads of a cell (nu-tilde, vnul, contravariant velocities,
 // velocities, metrics) is formed once for the tile and its one-cell ring in
 // LDS.  Bound by FP64 issue (about 1100 operations a cell, 40 divisions among
-// them).  60 cases (3.9 M cells): 178 us; with every thread gathering its
+// them).  60 cases (3.9 M cells): 175 us; with every thread gathering its
 // neighbours' planes and forming their quantities again 256 us (two
-// divisions a neighbour, 160-220 registers).  513x129: 9 us both ways.
+// divisions a neighbour, 160-220 registers).  513x129: 8.1 us (9).
 constexpr int SAR_N = VIS_NR;
 struct SaLds {
   double nt[SAR_N], vn[SAR_N], U[SAR_N], V[SAR_N], u[SAR_N], v[SAR_N], xx[SAR_N], xy[SAR_N], yx[SAR_N], yy[SAR_N];
@@ -754,8 +754,8 @@ __global__ __launch_bounds__(64) void k_sa_solve_j(const DevMesh* __restrict__ M
 // lsolvek (src/samodel2d.f:1347-1385), s2 and the nu-tilde update with its
 // clip (src/samodel2d.f:157-188), then the interior eddy viscosity (c_turm)
 // for TC adjacent j columns: 16 make whole 128-byte row segments for batches
-// (60 cases 113 us, 8 columns 137; lane per line and an update pass of its
-// own 125), 8 twice the workgroups for few columns (513x129: 8.9 us, 16
+// (60 cases 108 us, 8 columns 137; lane per line and an update pass of its
+// own 125), 8 twice the workgroups for few columns (513x129: 8.0 us, 16
 // columns 9.6; two lanes per column from both ends 17.4).
 constexpr int SAK_NT = 512;
 template <int TC>
