@@ -225,8 +225,8 @@ int32_t ot2d_batch_admit(ot2d_case* c, int32_t icase, const ot2d_params* p, cons
  * Launch shapes that change speed but not results: sweep (0, 1 or 2) picks
  * the FP32 LU-SGS sweep's LDS ring depth and producer count (15 slots and
  * 3 producer waves, 18 and 3, 12 and 4); sa_lane picks how
- * many adjacent columns a workgroup of the SA k solve takes (-1 by the number
- * of columns, 0 16 where columns hold up to 256 cells, 1 8).
+ * many adjacent columns a workgroup of the SA k solve takes (-1 and 1: 8, 0:
+ * 16 where columns hold up to 256 cells).
  * Every choice gives bit-identical states.  No counterpart in the reference,
  * whose loops have one shape. */
 int32_t ot2d_set_launch(ot2d_case* c, int32_t sweep, int32_t sa_lane);

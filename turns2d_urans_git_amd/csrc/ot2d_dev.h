@@ -497,7 +497,7 @@ hipError_t launch_rbc(const DevMesh* dM, int nmi, hipStream_t st);
 constexpr int LU32_SWEEP_VARIANTS = 3;   // FP32 sweep instantiations (ring steps, producers, prefetch)
 struct LaunchCfg {
   int sweep = 0;     // 0: 12 ring steps, 3 producers; 1: 18, 3; 2: 12, 4 (with deeper prefetch)
-  int sa_lane = -1;  // SA k solves: columns per workgroup, 0: 16, 1: 8, -1 by the number of columns
+  int sa_lane = -1;  // SA k solves: columns per workgroup, 0: 16, 1 and -1: 8
 };
 // fuse_update: 1 the q update and monitor in k_lu_finish (Euler), | 2
 // k_lu_finish also leaves the SA model's laminar viscosity and velocities

@@ -753,10 +753,12 @@ __global__ __launch_bounds__(64) void k_sa_solve_j(const DevMesh* __restrict__ M
 
 // lsolvek (src/samodel2d.f:1347-1385), s2 and the nu-tilde update with its
 // clip (src/samodel2d.f:157-188), then the interior eddy viscosity (c_turm)
-// for TC adjacent j columns: 16 make whole 128-byte row segments for batches
-// (60 cases 108 us, 8 columns 137; lane per line and an update pass of its
-// own 125), 8 twice the workgroups for few columns (513x129: 8.0 us, 16
-// columns 9.6; two lanes per column from both ends 17.4).
+// for TC adjacent j columns.  8 columns are half a 128-byte line; with the
+// neighbouring workgroup on the same XCD the other half comes out of its L2,
+// and twice the workgroups of 16 columns hide more latency: 60 cases 102 us
+// (16 columns 111, 4 columns 126; 8 without the runs per XCD 137; lane per line
+// and an update pass of its own 125), 20 cases 35 (16: 37), 513x129 8.0 (16:
+// 8.9, 4: 7.6; two lanes per column from both ends 17.4).
 constexpr int SAK_NT = 512;
 template <int TC>
 __global__ __launch_bounds__(SAK_NT) void k_sa_solve_k(const DevMesh* __restrict__ Ms, int ovl) {
@@ -876,12 +878,6 @@ hipError_t launch_sa_prim(const DevMesh* dM, const DevMesh* hM, int nmi, hipStre
   return hipGetLastError();
 }
 
-// columns (all instances) above which the k solves take 16 columns per
-// workgroup instead of 8: at 2048 columns, 8 fill the chip with 256
-// workgroups (figures at k_sa_solve_k).  Columns of more than 256 cells
-// (parts x 16 columns over 512 threads) always take 8.
-constexpr long long SAK_WIDE_COLS = 2048;
-
 // vmu_sa for every instance (src/samodel2d.f:2-197, itrans = 0)
 hipError_t launch_sa(const DevMesh* dM, const DevMesh* hM, int nmi, Marks* mk, hipStream_t st, int sa_lane,
                      int prim_done, int ovl) {
@@ -907,9 +903,9 @@ hipError_t launch_sa(const DevMesh* dM, const DevMesh* hM, int nmi, Marks* mk, h
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_SA_SOLVE_J, st);
   const int np = (mk_ + PCOL_M - 1) / PCOL_M;   // parts of the longest column
-  long long cols = 0;
-  for (int i = 0; i < nmi; ++i) cols += hM[i].je - hM[i].js + 1;
-  const bool wide = np * 16 <= SAK_NT && (sa_lane < 0 ? cols > SAK_WIDE_COLS : sa_lane == 0);
+  // 8 columns a workgroup; 16 where the launch choice asks for them and they
+  // fit 512 threads (columns of up to 256 cells).  Figures at k_sa_solve_k.
+  const bool wide = np * 16 <= SAK_NT && sa_lane == 0;
   auto solve_k = [&](auto kern, int tc) {
     const int nt = (np * tc + 63) / 64 * 64;
     hipLaunchKernelGGL(kern, dim3(xcd_grid((mj + tc - 1) / tc), nmi), dim3(nt), sizeof(double) * 6 * nt, st, dM, ovl);
