@@ -265,18 +265,20 @@ int32_t ot2d_set_convergence(ot2d_case* c, int32_t icase, double rsum_tol);
 /* Enqueues niter steps on the case's stream and returns without waiting
  * (no residual history); ot2d_sync or ot2d_batch_status waits.  Cases on
  * different streams overlap on the device, except that the steps of cases
- * with lu_fp32 = 1 are ordered across such cases on one device (each
- * waits for the FP32 work enqueued before it by any case). */
+ * whose LU-SGS sweeps pass values between workgroups (lu_fp32 = 1, or FP64
+ * with more than 32 rows, kmax > 33) are ordered across such cases on one
+ * device (each waits for the work of that kind enqueued before it by any
+ * case). */
 int32_t ot2d_iterate_async(ot2d_case* c, int32_t niter);
 int32_t ot2d_sync(ot2d_case* c);
 /* *idle = 1 when everything enqueued for the case has finished, else 0;
  * never waits.  For request loops that advance each batch as soon as its
  * previous steps are done; no counterpart in the reference. */
 int32_t ot2d_query(ot2d_case* c, int32_t* idle);
-/* on = 1 (the default): the order of FP32 work across cases above; on = 0:
- * lifted for the whole process, so FP32 cases on different streams overlap
- * like FP64 ones.  Applies to work enqueued after the call.  No counterpart
- * in the reference. */
+/* on = 1 (the default): the order of steps across cases above; on = 0:
+ * lifted for the whole process, so all cases on different streams overlap.
+ * Applies to work enqueued after the call.  No counterpart in the
+ * reference. */
 int32_t ot2d_set_fp32_order(int32_t on);
 
 /* ot2d_iterate without allocating: the same steps, the same outputs (hist,

@@ -531,9 +531,9 @@ def ihc_connect(lib, prefix, meshes, errfn=None) -> IHCLists:
 
 
 def set_fp32_order(lib, prefix, on: bool):
-    """Order FP32 LU-SGS work of different cases across streams (on, the
-    default) or let it overlap (off), for the whole process
-    (ot2d_set_fp32_order)."""
+    """Order the steps of cases with FP32 LU-SGS, or FP64 with more than 32
+    rows, across streams (on, the default) or let them overlap (off), for the
+    whole process (ot2d_set_fp32_order)."""
     rc = bind(lib, prefix)["set_fp32_order"](1 if on else 0)
     if rc:
         raise CaseError(rc, "set_fp32_order")

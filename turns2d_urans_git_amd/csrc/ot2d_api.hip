@@ -152,64 +152,78 @@ struct ot2d_ihc_lists {
 // stream the step runs the model after ilu2d, as before.
 constexpr bool kSaBesideLu = false;
 
-// ------------------------------------------------ order of FP32 LU-SGS work
-// Cases whose LU-SGS sweeps run in FP32 (lu_fp32) never run at the same time
-// as one another on a device: every call that enqueues such a case's sweeps
-// first makes the case's stream wait for the FP32 work last enqueued by any
-// case on that device, and records the end of its own.  FP32 batches
-// overlapping one another on several streams have diverged from their
-// one-stream results now and then; the cause is not shown (it is not the
-// sweeps' inter-workgroup mail, whose entries carry the sweep number), so
-// the library keeps such work apart.  FP64 cases still overlap freely.
+// ------------------------------------------- order of block-coupled sweeps
+// The LU-SGS sweeps of an FP32 case (lu_fp32), and those of an FP64 case with
+// more than one block of LU_R rows, pass values between workgroups of one
+// launch (tickets, tagged mail, bounded waits).  Such cases never run at the
+// same time as one another on a device: every call that enqueues such a
+// case's sweeps first makes the case's stream wait for the work of that kind
+// last enqueued by any case on that device, and records the end of its own.
+// FP32 batches overlapping one another on several streams have diverged from
+// their one-stream results now and then; the cause is not shown (it is not
+// the inter-workgroup mail, whose entries carry the sweep number).  No FP64
+// run has diverged, but its sweeps wait and post in the same way, so they
+// keep the same order.  Cohorts of 7 SA cases on streams of their own, FP64,
+// time for a step of all: 2 cohorts 691 us in order, 377 overlapping; 4
+// cohorts 1385 and 775; 8 cohorts 2825 and 1218.  FP64 cases of one block
+// pass nothing between workgroups and overlap with everything.
 // ot2d_set_fp32_order(0) lifts the order for the process.
 namespace {
 constexpr int kMaxDevices = 64;
-struct Fp32Chain {
+struct SweepChain {
   std::mutex mu;
   hipEvent_t ev[kMaxDevices] = {};
   std::atomic<int> on{1};
 };
-Fp32Chain g_fp32;
+SweepChain g_sweeps;
 
-// held while one FP32 case enqueues its work
-class Fp32Order {
+// held while one such case enqueues its work
+class SweepOrder {
  public:
-  explicit Fp32Order(const ot2d_case* c);
-  ~Fp32Order();
+  explicit SweepOrder(const ot2d_case* c);
+  ~SweepOrder();
   hipError_t error() const { return e_; }
 
  private:
   const ot2d_case* c_ = nullptr;
   hipError_t e_ = hipSuccess;
 };
+
+// some sweep of the case runs in several workgroups, or in FP32
+bool block_coupled(const ot2d_case* c) {
+  if (c->p.lu_fp32) return true;
+  for (const auto& mb : c->m)
+    if (mb.kmax - 1 > LU_R) return true;
+  return false;
+}
 }  // namespace
 
-Fp32Order::Fp32Order(const ot2d_case* c) {
-  if (!c->p.lu_fp32 || !g_fp32.on.load(std::memory_order_relaxed)) return;
+SweepOrder::SweepOrder(const ot2d_case* c) {
+  if (!g_sweeps.on.load(std::memory_order_relaxed) || !block_coupled(c)) return;
   c_ = c;
-  g_fp32.mu.lock();
-  e_ = hipStreamWaitEvent(c->stream, g_fp32.ev[c->device], 0);
+  g_sweeps.mu.lock();
+  e_ = hipStreamWaitEvent(c->stream, g_sweeps.ev[c->device], 0);
 }
 
-Fp32Order::~Fp32Order() {
+SweepOrder::~SweepOrder() {
   if (!c_) return;
-  (void)hipEventRecord(g_fp32.ev[c_->device], c_->stream);
-  g_fp32.mu.unlock();
+  (void)hipEventRecord(g_sweeps.ev[c_->device], c_->stream);
+  g_sweeps.mu.unlock();
 }
 
 extern "C" int32_t ot2d_set_fp32_order(int32_t on) {
   if (on != 0 && on != 1) return fail(OT2D_ERR_ARG, "ot2d_set_fp32_order: on must be 0 or 1");
   // taken so that no enqueue is half way through its ordered section
-  std::lock_guard<std::mutex> lock(g_fp32.mu);
-  g_fp32.on.store(on, std::memory_order_relaxed);
+  std::lock_guard<std::mutex> lock(g_sweeps.mu);
+  g_sweeps.on.store(on, std::memory_order_relaxed);
   return OT2D_OK;
 }
 
-// the device's ordering event, created with the first FP32 case on it
-static int32_t fp32_chain_init(int dev) {
+// the device's ordering event, created with the first case on it
+static int32_t sweep_chain_init(int dev) {
   if (dev < 0 || dev >= kMaxDevices) return fail(OT2D_ERR_ARG, "device %d out of range", dev);
-  std::lock_guard<std::mutex> lock(g_fp32.mu);
-  if (!g_fp32.ev[dev]) HIPCHK(hipEventCreateWithFlags(&g_fp32.ev[dev], hipEventDisableTiming));
+  std::lock_guard<std::mutex> lock(g_sweeps.mu);
+  if (!g_sweeps.ev[dev]) HIPCHK(hipEventCreateWithFlags(&g_sweeps.ev[dev], hipEventDisableTiming));
   return OT2D_OK;
 }
 
@@ -628,8 +642,7 @@ static int32_t create_impl(const ot2d_params* ps, int32_t ncase, int32_t nmesh, 
   (void)hipGetDevice(&c->device);
   hipError_t e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
   if (e != hipSuccess) { free_case(c); return fail(OT2D_ERR_HIP, "stream: %s", hipGetErrorString(e)); }
-  if (p->lu_fp32)
-    if (int32_t rc = fp32_chain_init(c->device)) { free_case(c); return rc; }
+  if (int32_t rc = sweep_chain_init(c->device)) { free_case(c); return rc; }
   if (kSaBesideLu && !c->lamin && c->iturb == 1) {
     if ((e = hipStreamCreateWithFlags(&c->st2, hipStreamNonBlocking)) != hipSuccess ||
         (e = hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming)) != hipSuccess ||
@@ -1121,7 +1134,7 @@ extern "C" int32_t ot2d_rbc(ot2d_case* c) {
 extern "C" int32_t ot2d_lhs(ot2d_case* c) {
   if (!c) return fail(OT2D_ERR_ARG, "null case");
   {
-    Fp32Order order(c);
+    SweepOrder order(c);
     HIPCHK(order.error());
     if (int32_t rc = clear_status(c)) return rc;
     HIPCHK(launch_lu(c->dM, c->hM.data(), nmi(c), 0, c->p.lu_fp32, nullptr, c->stream, c->cfg.sweep));
@@ -1280,7 +1293,7 @@ static int32_t connect_impl(ot2d_case* c, const ot2d_ihcbc* ihcbc, int32_t* nfri
 static int32_t run_recut_steps(ot2d_case* c, int32_t niter) {
   for (int it = 0; it < niter; ++it) {
     {
-      Fp32Order order(c);
+      SweepOrder order(c);
       HIPCHK(order.error());
       if (int32_t rc = enqueue_time_step(c, nullptr, 1)) return rc;
     }
@@ -1290,7 +1303,7 @@ static int32_t run_recut_steps(ot2d_case* c, int32_t niter) {
     if (st) break;   // a stopped case takes no further step
     if (int32_t rc = connect_impl(c, c->ihcbc_saved.data(), nullptr)) return rc;
     {
-      Fp32Order order(c);
+      SweepOrder order(c);
       HIPCHK(order.error());
       if (int32_t rc = enqueue_time_step(c, nullptr, 2)) return rc;
     }
@@ -1304,7 +1317,7 @@ extern "C" int32_t ot2d_step(ot2d_case* c, double* norms, int32_t* argmax) {
     if (!mb.has_grid) return fail(OT2D_ERR_STATE, "ot2d_set_grid not called for every mesh");
   const bool recut = recut_active(c);
   {
-    Fp32Order order(c);
+    SweepOrder order(c);
     HIPCHK(order.error());
     if (int32_t rc = open_call(c)) return rc;
     if (!recut)
@@ -1386,7 +1399,7 @@ extern "C" int32_t ot2d_iterate(ot2d_case* c, int32_t niter, double* hist, int32
   }
   const bool recut = recut_active(c);
   {
-    Fp32Order order(c);
+    SweepOrder order(c);
     HIPCHK(order.error());
     if (int32_t rc = open_call(c)) return rc;
     if (!recut) {
@@ -1477,7 +1490,7 @@ extern "C" int32_t ot2d_iterate_noalloc(ot2d_case* c, int32_t niter, double* his
     if (int32_t rc = scratch_address(c->device, &sp)) return rc;
   if (int32_t rc = set_history(c, sp, niter)) return rc;
   {
-    Fp32Order order(c);
+    SweepOrder order(c);
     HIPCHK(order.error());
     if (int32_t rc = open_call(c)) return rc;
     // the captured step when one exists (an earlier ot2d_iterate made it);
@@ -1530,7 +1543,7 @@ extern "C" int32_t ot2d_iterate_async(ot2d_case* c, int32_t niter) {
     for (auto& M : c->hM) { M.hist = nullptr; M.hist_cap = 0; }
     if (int32_t rc = upload_meshes(c)) return rc;
   }
-  Fp32Order order(c);
+  SweepOrder order(c);
   HIPCHK(order.error());
   if (int32_t rc = clear_status(c)) return rc;
   if (int32_t rc = ensure_graph(c)) return rc;
@@ -1618,7 +1631,7 @@ extern "C" int32_t ot2d_profile(ot2d_case* c, int32_t nsteps, double* stage_ms, 
     rc = fail(OT2D_ERR_HIP, "hipEventCreate: %s", hipGetErrorString(e));
     --created;
   } else if ((rc = clear_status(c)) == OT2D_OK) {
-    Fp32Order order(c);
+    SweepOrder order(c);
     if (order.error() != hipSuccess) rc = fail(OT2D_ERR_HIP, "hipStreamWaitEvent: %s", hipGetErrorString(order.error()));
     e = hipMemsetAsync(c->d_stepc, 0, sizeof(int) * c->ncase, c->stream);
     if (e != hipSuccess) rc = fail(OT2D_ERR_HIP, "hipMemsetAsync: %s", hipGetErrorString(e));
@@ -1989,7 +2002,7 @@ extern "C" int32_t ot2d_autotune(ot2d_case* c, int32_t steps, int32_t* measured)
       c->cfg = cand[k];
       c->graph_valid = 0;
       {
-        Fp32Order order(c);
+        SweepOrder order(c);
         if ((e = order.error()) != hipSuccess) break;
         if ((rc = clear_status(c)) != OT2D_OK) break;
         if ((rc = ensure_graph(c)) != OT2D_OK) break;

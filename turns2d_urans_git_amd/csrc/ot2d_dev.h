@@ -494,6 +494,7 @@ hipError_t launch_conv_check(const DevMesh* dM, const int* inst, const double* t
 hipError_t launch_zero_s(const DevMesh* dM, const DevMesh* hM, int nmi, hipStream_t st);
 hipError_t launch_rbc(const DevMesh* dM, int nmi, hipStream_t st);
 // launch choices that change no result (the autotuner's knobs)
+constexpr int LU_R = 32;   // rows of one LU-SGS sweep workgroup (two lanes per row)
 constexpr int LU32_SWEEP_VARIANTS = 3;   // FP32 sweep instantiations (ring steps, producers, prefetch)
 struct LaunchCfg {
   int sweep = 0;     // 0: 12 ring steps, 3 producers; 1: 18, 3; 2: 12, 4 (with deeper prefetch)

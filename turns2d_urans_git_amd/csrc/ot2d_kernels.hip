@@ -1151,7 +1151,6 @@ __device__ __forceinline__ void nb_k(const CellLoad& c, const LUCellF64& L, doub
 // when the case is created, nothing else writes there) and give zeros.
 // ----------------------------------------------------------------------
 
-constexpr int LU_R = 32;           // rows of one sweep workgroup (two lanes per row)
 constexpr int LU32_R = LU_R;
 constexpr int LU64_PL = 12;        // 16-byte vectors of an FP64 cell record
 constexpr int LU64_STEP = LU64_PL * LU_R;   // ... of one block and step

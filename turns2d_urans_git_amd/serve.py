@@ -14,9 +14,10 @@ time.  Between iterations the loop
 * advances each resident cohort by ``steps_per_tick`` iterations with
   ``ot2d_iterate_async`` as soon as its previous ones are done
   (``ot2d_query`` never waits), so cohorts advance independently and their
-  kernels overlap on the device (the library orders the FP32 LU-SGS work of
-  different cohorts among themselves unless ``ot2d_set_fp32_order(0)``
-  lifts that; FP64 work overlaps with everything);
+  kernels overlap on the device (the library orders the steps of cohorts
+  with FP32 LU-SGS, or FP64 with more than 32 rows, among themselves unless
+  ``ot2d_set_fp32_order(0)`` lifts that; other work overlaps with
+  everything);
 * reads a cohort's per-case states (``ot2d_batch_status``) once its steps
   are done: a case whose residual has reached the tolerance stopped on the
   device (status ``CONVERGED``, set by the step itself before its update), and its
