@@ -1,0 +1,33 @@
+"""Rules the kernels share with the host (csrc/ot2d_plain.h), compiled for the
+CPU.  Each check program says what it holds the rule to."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+CSRC = os.path.join(os.path.dirname(HERE), "turns2d_urans_git_amd", "csrc")
+
+
+@pytest.fixture(scope="module")
+def run_check(tmp_path_factory):
+    if not shutil.which("g++"):
+        pytest.skip("g++ not available")
+    out = tmp_path_factory.mktemp("plain")
+
+    def run(name, *args):
+        exe = str(out / name)
+        subprocess.run(["g++", "-O2", "-std=gnu++17", "-ffp-contract=off", "-Wall", "-Wno-unknown-pragmas", "-I", CSRC,
+                        "-o", exe, os.path.join(HERE, name + ".cpp")], check=True)
+        r = subprocess.run([exe, *args], capture_output=True, text=True, timeout=300)
+        print(r.stdout)
+        assert r.returncode == 0, r.stdout + r.stderr
+
+    return run
+
+
+def test_sweep_waits_outlast_a_queue_put_aside(run_check):
+    """A wait of the sweeps is not given up because the queue was put aside
+    between two polls, and always ends when no answer comes."""
+    run_check("wait_limit_check")

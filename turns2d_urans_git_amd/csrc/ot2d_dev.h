@@ -11,6 +11,7 @@
 #include <stdint.h>
 
 #include "../../include/ot2d.h"
+#include "ot2d_plain.h"
 
 #define OT2D_MAXQ 8
 // longest grid line (interior cells) of the turbulence-model line solves

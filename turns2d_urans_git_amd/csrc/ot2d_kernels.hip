@@ -1527,23 +1527,19 @@ __global__ __launch_bounds__(64 * LP_WAVES) void k_lu_prep32(const DevMesh* __re
       f32x4_t{(float)cb[0], (float)cb[1], (float)cb[2], (float)cb[3]};
 }
 
-// Bounded waits.  Every wait of the FP32 sweeps gives up after LU32_WAIT
-// ticks of the 100 MHz real-time counter (0.5 s; a normal wait is a few
-// microseconds), raising the workgroup's abort flag, so every wave of every
-// workgroup always reaches the end of the kernel; the sweep then reports
-// status 3.
-constexpr unsigned long long LU32_WAIT = 50000000ull;
-
-__device__ __forceinline__ unsigned long long rt_now() { return __builtin_amdgcn_s_memrealtime(); }
-
+// Bounded waits.  Every wait of the FP32 and of the FP64 sweeps gives up at
+// BoundedWait's limit, raising the workgroup's abort flag, so every wave of
+// every workgroup always reaches the end of the kernel; the sweep then
+// reports status 3.
 template <int SLEEP>
 __device__ __forceinline__ bool spin_until_ge(int* w, int target, int* abort_flag) {
   if (__hip_atomic_load(w, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) >= target) return true;
-  const unsigned long long t0 = rt_now();
+  BoundedWait wait;
+  wait.start();
   for (;;) {
     if (__hip_atomic_load(w, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) >= target) return true;
     if (__hip_atomic_load(abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) return false;
-    if (rt_now() - t0 > LU32_WAIT) break;
+    if (wait.over()) break;
     __builtin_amdgcn_s_sleep(SLEEP);
   }
   __hip_atomic_store(abort_flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -1684,7 +1680,8 @@ __global__ __launch_bounds__(64 * (2 + NP)) void k_lu_sweep32(const DevMesh* __r
     const bool writer = (l & 1) == 0;
     int tt = 0;
     bool ok = true;
-    unsigned long long t_wait = rt_now();
+    BoundedWait wait;
+    wait.start();
     while (ok && tt < NT) {
       unsigned v = 0u, vn = 0u;
       int n = 0;   // entries ready from tt on
@@ -1711,7 +1708,7 @@ __global__ __launch_bounds__(64 * (2 + NP)) void k_lu_sweep32(const DevMesh* __r
         vn = __builtin_bit_cast(unsigned, __builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xf, 0xf, true));   // word of lane l^1
         if (n == 0) {
           if (__hip_atomic_load(&abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) break;
-          if (rt_now() - t_wait > LU32_WAIT) {
+          if (wait.over()) {
             __hip_atomic_store(&abort_flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             ok = false;
             break;
@@ -1719,7 +1716,7 @@ __global__ __launch_bounds__(64 * (2 + NP)) void k_lu_sweep32(const DevMesh* __r
           __builtin_amdgcn_s_sleep(1);
           continue;
         }
-        t_wait = rt_now();
+        wait.start();
       } else {
         n = NT - tt < 16 ? NT - tt : 16;   // zero fills
       }
@@ -2125,7 +2122,8 @@ __global__ __launch_bounds__(64 * (2 + NP)) void k_lu_sweep64(const DevMesh* __r
         ok = deliver(e0 + 1, 0, ne, b);
       } else {
         int done = 0;
-        unsigned long long t_wait = rt_now();
+        BoundedWait wait;
+        wait.start();
         while (ok && done < ne) {
           const unsigned long long x0 = word(e0 + (l >> 3), l & 7), x1 = word(e0 + 8 + (l >> 3), l & 7);
           // entry i is ready when its eight lanes are: count the ready prefix
@@ -2139,7 +2137,7 @@ __global__ __launch_bounds__(64 * (2 + NP)) void k_lu_sweep64(const DevMesh* __r
           n = n < ne ? n : ne;
           if (n <= done) {
             if (__hip_atomic_load(&abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) { ok = false; break; }
-            if (rt_now() - t_wait > LU32_WAIT) {
+            if (wait.over()) {
               __hip_atomic_store(&abort_flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
               ok = false;
               break;
@@ -2147,7 +2145,7 @@ __global__ __launch_bounds__(64 * (2 + NP)) void k_lu_sweep64(const DevMesh* __r
             __builtin_amdgcn_s_sleep(1);
             continue;
           }
-          t_wait = rt_now();
+          wait.start();
           // gather each entry's four doubles in its lane through LDS (one
           // wave's LDS operations run in order)
           stage[sw] = (unsigned)x0;
