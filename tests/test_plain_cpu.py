@@ -31,3 +31,10 @@ def test_sweep_waits_outlast_a_queue_put_aside(run_check):
     """A wait of the sweeps is not given up because the queue was put aside
     between two polls, and always ends when no answer comes."""
     run_check("wait_limit_check")
+
+
+def test_tiles_go_round_the_xcds(run_check):
+    """Every tile of a record goes to one workgroup, each XCD takes a run of
+    neighbours, no workgroup of a record's own number of tiles is empty, and
+    over equal records no XCD is left behind."""
+    run_check("xcd_deal_check")

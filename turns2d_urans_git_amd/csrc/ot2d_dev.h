@@ -326,17 +326,11 @@ __device__ __forceinline__ void part_columns(double (&a)[PCOL_M], const double (
   part_expand<M>(a, c, s, XL, w.D);
 }
 
-// Tile of this workgroup among the n of a record, or -1.  Workgroups go to the
-// 8 XCDs in turn; the tiles are dealt out so that each XCD gets a run of
-// neighbours, whose shared halos then come out of its L2.  385x97 with 401x401:
-// FP32 operators 27.7 -> 23.6 us, viscous terms 23.5 -> 21.5; 60 cases: viscous
-// terms 231 -> 223, residual 260 -> 254, SA right-hand side 189 -> 182.  gridDim.x is a
-// multiple of 8 (xcd_grid), at least the n of every record.
-__device__ __forceinline__ int xcd_tile(int n) {
-  const int x = blockIdx.x, run = (n + 7) >> 3, t = (x & 7) * run + (x >> 3);
-  return (x >> 3) < run && t < n ? t : -1;
-}
-inline unsigned xcd_grid(long long n) { return (unsigned)((n + 7) / 8 * 8); }
+// Tile of this workgroup among the n of its record, or -1: xcd_deal.  Against
+// tiles in dispatch order: 385x97 with 401x401, FP32 operators 27.7 -> 23.6
+// us, viscous terms 23.5 -> 21.5; 60 cases: viscous terms 231 -> 223, residual
+// 260 -> 254, SA right-hand side 189 -> 182.
+__device__ __forceinline__ int xcd_tile(int n) { return xcd_deal((int)blockIdx.x, n); }
 
 constexpr int RES_TJ = 32;
 constexpr int RES_TK = 8;

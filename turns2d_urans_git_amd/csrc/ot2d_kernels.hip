@@ -2870,7 +2870,7 @@ constexpr int RES_WIDE_TILES = 2048;
 hipError_t launch_residual(const DevMesh* dM, const ResTile* tiles, int ntiles, int do_norms, int weno,
                            hipStream_t st) {
   auto launch = [&](auto kern, int nt) {
-    hipLaunchKernelGGL(kern, dim3(xcd_grid(ntiles)), dim3(nt), 0, st, dM, tiles, ntiles, do_norms);
+    hipLaunchKernelGGL(kern, dim3(ntiles), dim3(nt), 0, st, dM, tiles, ntiles, do_norms);
   };
   if (ntiles <= RES_WIDE_TILES) {
     if (weno) launch(k_residual<3, 576>, 576);
@@ -3028,7 +3028,7 @@ static hipError_t launch_lu32(const DevMesh* dM, const DevMesh* hM, int nmi, int
     (void)hipFuncSetAttribute((const void*)k_lu_prep32, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LP_LDS);
     attr_set = true;
   }
-  hipLaunchKernelGGL(k_lu_prep32, dim3(xcd_grid(nc), nmi), dim3(64 * LP_WAVES), LP_LDS, st, dM);
+  hipLaunchKernelGGL(k_lu_prep32, dim3((unsigned)nc, nmi), dim3(64 * LP_WAVES), LP_LDS, st, dM);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   mark(mk, OT2D_ST_LU_PREP, st);

@@ -50,6 +50,11 @@ __device__ __forceinline__ double findturm(double rho, double q5, double q6, dou
   double t = a1 * rho * q5 / dmax(a1 * q6, X);
   return dmax(t, 1e-20);
 }
+// workgroups of 256 cells that take the n cells of a record
+__host__ __device__ inline int blocks_of(long long n) {
+  const long long b = (n + 255) / 256;
+  return (int)(b > 4096 ? 4096 : b);
+}
 }  // namespace
 
 // komegabc (src/komegasst.f:906-1434) for one segment
@@ -206,7 +211,9 @@ __global__ __launch_bounds__(256) void k_sst_blend(const DevMesh* __restrict__ M
   const gd_t u = M.sa_u;
   const gd_t v = M.sa_v;
   long long n2 = (long long)jd * M.kd;
-  for (long long i = xcd_tile(gridDim.x) * 256ll + threadIdx.x; i < n2; i += 256ll * gridDim.x) {
+  const int nb = blocks_of(n2), tile = xcd_tile(nb);
+  if (tile < 0) return;
+  for (long long i = tile * 256ll + threadIdx.x; i < n2; i += 256ll * nb) {
     const int j = 1 + (int)(i % jd), k = 1 + (int)(i / jd);
     const double rho = rho_of(M, i);
     double f1 = 0.0, X = 0.0;
@@ -281,7 +288,9 @@ __global__ __launch_bounds__(256) void k_sst_rhs(const DevMesh* __restrict__ Ms)
   const gd_t yx = M.yx;
   const gd_t yy = M.yy;
   long long ncell = (long long)nj * nk;
-  for (long long w = xcd_tile(gridDim.x) * 256ll + threadIdx.x; w < ncell; w += 256ll * gridDim.x) {
+  const int nb = blocks_of(ncell), tile = xcd_tile(nb);
+  if (tile < 0) return;
+  for (long long w = tile * 256ll + threadIdx.x; w < ncell; w += 256ll * nb) {
     const int j = js + (int)(w % nj), k = ks + (int)(w / nj);
     const long long i = cell(M, j, k);
     const long long iw = i - 1, ie = i + 1, is = i - jd, in = i + jd;
@@ -467,11 +476,6 @@ __global__ __launch_bounds__(512) void k_sst_solve_k(const DevMesh* __restrict__
   }
 }
 
-static inline int nblk3(long long n, int per) {
-  long long b = (n + per - 1) / per;
-  return (int)(b < 1 ? 1 : (b > 4096 ? 4096 : b));
-}
-
 // parts of the longest column up to which 8 columns fit 512 threads (beyond: 4)
 constexpr int SSTK_NP8 = 32;
 
@@ -490,9 +494,9 @@ hipError_t launch_sst(const DevMesh* dM, const DevMesh* hM, int nmi, Marks* mk, 
   hipLaunchKernelGGL(k_sst_bc, dim3(nmi), dim3(BC_ALL_THREADS), 0, st, dM, 0);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_SA_BC, st);
-  hipLaunchKernelGGL(k_sst_blend, dim3(xcd_grid(nblk3(mx, 256)), nmi), dim3(256), 0, st, dM);
+  hipLaunchKernelGGL(k_sst_blend, dim3(blocks_of(mx), nmi), dim3(256), 0, st, dM);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  hipLaunchKernelGGL(k_sst_rhs, dim3(xcd_grid(nblk3(mx, 256)), nmi), dim3(256), 0, st, dM);
+  hipLaunchKernelGGL(k_sst_rhs, dim3(blocks_of(mx), nmi), dim3(256), 0, st, dM);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_SA_RHS, st);
   hipLaunchKernelGGL(k_sst_solve_j, dim3(2 * mk_, nmi), dim3(64), 0, st, dM);
@@ -502,7 +506,7 @@ hipError_t launch_sst(const DevMesh* dM, const DevMesh* hM, int nmi, Marks* mk, 
     const int np = (mk_ + PCOL_M - 1) / PCOL_M;   // parts of the longest column
     auto solve_k = [&](auto kern, int tc) {
       const int nt = (2 * np * tc + 63) / 64 * 64;
-      hipLaunchKernelGGL(kern, dim3(xcd_grid((mj + tc - 1) / tc), nmi), dim3(nt), sizeof(double) * 6 * nt, st, dM);
+      hipLaunchKernelGGL(kern, dim3((mj + tc - 1) / tc, nmi), dim3(nt), sizeof(double) * 6 * nt, st, dM);
     };
     if (np <= SSTK_NP8) solve_k(k_sst_solve_k<8>, 8);
     else solve_k(k_sst_solve_k<4>, 4);

@@ -864,7 +864,7 @@ hipError_t launch_visrhs(const DevMesh* dM, const DevMesh* hM, int nmi, hipStrea
     if (e != hipSuccess) return e;
     lds_set = true;
   }
-  hipLaunchKernelGGL(k_visrhs, dim3(xcd_grid(tiles), nmi), dim3(VIS_THREADS), VIS_LDS, st, dM, norms);
+  hipLaunchKernelGGL(k_visrhs, dim3(tiles, nmi), dim3(VIS_THREADS), VIS_LDS, st, dM, norms);
   return hipGetLastError();
 }
 
@@ -896,7 +896,7 @@ hipError_t launch_sa(const DevMesh* dM, const DevMesh* hM, int nmi, Marks* mk, h
   hipLaunchKernelGGL(k_turbc, dim3(nmi), dim3(BC_ALL_THREADS), 0, st, dM, 0, ovl);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_SA_BC, st);
-  hipLaunchKernelGGL(k_sa_rhs, dim3(xcd_grid(vis_tiles(hM, nmi)), nmi), dim3(VIS_THREADS), 0, st, dM);
+  hipLaunchKernelGGL(k_sa_rhs, dim3(vis_tiles(hM, nmi), nmi), dim3(VIS_THREADS), 0, st, dM);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_SA_RHS, st);
   hipLaunchKernelGGL(k_sa_solve_j, dim3(mk_, nmi), dim3(64), 0, st, dM);
@@ -908,7 +908,7 @@ hipError_t launch_sa(const DevMesh* dM, const DevMesh* hM, int nmi, Marks* mk, h
   const bool wide = np * 16 <= SAK_NT && sa_lane == 0;
   auto solve_k = [&](auto kern, int tc) {
     const int nt = (np * tc + 63) / 64 * 64;
-    hipLaunchKernelGGL(kern, dim3(xcd_grid((mj + tc - 1) / tc), nmi), dim3(nt), sizeof(double) * 6 * nt, st, dM, ovl);
+    hipLaunchKernelGGL(kern, dim3((mj + tc - 1) / tc, nmi), dim3(nt), sizeof(double) * 6 * nt, st, dM, ovl);
   };
   if (wide) solve_k(k_sa_solve_k<16>, 16);
   else solve_k(k_sa_solve_k<8>, 8);
