@@ -341,7 +341,7 @@ constexpr int RES_THREADS = RES_TJ * RES_TK;
 // f(segment, t, nt) runs for as many of them side by side as there are waves,
 // each on a group of whole waves (t, nt: the thread's number in its group and
 // the group's size); the phases follow one another with a barrier between.
-constexpr int BC_THREADS = 256, BC_ALL_THREADS = 1024;
+constexpr int BC_THREADS = 256, BC_MAX_THREADS = 1024;
 template <typename F>
 __device__ __forceinline__ void for_phases(const DevMesh& M, F f) {
   const int nw = (int)(blockDim.x >> 6);
@@ -488,6 +488,8 @@ hipError_t launch_conv_check(const DevMesh* dM, const int* inst, const double* t
                              hipStream_t st);
 hipError_t launch_zero_s(const DevMesh* dM, const DevMesh* hM, int nmi, hipStream_t st);
 hipError_t launch_rbc(const DevMesh* dM, int nmi, hipStream_t st);
+// threads of a workgroup that runs an instance's turbulence boundary conditions
+int bc_threads(const DevMesh* hM, int nmi);
 // launch choices that change no result (the autotuner's knobs)
 constexpr int LU_R = 32;   // rows of one LU-SGS sweep workgroup (two lanes per row)
 constexpr int LU32_SWEEP_VARIANTS = 3;   // FP32 sweep instantiations (ring steps, producers, prefetch)

@@ -179,7 +179,7 @@ __device__ void sst_bc_segment(const DevMesh& M, const DevBC& b, int t, int nt) 
 
 // komegabc of an instance by one workgroup, the segments of a phase side by
 // side (they touch disjoint cells), the phases in order
-__global__ __launch_bounds__(BC_ALL_THREADS) void k_sst_bc(const DevMesh* __restrict__ Ms, int eddy) {
+__global__ __launch_bounds__(BC_MAX_THREADS) void k_sst_bc(const DevMesh* __restrict__ Ms, int eddy) {
   const DevMesh& M = Ms[blockIdx.x];
   if (*M.status) return;
   for_phases(M, [&](const DevBC& b, int t, int nt) { sst_bc_segment(M, b, t, nt); });
@@ -187,7 +187,7 @@ __global__ __launch_bounds__(BC_ALL_THREADS) void k_sst_bc(const DevMesh* __rest
   // findturm on the halo ring (F2 = strain = 0 there)
   const int jd = M.jd, kd = M.kd;
   int nring = 2 * jd + 2 * (kd - 2);
-  for (int w = threadIdx.x; w < nring; w += BC_ALL_THREADS) {
+  for (int w = threadIdx.x; w < nring; w += (int)blockDim.x) {
     int j, k;
     if (w < jd) { j = w + 1; k = 1; }
     else if (w < 2 * jd) { j = w - jd + 1; k = kd; }
@@ -491,7 +491,8 @@ hipError_t launch_sst(const DevMesh* dM, const DevMesh* hM, int nmi, Marks* mk, 
   hipError_t e;
   if (!prim_done && (e = launch_sa_prim(dM, hM, nmi, st)) != hipSuccess) return e;
   mark(mk, OT2D_ST_SA_PRIM, st);
-  hipLaunchKernelGGL(k_sst_bc, dim3(nmi), dim3(BC_ALL_THREADS), 0, st, dM, 0);
+  const int nbc = bc_threads(hM, nmi);
+  hipLaunchKernelGGL(k_sst_bc, dim3(nmi), dim3(nbc), 0, st, dM, 0);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_SA_BC, st);
   hipLaunchKernelGGL(k_sst_blend, dim3(blocks_of(mx), nmi), dim3(256), 0, st, dM);
@@ -513,7 +514,7 @@ hipError_t launch_sst(const DevMesh* dM, const DevMesh* hM, int nmi, Marks* mk, 
   }
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_SA_SOLVE_K, st);
-  hipLaunchKernelGGL(k_sst_bc, dim3(nmi), dim3(BC_ALL_THREADS), 0, st, dM, 1);
+  hipLaunchKernelGGL(k_sst_bc, dim3(nmi), dim3(nbc), 0, st, dM, 1);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_SA_EDDY, st);
   return hipSuccess;

@@ -525,14 +525,14 @@ __device__ void turbc_segment(const DevMesh& M, const DevBC& b, int t, int nt) {
 // turbc of an instance by one workgroup (the segments of a phase side by
 // side).  With eddy set (the final turbc) the eddy viscosity of the halo ring
 // follows (c_turm)
-__global__ __launch_bounds__(BC_ALL_THREADS) void k_turbc(const DevMesh* __restrict__ Ms, int eddy, int ovl) {
+__global__ __launch_bounds__(BC_MAX_THREADS) void k_turbc(const DevMesh* __restrict__ Ms, int eddy, int ovl) {
   const DevMesh& M = Ms[blockIdx.x];
   if (*M.status) return;
   for_phases(M, [&](const DevBC& b, int t, int nt) { turbc_segment(M, b, t, nt); });
   if (!eddy) return;
   const int jd = M.jd, kd = M.kd;
   const int nring = 2 * jd + 2 * (kd - 2);
-  for (int w = threadIdx.x; w < nring; w += BC_ALL_THREADS) {
+  for (int w = threadIdx.x; w < nring; w += (int)blockDim.x) {
     int j, k;
     if (w < jd) { j = w + 1; k = 1; }
     else if (w < 2 * jd) { j = w - jd + 1; k = kd; }
@@ -845,6 +845,30 @@ static long long max_cells(const DevMesh* hM, int nmi) {
   return mx;
 }
 
+// As many waves for each segment of an instance's largest phase as its longest
+// segment fills, 256 to 1024 threads in all.  Waves beyond that hold a CU
+// without work while other instances of the batch wait for one: the two calls
+// of a step, 1000 cases of 33x17, SA 11.5 and 12.3 us (1024 threads: 19.6 and
+// 19.8), SST 14.1 and 15.0 (34.5 and 31.9); 1000 cases of 65x33, SA 14.9 and
+// 17.2 (21.4 and 23.9).  From about 129 columns on it is 1024 as before.
+int bc_threads(const DevMesh* hM, int nmi) {
+  int waves = BC_THREADS / 64;
+  for (int i = 0; i < nmi; ++i)
+    for (int ph = 0; ph < hM[i].nbc_phase; ++ph) {
+      int m = 0, longest = 0;
+      for (int ib = 0; ib < hM[i].nbc; ++ib) {
+        const DevBC& b = hM[i].bc[ib];
+        if (b.phase != ph) continue;
+        const int cells = (b.je - b.js + 1) * (b.ke - b.ks + 1);
+        longest = cells > longest ? cells : longest;
+        ++m;
+      }
+      const int w = m * ((longest + 63) / 64);
+      waves = w > waves ? w : waves;
+    }
+  return 64 * waves < BC_MAX_THREADS ? 64 * waves : BC_MAX_THREADS;
+}
+
 // 32x8 tiles of the largest instance
 static int vis_tiles(const DevMesh* hM, int nmi) {
   int tiles = 1;
@@ -893,7 +917,8 @@ hipError_t launch_sa(const DevMesh* dM, const DevMesh* hM, int nmi, Marks* mk, h
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
   mark(mk, OT2D_ST_SA_PRIM, st);
-  hipLaunchKernelGGL(k_turbc, dim3(nmi), dim3(BC_ALL_THREADS), 0, st, dM, 0, ovl);
+  const int nbc = bc_threads(hM, nmi);
+  hipLaunchKernelGGL(k_turbc, dim3(nmi), dim3(nbc), 0, st, dM, 0, ovl);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_SA_BC, st);
   hipLaunchKernelGGL(k_sa_rhs, dim3(vis_tiles(hM, nmi), nmi), dim3(VIS_THREADS), 0, st, dM);
@@ -914,7 +939,7 @@ hipError_t launch_sa(const DevMesh* dM, const DevMesh* hM, int nmi, Marks* mk, h
   else solve_k(k_sa_solve_k<8>, 8);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_SA_SOLVE_K, st);
-  hipLaunchKernelGGL(k_turbc, dim3(nmi), dim3(BC_ALL_THREADS), 0, st, dM, 1, ovl);
+  hipLaunchKernelGGL(k_turbc, dim3(nmi), dim3(nbc), 0, st, dM, 1, ovl);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_SA_EDDY, st);
   return hipSuccess;
