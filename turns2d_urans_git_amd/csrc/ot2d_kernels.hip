@@ -2863,16 +2863,19 @@ hipError_t launch_bc(const DevMesh* dM, const DevMesh* hM, int nmi, int zero_s, 
   return hipSuccess;
 }
 
-// tiles up to which one thread takes at most one face (576 threads); figures
-// at k_residual
-constexpr int RES_WIDE_TILES = 2048;
+// Tiles up to which one thread takes at most one face (576 threads): three and
+// five to a CU.  Both, us, batches of 513x129 (256 tiles each), 576 / 256
+// threads: MUSCL 512 tiles 16.4 / 19.1, 768 21.3 / 22.1, 1024 29.5 / 25.7,
+// 1536 39.8 / 34.1, 2048 49.6 / 42.8; WENO5 768 35.1 / 36.1, 1024 46.8 / 47.8,
+// 1280 50.9 / 53.7, 1536 62.3 / 60.2, 2048 78.2 / 77.3.
+constexpr int RES_WIDE_MUSCL = 768, RES_WIDE_WENO = 1280;
 
 hipError_t launch_residual(const DevMesh* dM, const ResTile* tiles, int ntiles, int do_norms, int weno,
                            hipStream_t st) {
   auto launch = [&](auto kern, int nt) {
     hipLaunchKernelGGL(kern, dim3(ntiles), dim3(nt), 0, st, dM, tiles, ntiles, do_norms);
   };
-  if (ntiles <= RES_WIDE_TILES) {
+  if (ntiles <= (weno ? RES_WIDE_WENO : RES_WIDE_MUSCL)) {
     if (weno) launch(k_residual<3, 576>, 576);
     else launch(k_residual<2, 576>, 576);
   } else {
