@@ -38,3 +38,9 @@ def test_tiles_go_round_the_xcds(run_check):
     neighbours, no workgroup of a record's own number of tiles is empty, and
     over equal records no XCD is left behind."""
     run_check("xcd_deal_check")
+
+
+def test_search_keeps_the_default_unless_clearly_slower(run_check):
+    """A launch choice is taken over the default only when it wins by more
+    than the timings differ among themselves."""
+    run_check("launch_pick_check")

@@ -1932,11 +1932,13 @@ extern "C" int32_t ot2d_autotune(ot2d_case* c, int32_t steps, int32_t* measured)
   std::vector<LaunchCfg> cand;
   const int nsw = c->p.lu_fp32 ? LU32_SWEEP_VARIANTS : 1;
   const bool sa = !c->lamin && c->iturb == 1;
+  int def = 0;   // the default choice's place: sweep 0, and of SA 8 columns
   for (int sw = 0; sw < nsw; ++sw)
     for (int sl = sa ? 0 : -1; sl <= (sa ? 1 : -1); ++sl) {
       LaunchCfg cfg;
       cfg.sweep = sw;
       cfg.sa_lane = sl;
+      if (sw == 0 && sl != 0) def = (int)cand.size();
       cand.push_back(cfg);
     }
   if (int32_t rc = sync(c)) return rc;
@@ -1992,10 +1994,10 @@ extern "C" int32_t ot2d_autotune(ot2d_case* c, int32_t steps, int32_t* measured)
   if (e == hipSuccess) e = hipEventCreate(&e0);
   if (e == hipSuccess) e = hipEventCreate(&e1);
   const LaunchCfg keep = c->cfg;
-  // three rounds over the candidates, each candidate's best round counts
-  // (the rounds interleave, so a slow spell of the device is shared out)
+  // three rounds over the candidates (they interleave, so a slow spell of the
+  // device is shared out)
   constexpr int ROUNDS = 3;
-  std::vector<float> cand_ms(cand.size(), 3.0e38f);
+  std::vector<float> cand_ms(cand.size() * ROUNDS, 0.f);
   int32_t rc = OT2D_OK;
   for (int round = 0; round < ROUNDS && e == hipSuccess && rc == OT2D_OK; ++round)
     for (size_t k = 0; k < cand.size() && e == hipSuccess && rc == OT2D_OK; ++k) {
@@ -2015,21 +2017,18 @@ extern "C" int32_t ot2d_autotune(ot2d_case* c, int32_t steps, int32_t* measured)
       if (e == hipSuccess) e = hipEventSynchronize(e1);
       if (e == hipSuccess) e = hipEventElapsedTime(&ms, e0, e1);
       if (e == hipSuccess) e = copy_state(true);
-      if (e == hipSuccess && ms < cand_ms[k]) cand_ms[k] = ms;
+      cand_ms[k * ROUNDS + round] = ms;
     }
-  int best = -1;
-  for (size_t k = 0; k < cand.size(); ++k)
-    if (cand_ms[k] < 1.0e38f && (best < 0 || cand_ms[k] < cand_ms[best])) best = (int)k;
   if (e0) (void)hipEventDestroy(e0);
   if (e1) (void)hipEventDestroy(e1);
   dfree(save_i);
   cleanup();
   c->graph_valid = 0;
-  if (rc != OT2D_OK || e != hipSuccess || best < 0) {
+  if (rc != OT2D_OK || e != hipSuccess) {
     c->cfg = keep;
     return rc != OT2D_OK ? rc : fail(OT2D_ERR_HIP, "autotune: %s", hipGetErrorString(e));
   }
-  c->cfg = cand[best];
+  c->cfg = cand[pick_launch(cand_ms.data(), (int)cand.size(), ROUNDS, def)];
   {
     std::lock_guard<std::mutex> lk(g_tune.mu);
     tune_cache_store(key, c->cfg);

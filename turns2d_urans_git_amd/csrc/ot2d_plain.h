@@ -38,4 +38,29 @@ OT2D_PLAIN int xcd_deal(int x, int n) {
   return x < n ? c * len + (c < more ? c : more) + (x >> 3) : -1;
 }
 
+// The launch choice a search keeps: n candidates timed in `rounds` rounds,
+// candidate k's times at ms[k * rounds].  The fastest (by its best round) is
+// taken over candidate `def` only if it wins by more than the rounds of
+// both differ among themselves, and by more than 1 %: the choices of a
+// class often lie closer than that (513x129 SA FP32: 263.3, 264.4, 264.8,
+// 265.6, 268.6, 270.0 us a step), and by the best time alone a search took
+// one that is slower than the default.
+inline int pick_launch(const float* ms, int n, int rounds, int def) {
+  auto low = [&](int k) {
+    float v = ms[k * rounds];
+    for (int r = 1; r < rounds; ++r) v = ms[k * rounds + r] < v ? ms[k * rounds + r] : v;
+    return v;
+  };
+  auto spread = [&](int k) {
+    float v = ms[k * rounds];
+    for (int r = 1; r < rounds; ++r) v = ms[k * rounds + r] > v ? ms[k * rounds + r] : v;
+    return v - low(k);
+  };
+  int best = def;
+  for (int k = 0; k < n; ++k)
+    if (low(k) < low(best)) best = k;
+  const float both = spread(def) + spread(best), least = 0.01f * low(def), need = both > least ? both : least;
+  return low(def) - low(best) > need ? best : def;
+}
+
 }  // namespace ot2d
