@@ -1848,9 +1848,9 @@ extern "C" int32_t ot2d_get_launch(ot2d_case* c, int32_t* sweep, int32_t* sa_lan
 }
 
 namespace {
-// a case's shape class: what the launch choices' speed depends on (model,
-// precision, instances, and the number of cases, cells, columns and sweep
-// blocks in powers of two)
+// a case's shape class: what the launch choices' speed depends on (the set of
+// choices, model, precision, instances, and the number of cases, cells,
+// columns and sweep blocks in powers of two)
 std::string shape_class(const ot2d_case* c) {
   int maxj = 0, maxk = 0;
   long long cells = 0;
@@ -1862,8 +1862,9 @@ std::string shape_class(const ot2d_case* c) {
   cells *= c->nspec;
   auto lg = [](long long v) { int b = 0; while (v > 1) { v >>= 1; ++b; } return b; };
   char buf[192];
-  snprintf(buf, sizeof buf, "iturb=%d,lamin=%d,fp32=%d,nspec=%d,cases=2^%d,cells=2^%d,jmax=2^%d,blocks=%d", c->iturb,
-           c->lamin, c->p.lu_fp32 ? 1 : 0, c->nspec, lg(c->ncase), lg(cells), lg(maxj), (maxk - 1 + 31) / 32);
+  snprintf(buf, sizeof buf, "set=%d,iturb=%d,lamin=%d,fp32=%d,nspec=%d,cases=2^%d,cells=2^%d,jmax=2^%d,blocks=%d",
+           LAUNCH_SET, c->iturb, c->lamin, c->p.lu_fp32 ? 1 : 0, c->nspec, lg(c->ncase), lg(cells), lg(maxj),
+           (maxk - 1 + 31) / 32);
   return buf;
 }
 

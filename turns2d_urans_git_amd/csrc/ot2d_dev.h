@@ -493,8 +493,12 @@ int bc_threads(const DevMesh* hM, int nmi);
 // launch choices that change no result (the autotuner's knobs)
 constexpr int LU_R = 32;   // rows of one LU-SGS sweep workgroup (two lanes per row)
 constexpr int LU32_SWEEP_VARIANTS = 3;   // FP32 sweep instantiations (ring steps, producers, prefetch)
+// Version of what the numbers of a LaunchCfg stand for, part of the key that
+// choices are cached under (also in files): raised with every change of an
+// instantiation behind a number.
+constexpr int LAUNCH_SET = 2;
 struct LaunchCfg {
-  int sweep = 0;     // 0: 12 ring steps, 3 producers; 1: 18, 3; 2: 12, 4 (with deeper prefetch)
+  int sweep = 0;     // 0: 15 ring steps, 3 producers; 1: 18, 3; 2: 12, 4 (with deeper prefetch)
   int sa_lane = -1;  // SA k solves: columns per workgroup, 0: 16, 1 and -1: 8
 };
 // fuse_update: 1 the q update and monitor in k_lu_finish (Euler), | 2
