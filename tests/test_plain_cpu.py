@@ -44,3 +44,9 @@ def test_search_keeps_the_default_unless_clearly_slower(run_check):
     """A launch choice is taken over the default only when it wins by more
     than the timings differ among themselves."""
     run_check("launch_pick_check")
+
+
+def test_line_solves_in_parts_are_as_accurate_as_the_recurrence(run_check):
+    """Lines in parts against 113-bit solutions, non-dominant rows among them,
+    beside the one-sided recurrence."""
+    run_check("line_parts_check")

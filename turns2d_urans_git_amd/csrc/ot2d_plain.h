@@ -63,4 +63,95 @@ inline int pick_launch(const float* ms, int n, int rounds, int def) {
   return low(def) - low(best) > need ? best : def;
 }
 
+// ------------------------------------------------- turbulence line solves
+// Tridiagonal line of n cells, a x(i-1) + b x(i) + c x(i+1) = s, solved in
+// parts of M cells, one lane per part (the turbulence models' line solves:
+// lsolvej / lsolvek and their two-equation forms).  The last cell of every
+// part is its separator.  Each lane eliminates its inner cells against the
+// separators on both sides, x(i) = S(i) + L(i) XL + R(i) XR; the separators'
+// own tridiagonal system (one row per part) is solved by parallel cyclic
+// reduction across the parts; the inner cells follow in parallel.  The
+// dependent chain is 2 M + log2(n / M) steps instead of n / 2 for an
+// elimination from both ends by two lanes, which bound these solves.
+// Parts depend on n alone, so every mapping of lines to workgroups gives the
+// same bits.  Quotients are corrected by one residual step (num - den q)
+// and sums use fused operations.  Rows need not be dominant (an upwind row's
+// off-diagonals carry the neighbours' speeds): of 25600 lines of 24 to 1000
+// cells, convective, diffusive and mixed, with speeds that change sign and
+// rows down to a dominance of 1e-3, the median errors relative to the line's
+// largest value are 1.1-3.9e-16 by kind (the one-sided recurrence 1.2-5.1e-16)
+// and the 99th percentiles no larger than the recurrence's
+// (tests/line_parts_check.cpp, against 113-bit solutions).
+// Cells past the line's end are identity rows; a of the first cell and c of
+// the last are zero.
+OT2D_PLAIN int part_cells(int n) { return n <= 512 ? 8 : (n <= 768 ? 12 : 16); }   // at most 64 parts
+
+OT2D_PLAIN double quot(double num, double den, double r) {   // num / den, r = 1 / den
+  const double q = num * r;
+  return __builtin_fma(__builtin_fma(-den, q, num), r, q);
+}
+
+// inner cells 0 .. M-2: s, a, c become S, L, R
+template <int M>
+OT2D_PLAIN void part_eliminate(double (&a)[M], const double (&b)[M], double (&c)[M], double (&s)[M]) {
+  {
+    const double r = 1. / b[0];
+    s[0] = quot(s[0], b[0], r);
+    a[0] = -quot(a[0], b[0], r);
+    c[0] = quot(c[0], b[0], r);
+  }
+#pragma unroll
+  for (int i = 1; i < M - 1; ++i) {
+    const double ai = a[i], den = __builtin_fma(-ai, c[i - 1], b[i]);
+    const double r = 1. / den;
+    c[i] = quot(c[i], den, r);
+    s[i] = quot(__builtin_fma(-ai, s[i - 1], s[i]), den, r);
+    a[i] = -quot(ai * a[i - 1], den, r);
+  }
+  c[M - 2] = -c[M - 2];
+#pragma unroll
+  for (int i = M - 3; i >= 0; --i) {
+    const double ci = c[i];
+    s[i] = __builtin_fma(-ci, s[i + 1], s[i]);
+    a[i] = __builtin_fma(-ci, a[i + 1], a[i]);
+    c[i] = -ci * c[i + 1];
+  }
+}
+
+// the separator's row A X(p-1) + X(p) + C X(p+1) = D from the part's inner
+// cells and the next part's first cell (S, L, R)
+struct SepRow { double A, C, D; };
+template <int M>
+OT2D_PLAIN SepRow part_separator(const double (&a)[M], const double (&b)[M], const double (&c)[M],
+                                 const double (&s)[M], double Sn, double Ln, double Rn) {
+  const double am = a[M - 1], cm = c[M - 1];
+  const double den = __builtin_fma(am, c[M - 2], __builtin_fma(cm, Ln, b[M - 1]));
+  const double r = 1. / den;
+  SepRow o;
+  o.A = quot(am * a[M - 2], den, r);
+  o.C = quot(cm * Rn, den, r);
+  o.D = quot(__builtin_fma(-am, s[M - 2], __builtin_fma(-cm, Sn, s[M - 1])), den, r);
+  return o;
+}
+
+// one step of the cyclic reduction from the rows at distance d on both sides
+// (zero rows past the ends)
+OT2D_PLAIN SepRow sep_reduce(const SepRow& x, const SepRow& m, const SepRow& p) {
+  const double den = __builtin_fma(-x.C, p.A, __builtin_fma(-x.A, m.C, 1.));
+  const double r = 1. / den;
+  SepRow o;
+  o.A = -quot(x.A * m.A, den, r);
+  o.C = -quot(x.C * p.C, den, r);
+  o.D = quot(__builtin_fma(-x.C, p.D, __builtin_fma(-x.A, m.D, x.D)), den, r);
+  return o;
+}
+
+// x of the part's cells from its separators
+template <int M>
+OT2D_PLAIN void part_expand(const double (&a)[M], const double (&c)[M], double (&s)[M], double XL, double XR) {
+#pragma unroll
+  for (int i = 0; i < M - 1; ++i) s[i] = __builtin_fma(c[i], XR, __builtin_fma(a[i], XL, s[i]));
+  s[M - 1] = XR;
+}
+
 }  // namespace ot2d
