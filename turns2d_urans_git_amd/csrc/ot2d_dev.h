@@ -66,6 +66,7 @@ struct GPtr {
   __device__ __forceinline__ GPtr operator+(I i) const { GPtr r; r.p = p + i; return r; }
 };
 typedef GPtr<double> gd_t;
+typedef GPtr<const double> gcd_t;
 
 struct DevMesh {
   int jd, kd, jmax, kmax;
@@ -80,6 +81,7 @@ struct DevMesh {
   GPtr<double> q[OT2D_MAXQ];  // q(:,:,nsp,n) planes, n = 1..nq  (index n-1)
   GPtr<double> s[OT2D_MAXQ];  // s(:,:,nsp,n) planes
   GPtr<double> x, y, xx, xy, yx, yy, ug, vg, turmu, tscale, bt;
+  GPtr<double> turmu_n;  // SA beside ilu2d: the new eddy viscosity until the update takes it
   GPtr<double> xv, yv, ugv, vgv;  // vertex arrays (jmax,kmax) of this instance
   GPtr<const double> xv0, yv0;  // instance-1 vertices (time-spectral rotation)
   GPtr<double> xold, yold, xole, yole;  // vertices one and two time steps back (moving grids), or null
@@ -374,9 +376,9 @@ inline void mark(Marks* m, int s, hipStream_t st) {
   }
 }
 
+// metrics_only: metfv alone on moved vertices (no cell centres, no
+// free-stream state), as the time loop of a moving grid does
 hipError_t launch_init_geometry(const DevMesh* dM, int nmi, hipStream_t st);
-// metfv alone on moved vertices (no cell centres, no free-stream state), as
-// the time loop of a moving grid does
 hipError_t launch_metrics(const DevMesh* dM, const DevMesh* hM, int nmi, hipStream_t st);
 // pitch (src/motion.f:546-632): the grid turns by this time step's angle
 hipError_t launch_pitch(const DevMesh* dM, const DevMesh* hM, int nmi, hipStream_t st);
@@ -397,6 +399,7 @@ hipError_t launch_norms(const DevMesh* dM, const ResTile* tiles, int ntiles, hip
 hipError_t launch_norms_final(const DevMesh* dM, int nmi, hipStream_t st, int rbc = 0);
 hipError_t launch_conv_check(const DevMesh* dM, const int* inst, const double* tol, int* status, int ncase,
                              hipStream_t st);
+hipError_t launch_zero_s(const DevMesh* dM, const DevMesh* hM, int nmi, hipStream_t st);
 hipError_t launch_rbc(const DevMesh* dM, int nmi, hipStream_t st);
 // threads of a workgroup that runs an instance's turbulence boundary conditions
 int bc_threads(const DevMesh* hM, int nmi);
@@ -412,12 +415,14 @@ struct LaunchCfg {
   int sa_lane = -1;  // SA k solves: columns per workgroup, 0: 16, 1 and -1: 8
 };
 // fuse_update: 1 the q update and monitor in k_lu_finish (Euler), | 2
-// k_lu_finish also leaves the turbulence models' laminar viscosity and
-// velocities (what k_sa_prim computes) from the state it writes
+// k_lu_finish also leaves the SA model's laminar viscosity and velocities
+// (what k_sa_prim computes) from the state it writes
 hipError_t launch_lu(const DevMesh* dM, const DevMesh* hM, int nmi, int fuse_update, int fp32, Marks* mk,
                      hipStream_t st, int sweep = 0);
 hipError_t launch_monitor(const DevMesh* dM, const DevMesh* hM, int nmi, hipStream_t st);
-hipError_t launch_update_monitor(const DevMesh* dM, const DevMesh* hM, int nmi, hipStream_t st);
+hipError_t launch_update_monitor(const DevMesh* dM, const DevMesh* hM, int nmi, hipStream_t st, int take_turmu = 0);
+// k_lu_finish alone (launch_lu with fuse_update | 4 leaves it out)
+hipError_t launch_lu_finish(const DevMesh* dM, const DevMesh* hM, int nmi, int flags, int fp32, hipStream_t st);
 hipError_t launch_forces(const DevMesh* dM, int mi, double* out, hipStream_t st);
 hipError_t launch_tsrhs(const DevMesh* dM, const DevMesh* hM, int nmi, hipStream_t st);
 // bytes of one instance's LU-SGS workspace (rl: ceil(rows / 64) of the case's
@@ -426,8 +431,11 @@ size_t lu_workspace_bytes(int jd, int kd, int rl);
 hipError_t launch_visrhs(const DevMesh* dM, const DevMesh* hM, int nmi, hipStream_t st, int norms = 0);
 // prim_done: the laminar viscosity and velocities are already in place
 // (k_lu_finish with flag 2)
+// ovl: the SA model runs beside ilu2d (another stream, before k_lu_finish):
+// it takes q1-q4 through ilu2d's primitive round trip itself and leaves the
+// eddy viscosity in turmu_n, which k_update_monitor copies
 hipError_t launch_sa(const DevMesh* dM, const DevMesh* hM, int nmi, Marks* mk, hipStream_t st, int sa_lane = -1,
-                     int prim_done = 0);
+                     int prim_done = 0, int ovl = 0);
 hipError_t launch_sa_dist(const DevMesh* dM, const DevMesh* hM, int nmi, hipStream_t st);
 hipError_t launch_sa_prim(const DevMesh* dM, const DevMesh* hM, int nmi, hipStream_t st);
 hipError_t launch_sst(const DevMesh* dM, const DevMesh* hM, int nmi, Marks* mk, hipStream_t st, int prim_done = 0);
@@ -437,8 +445,6 @@ hipError_t launch_interp(const DevMesh* dM, const void* don, int ndon, const voi
                          hipStream_t st);
 size_t interp_donor_bytes();
 size_t interp_fringe_bytes();
-// longest j line (interior cells) a case may have: what the sweeps' staging
-// in LDS once allowed, kept as the library's limit (the sweeps stage nothing
-// by line length; at 512 rows their records end well inside 32-bit offsets)
+// longest j line (interior cells) a case may have
 int lu_max_ni(int fp32);
 }  // namespace ot2d

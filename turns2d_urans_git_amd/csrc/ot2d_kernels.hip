@@ -47,6 +47,7 @@ __device__ inline double swept_tj(const DevMesh& M, long long p, long long m, do
   return tj;
 }
 __device__ __forceinline__ int imax(int a, int b) { return a > b ? a : b; }
+__device__ __forceinline__ int imin(int a, int b) { return a < b ? a : b; }
 
 // =================================================================== time_step
 // src/time.f:2-107 (one value per cell, all cells incl. halo)
@@ -1010,6 +1011,13 @@ __global__ __launch_bounds__(BC_THREADS) void k_rbc(const DevMesh* __restrict__ 
 // Per-cell quantities ilu2d derives from the primitive state
 // (src/lhs.f:524-564): u, v, uv2, ge, contravariant velocities, spectral
 // radii, viscous term and the diagonal d.
+template <typename T>
+struct LUCoef {
+  T uu, vv, uv2, ge;   // primitive velocity, kinetic energy, gamma*e - gm1*uv2
+  T ri1, ri2, qq;      // metric pair and contravariant velocity of the direction
+  T chk, spec;         // upwind switch and spectral term of the direction/sweep
+};
+
 struct LUCellF64 {
   double uu, vv, uv2, ge, qx, qy, cx, cy, vn, d, qqx_s, qqy_s;
 };
@@ -1039,7 +1047,20 @@ __device__ __forceinline__ LUCellF64 lu_cell(const DevConst& C, double q1, doubl
   return o;
 }
 
-struct LUNb {           // a cell's operator for the neighbour of one direction
+// A(+/-) or B(+/-) operator of a neighbour applied to its s (src/lhs.f:633-651)
+__device__ __forceinline__ void lu_apply(const double gm1, double chk, double spec, double ri1, double ri2,
+                                         double qq, double uu, double vv, double uv2, double ge, const double* s,
+                                         double* a) {
+  double a4 = chk * (ri1 * s[1] + ri2 * s[2] - qq * s[0]);
+  double a2 = chk * gm1 * (uv2 * s[0] - (uu * s[1] + vv * s[2]) + s[3]);
+  a[0] = a4 + spec * s[0];
+  a[1] = ri1 * a2 + uu * a4 + spec * s[1];
+  a[2] = ri2 * a2 + vv * a4 + spec * s[2];
+  a[3] = qq * a2 + ge * a4 + spec * s[3];
+}
+
+struct LUNb {           // what a consumer needs of a neighbour cell
+  double s[4];
   double ri1, ri2, qq, uu, vv, uv2, ge, chk, spec;
 };
 
@@ -1142,6 +1163,7 @@ struct LUGeom {
                                    // TA >= TW step rows of the record arrays (a multiple of 8)
   int TD;                          // FP64 sweep: step rows of a block's arrays
   long long off_dh, off_dh2, off_hrf, off_hrb, off_dtk;  // FP64 arrays (16-byte vectors; records at 0)
+  long long ncell;                 // FP32: interior cells
   long long off_f32, off_b32, off_cb, off_h, off_h2;   // FP32 arrays
   long long off_tk;                // FP32 workgroup tickets (forward, backward): one vector
 };
@@ -1166,6 +1188,7 @@ __host__ __device__ inline LUGeom lu_geom(int ni, int nk) {
   // bytes per lane, each value beside the sweep's tag: 64 units each; the
   // edge rows' results are also the inter-workgroup mail); then the two
   // ticket counters
+  g.ncell = (long long)ni * nk;
   g.off_f32 = 0;
   g.off_b32 = g.off_f32 + 288ll * g.W * g.TA;
   g.off_cb = g.off_b32 + 256ll * g.W * g.TA;
@@ -2295,7 +2318,7 @@ __device__ __forceinline__ bool asq_bad(const DevConst& C, double q1, double q2,
 }
 
 template <typename T>
-// flags: 1 the q update and monitor follow here (Euler); 2 the turbulence models'
+// flags: 1 the q update and monitor follow here (Euler); 2 the SA model's
 // laminar viscosity and velocities of every cell follow from the state
 // written here (k_sa_prim's values)
 __global__ __launch_bounds__(256) void k_lu_finish(const DevMesh* __restrict__ Ms, int flags) {
@@ -2354,7 +2377,9 @@ __global__ __launch_bounds__(256) void k_lu_finish(const DevMesh* __restrict__ M
 // one pass: interior cells are updated, then every cell (halo included) is
 // checked; each cell's update reads only that cell, so this is the update
 // followed by the monitor
-__global__ __launch_bounds__(256) void k_update_monitor(const DevMesh* __restrict__ Ms) {
+// take_turmu: the eddy viscosity the SA model left in turmu_n (it ran beside
+// ilu2d) becomes turmu
+__global__ __launch_bounds__(256) void k_update_monitor(const DevMesh* __restrict__ Ms, int take_turmu) {
   const DevMesh& M = Ms[blockIdx.y];
   if (*M.status) return;
   const int jd = M.jd;
@@ -2368,6 +2393,7 @@ __global__ __launch_bounds__(256) void k_update_monitor(const DevMesh* __restric
       q1 = q1 + M.s[0][i] * ibp; q2 = q2 + M.s[1][i] * ibp; q3 = q3 + M.s[2][i] * ibp; q4 = q4 + M.s[3][i] * ibp;
       M.q[0][i] = q1; M.q[1][i] = q2; M.q[2][i] = q3; M.q[3][i] = q4;
     }
+    if (take_turmu) M.turmu[i] = M.turmu_n[i];
     bad |= asq_bad(M.c, q1, q2, q3, q4);
   }
   if (bad) atomicCAS(M.status, 0, 1);
@@ -2941,6 +2967,7 @@ static hipError_t launch_lu64(const DevMesh* dM, const DevMesh* hM, int nmi, int
   hipLaunchKernelGGL((k_lu_sweep64<-1, S, NP, PD>), dim3(wmax, nmi), dim3(64 * (2 + NP)), lds, st, dM);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_LU_BACKWARD, st);
+  if (fuse_update & 4) return hipSuccess;
   hipLaunchKernelGGL(k_lu_finish<double>, dim3(nblk(mx, 256), nmi), dim3(256), 0, st, dM, fuse_update);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_LU_FINISH, st);
@@ -3015,10 +3042,19 @@ static hipError_t launch_lu32(const DevMesh* dM, const DevMesh* hM, int nmi, int
     default: return hipErrorInvalidValue;
   }
   if (e != hipSuccess) return e;
+  if (fuse_update & 4) return hipSuccess;
   hipLaunchKernelGGL(k_lu_finish<float>, dim3(nblk(mx, 256), nmi), dim3(256), 0, st, dM, fuse_update);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_LU_FINISH, st);
   return hipSuccess;
+}
+
+hipError_t launch_lu_finish(const DevMesh* dM, const DevMesh* hM, int nmi, int flags, int fp32, hipStream_t st) {
+  long long mx = 0;
+  for (int i = 0; i < nmi; ++i) mx = hM[i].jd * (long long)hM[i].kd > mx ? hM[i].jd * (long long)hM[i].kd : mx;
+  if (fp32) hipLaunchKernelGGL(k_lu_finish<float>, dim3(nblk(mx, 256), nmi), dim3(256), 0, st, dM, flags);
+  else hipLaunchKernelGGL(k_lu_finish<double>, dim3(nblk(mx, 256), nmi), dim3(256), 0, st, dM, flags);
+  return hipGetLastError();
 }
 
 hipError_t launch_lu(const DevMesh* dM, const DevMesh* hM, int nmi, int fuse_update, int fp32, Marks* mk,
@@ -3033,10 +3069,10 @@ size_t lu_workspace_bytes(int jd, int kd, int rl) {
   return 16 * (size_t)lu_total(jd - 2, kd - 2, rl);
 }
 
-hipError_t launch_update_monitor(const DevMesh* dM, const DevMesh* hM, int nmi, hipStream_t st) {
+hipError_t launch_update_monitor(const DevMesh* dM, const DevMesh* hM, int nmi, hipStream_t st, int take_turmu) {
   long long mx = 0;
   for (int i = 0; i < nmi; ++i) mx = hM[i].jd * (long long)hM[i].kd > mx ? hM[i].jd * (long long)hM[i].kd : mx;
-  hipLaunchKernelGGL(k_update_monitor, dim3(nblk(mx, 256), nmi), dim3(256), 0, st, dM);
+  hipLaunchKernelGGL(k_update_monitor, dim3(nblk(mx, 256), nmi), dim3(256), 0, st, dM, take_turmu);
   return hipGetLastError();
 }
 hipError_t launch_monitor(const DevMesh* dM, const DevMesh* hM, int nmi, hipStream_t st) {

@@ -393,12 +393,16 @@ __device__ __forceinline__ double ip6(double x) { return ((((x * x) * x) * x) * 
 
 // laminar viscosity (lamvis, src/samodel2d.f:200-238) and the velocities
 // vmu_sa keeps (src/samodel2d.f:61-72), all cells
-__global__ __launch_bounds__(256) void k_sa_prim(const DevMesh* __restrict__ Ms) {
+// ovl: the state as ilu2d's primitive round trip leaves it
+__global__ __launch_bounds__(256) void k_sa_prim(const DevMesh* __restrict__ Ms, int ovl) {
   const DevMesh& M = Ms[blockIdx.y];
   if (*M.status) return;
   long long n2 = (long long)M.jd * M.kd;
-  for (long long i = blockIdx.x * 256ll + threadIdx.x; i < n2; i += 256ll * gridDim.x)
-    sa_prim_cell(M, i, M.q[0][i], M.q[1][i], M.q[2][i], M.q[3][i]);
+  for (long long i = blockIdx.x * 256ll + threadIdx.x; i < n2; i += 256ll * gridDim.x) {
+    double q1 = M.q[0][i], q2 = M.q[1][i], q3 = M.q[2][i], q4 = M.q[3][i];
+    if (ovl) q_roundtrip(q1, q2, q3, q4, M.q[M.nq - 1][i]);
+    sa_prim_cell(M, i, q1, q2, q3, q4);
+  }
 }
 
 __device__ __forceinline__ int sa_periodic_src(int idir, int js, int je, int ks, int ke, int jd, int kd, int jk) {
@@ -418,8 +422,17 @@ __device__ __forceinline__ double c_turm_val(double q1, double qn, double vmul, 
   double fv1 = ip3(chi) / (ip3(chi) + ip3(SA_cv1));
   return q1 * qn * q5 * fv1;
 }
-__device__ __forceinline__ void c_turm_cell(const DevMesh& M, long long i) {
-  M.turmu[i] = c_turm_val(M.q[0][i], M.q[M.nq - 1][i], M.sa_vmul[i], M.q[4][i]);
+// the eddy viscosity of cell i; with ovl the SA model runs beside ilu2d, so
+// q1 is taken through ilu2d's round trip, (q1 qj) / qj, and the value goes
+// to turmu_n
+__device__ __forceinline__ void put_turm(const DevMesh& M, long long i, double q1, double qj, double vmul, double q5,
+                                         int ovl) {
+  if (ovl) M.turmu_n[i] = c_turm_val((q1 * qj) / qj, qj, vmul, q5);
+  else M.turmu[i] = c_turm_val(q1, qj, vmul, q5);
+}
+
+__device__ __forceinline__ void c_turm_cell(const DevMesh& M, long long i, int ovl) {
+  put_turm(M, i, M.q[0][i], M.q[M.nq - 1][i], M.sa_vmul[i], M.q[4][i], ovl);
 }
 
 // turbc (src/samodel2d.f:827-1303) for one boundary segment
@@ -512,7 +525,7 @@ __device__ void turbc_segment(const DevMesh& M, const DevBC& b, int t, int nt) {
 // turbc of an instance by one workgroup (the segments of a phase side by
 // side).  With eddy set (the final turbc) the eddy viscosity of the halo ring
 // follows (c_turm)
-__global__ __launch_bounds__(BC_MAX_THREADS) void k_turbc(const DevMesh* __restrict__ Ms, int eddy) {
+__global__ __launch_bounds__(BC_MAX_THREADS) void k_turbc(const DevMesh* __restrict__ Ms, int eddy, int ovl) {
   const DevMesh& M = Ms[blockIdx.x];
   if (*M.status) return;
   for_phases(M, [&](const DevBC& b, int t, int nt) { turbc_segment(M, b, t, nt); });
@@ -525,7 +538,7 @@ __global__ __launch_bounds__(BC_MAX_THREADS) void k_turbc(const DevMesh* __restr
     else if (w < 2 * jd) { j = w - jd + 1; k = kd; }
     else if (w < 2 * jd + kd - 2) { j = 1; k = w - 2 * jd + 2; }
     else { j = jd; k = w - 2 * jd - (kd - 2) + 2; }
-    c_turm_cell(M, cell(M, j, k));
+    c_turm_cell(M, cell(M, j, k), ovl);
   }
 }
 
@@ -748,7 +761,7 @@ __global__ __launch_bounds__(64) void k_sa_solve_j(const DevMesh* __restrict__ M
 // 8.9, 4: 7.6; two lanes per column from both ends 17.4).
 constexpr int SAK_NT = 512;
 template <int TC>
-__global__ __launch_bounds__(SAK_NT) void k_sa_solve_k(const DevMesh* __restrict__ Ms) {
+__global__ __launch_bounds__(SAK_NT) void k_sa_solve_k(const DevMesh* __restrict__ Ms, int ovl) {
   extern __shared__ __attribute__((aligned(16))) double sak_ex[];
   constexpr int PM = PCOL_M;
   const DevMesh& M = Ms[blockIdx.y];
@@ -792,7 +805,7 @@ __global__ __launch_bounds__(SAK_NT) void k_sa_solve_k(const DevMesh* __restrict
     const double dq = relfac * (0. + s[u]);
     const double v = fmax((q5[u] + dq * (double)imx(ib[u], 0)), vnulim);
     M.q[4][i] = v;
-    M.turmu[i] = c_turm_val(q1[u], qj[u], vm[u], v);
+    put_turm(M, i, q1[u], qj[u], vm[u], v, ovl);
   }
 }
 
@@ -885,13 +898,13 @@ hipError_t launch_sa_dist(const DevMesh* dM, const DevMesh* hM, int nmi, hipStre
 }
 
 hipError_t launch_sa_prim(const DevMesh* dM, const DevMesh* hM, int nmi, hipStream_t st) {
-  hipLaunchKernelGGL(k_sa_prim, dim3(nblk2(max_cells(hM, nmi), 256), nmi), dim3(256), 0, st, dM);
+  hipLaunchKernelGGL(k_sa_prim, dim3(nblk2(max_cells(hM, nmi), 256), nmi), dim3(256), 0, st, dM, 0);
   return hipGetLastError();
 }
 
 // vmu_sa for every instance (src/samodel2d.f:2-197, itrans = 0)
 hipError_t launch_sa(const DevMesh* dM, const DevMesh* hM, int nmi, Marks* mk, hipStream_t st, int sa_lane,
-                     int prim_done) {
+                     int prim_done, int ovl) {
   long long mx = max_cells(hM, nmi);
   int mj = 1, mk_ = 1;
   for (int i = 0; i < nmi; ++i) {
@@ -900,12 +913,12 @@ hipError_t launch_sa(const DevMesh* dM, const DevMesh* hM, int nmi, Marks* mk, h
   }
   hipError_t e = hipSuccess;
   if (!prim_done) {
-    hipLaunchKernelGGL(k_sa_prim, dim3(nblk2(mx, 256), nmi), dim3(256), 0, st, dM);
+    hipLaunchKernelGGL(k_sa_prim, dim3(nblk2(mx, 256), nmi), dim3(256), 0, st, dM, ovl);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
   mark(mk, OT2D_ST_SA_PRIM, st);
   const int nbc = bc_threads(hM, nmi);
-  hipLaunchKernelGGL(k_turbc, dim3(nmi), dim3(nbc), 0, st, dM, 0);
+  hipLaunchKernelGGL(k_turbc, dim3(nmi), dim3(nbc), 0, st, dM, 0, ovl);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_SA_BC, st);
   hipLaunchKernelGGL(k_sa_rhs, dim3(vis_tiles(hM, nmi), nmi), dim3(VIS_THREADS), 0, st, dM);
@@ -920,13 +933,13 @@ hipError_t launch_sa(const DevMesh* dM, const DevMesh* hM, int nmi, Marks* mk, h
   const bool wide = np * 16 <= SAK_NT && sa_lane == 0;
   auto solve_k = [&](auto kern, int tc) {
     const int nt = (np * tc + 63) / 64 * 64;
-    hipLaunchKernelGGL(kern, dim3((mj + tc - 1) / tc, nmi), dim3(nt), sizeof(double) * 6 * nt, st, dM);
+    hipLaunchKernelGGL(kern, dim3((mj + tc - 1) / tc, nmi), dim3(nt), sizeof(double) * 6 * nt, st, dM, ovl);
   };
   if (wide) solve_k(k_sa_solve_k<16>, 16);
   else solve_k(k_sa_solve_k<8>, 8);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_SA_SOLVE_K, st);
-  hipLaunchKernelGGL(k_turbc, dim3(nmi), dim3(nbc), 0, st, dM, 1);
+  hipLaunchKernelGGL(k_turbc, dim3(nmi), dim3(nbc), 0, st, dM, 1, ovl);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark(mk, OT2D_ST_SA_EDDY, st);
   return hipSuccess;
