@@ -189,11 +189,11 @@ class SweepOrder {
   hipError_t e_ = hipSuccess;
 };
 
-// some sweep of the case runs in several workgroups, or in FP32
+// the sweep of a mesh of kmax rows of vertices runs in several workgroups, or in FP32
+bool block_coupled(const ot2d_params* p, int kmax) { return p->lu_fp32 || kmax - 1 > LU_R; }
 bool block_coupled(const ot2d_case* c) {
-  if (c->p.lu_fp32) return true;
   for (const auto& mb : c->m)
-    if (mb.kmax - 1 > LU_R) return true;
+    if (block_coupled(&c->p, mb.kmax)) return true;
   return false;
 }
 }  // namespace
@@ -219,7 +219,7 @@ extern "C" int32_t ot2d_set_fp32_order(int32_t on) {
   return OT2D_OK;
 }
 
-// the device's ordering event, created with the first case on it
+// the device's ordering event, created with the first such case on it
 static int32_t sweep_chain_init(int dev) {
   if (dev < 0 || dev >= kMaxDevices) return fail(OT2D_ERR_ARG, "device %d out of range", dev);
   std::lock_guard<std::mutex> lock(g_sweeps.mu);
@@ -642,7 +642,9 @@ static int32_t create_impl(const ot2d_params* ps, int32_t ncase, int32_t nmesh, 
   (void)hipGetDevice(&c->device);
   hipError_t e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
   if (e != hipSuccess) { free_case(c); return fail(OT2D_ERR_HIP, "stream: %s", hipGetErrorString(e)); }
-  if (int32_t rc = sweep_chain_init(c->device)) { free_case(c); return rc; }
+  for (int im = 0; im < nmesh; ++im)
+    if (block_coupled(p, md[im].kmax))
+      if (int32_t rc = sweep_chain_init(c->device)) { free_case(c); return rc; }
   if (kSaBesideLu && !c->lamin && c->iturb == 1) {
     if ((e = hipStreamCreateWithFlags(&c->st2, hipStreamNonBlocking)) != hipSuccess ||
         (e = hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming)) != hipSuccess ||
@@ -1789,6 +1791,8 @@ extern "C" int32_t ot2d_batch_admit(ot2d_case* c, int32_t icase, const ot2d_para
   for (int ib = 0; ib < md->nbc; ++ib)
     if (!bc_in_range(fix_bc(md->bc[ib], jmax, kmax, jd, kd), jd, kd))
       return fail(OT2D_ERR_ARG, "boundary segment %d indexes outside the grid", ib + 1);
+  if (block_coupled(p, kmax))
+    if (int32_t rc = sweep_chain_init(c->device)) return rc;
   // the slot's memory as a new case finds it: zero (the FP32 sweeps' zero
   // records off the grid included)
   const size_t cap2 = mb.cap_n2 * ns, capv = mb.cap_nv2 * ns;
