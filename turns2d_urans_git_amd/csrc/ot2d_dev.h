@@ -66,7 +66,6 @@ struct GPtr {
   __device__ __forceinline__ GPtr operator+(I i) const { GPtr r; r.p = p + i; return r; }
 };
 typedef GPtr<double> gd_t;
-typedef GPtr<const double> gcd_t;
 
 struct DevMesh {
   int jd, kd, jmax, kmax;
@@ -376,9 +375,9 @@ inline void mark(Marks* m, int s, hipStream_t st) {
   }
 }
 
-// metrics_only: metfv alone on moved vertices (no cell centres, no
-// free-stream state), as the time loop of a moving grid does
 hipError_t launch_init_geometry(const DevMesh* dM, int nmi, hipStream_t st);
+// metfv alone on moved vertices (no cell centres, no free-stream state), as
+// the time loop of a moving grid does
 hipError_t launch_metrics(const DevMesh* dM, const DevMesh* hM, int nmi, hipStream_t st);
 // pitch (src/motion.f:546-632): the grid turns by this time step's angle
 hipError_t launch_pitch(const DevMesh* dM, const DevMesh* hM, int nmi, hipStream_t st);
@@ -399,7 +398,6 @@ hipError_t launch_norms(const DevMesh* dM, const ResTile* tiles, int ntiles, hip
 hipError_t launch_norms_final(const DevMesh* dM, int nmi, hipStream_t st, int rbc = 0);
 hipError_t launch_conv_check(const DevMesh* dM, const int* inst, const double* tol, int* status, int ncase,
                              hipStream_t st);
-hipError_t launch_zero_s(const DevMesh* dM, const DevMesh* hM, int nmi, hipStream_t st);
 hipError_t launch_rbc(const DevMesh* dM, int nmi, hipStream_t st);
 // threads of a workgroup that runs an instance's turbulence boundary conditions
 int bc_threads(const DevMesh* hM, int nmi);
@@ -415,8 +413,8 @@ struct LaunchCfg {
   int sa_lane = -1;  // SA k solves: columns per workgroup, 0: 16, 1 and -1: 8
 };
 // fuse_update: 1 the q update and monitor in k_lu_finish (Euler), | 2
-// k_lu_finish also leaves the SA model's laminar viscosity and velocities
-// (what k_sa_prim computes) from the state it writes
+// k_lu_finish also leaves the turbulence models' laminar viscosity and
+// velocities (what k_sa_prim computes) from the state it writes
 hipError_t launch_lu(const DevMesh* dM, const DevMesh* hM, int nmi, int fuse_update, int fp32, Marks* mk,
                      hipStream_t st, int sweep = 0);
 hipError_t launch_monitor(const DevMesh* dM, const DevMesh* hM, int nmi, hipStream_t st);
@@ -445,6 +443,8 @@ hipError_t launch_interp(const DevMesh* dM, const void* don, int ndon, const voi
                          hipStream_t st);
 size_t interp_donor_bytes();
 size_t interp_fringe_bytes();
-// longest j line (interior cells) a case may have
+// longest j line (interior cells) a case may have: what the sweeps' staging
+// in LDS once allowed, kept as the library's limit (the sweeps stage nothing
+// by line length; at 512 rows their records end well inside 32-bit offsets)
 int lu_max_ni(int fp32);
 }  // namespace ot2d

@@ -47,7 +47,6 @@ __device__ inline double swept_tj(const DevMesh& M, long long p, long long m, do
   return tj;
 }
 __device__ __forceinline__ int imax(int a, int b) { return a > b ? a : b; }
-__device__ __forceinline__ int imin(int a, int b) { return a < b ? a : b; }
 
 // =================================================================== time_step
 // src/time.f:2-107 (one value per cell, all cells incl. halo)
@@ -1011,13 +1010,6 @@ __global__ __launch_bounds__(BC_THREADS) void k_rbc(const DevMesh* __restrict__ 
 // Per-cell quantities ilu2d derives from the primitive state
 // (src/lhs.f:524-564): u, v, uv2, ge, contravariant velocities, spectral
 // radii, viscous term and the diagonal d.
-template <typename T>
-struct LUCoef {
-  T uu, vv, uv2, ge;   // primitive velocity, kinetic energy, gamma*e - gm1*uv2
-  T ri1, ri2, qq;      // metric pair and contravariant velocity of the direction
-  T chk, spec;         // upwind switch and spectral term of the direction/sweep
-};
-
 struct LUCellF64 {
   double uu, vv, uv2, ge, qx, qy, cx, cy, vn, d, qqx_s, qqy_s;
 };
@@ -1047,20 +1039,7 @@ __device__ __forceinline__ LUCellF64 lu_cell(const DevConst& C, double q1, doubl
   return o;
 }
 
-// A(+/-) or B(+/-) operator of a neighbour applied to its s (src/lhs.f:633-651)
-__device__ __forceinline__ void lu_apply(const double gm1, double chk, double spec, double ri1, double ri2,
-                                         double qq, double uu, double vv, double uv2, double ge, const double* s,
-                                         double* a) {
-  double a4 = chk * (ri1 * s[1] + ri2 * s[2] - qq * s[0]);
-  double a2 = chk * gm1 * (uv2 * s[0] - (uu * s[1] + vv * s[2]) + s[3]);
-  a[0] = a4 + spec * s[0];
-  a[1] = ri1 * a2 + uu * a4 + spec * s[1];
-  a[2] = ri2 * a2 + vv * a4 + spec * s[2];
-  a[3] = qq * a2 + ge * a4 + spec * s[3];
-}
-
-struct LUNb {           // what a consumer needs of a neighbour cell
-  double s[4];
+struct LUNb {           // a cell's operator for the neighbour of one direction
   double ri1, ri2, qq, uu, vv, uv2, ge, chk, spec;
 };
 
@@ -1163,7 +1142,6 @@ struct LUGeom {
                                    // TA >= TW step rows of the record arrays (a multiple of 8)
   int TD;                          // FP64 sweep: step rows of a block's arrays
   long long off_dh, off_dh2, off_hrf, off_hrb, off_dtk;  // FP64 arrays (16-byte vectors; records at 0)
-  long long ncell;                 // FP32: interior cells
   long long off_f32, off_b32, off_cb, off_h, off_h2;   // FP32 arrays
   long long off_tk;                // FP32 workgroup tickets (forward, backward): one vector
 };
@@ -1188,7 +1166,6 @@ __host__ __device__ inline LUGeom lu_geom(int ni, int nk) {
   // bytes per lane, each value beside the sweep's tag: 64 units each; the
   // edge rows' results are also the inter-workgroup mail); then the two
   // ticket counters
-  g.ncell = (long long)ni * nk;
   g.off_f32 = 0;
   g.off_b32 = g.off_f32 + 288ll * g.W * g.TA;
   g.off_cb = g.off_b32 + 256ll * g.W * g.TA;
@@ -1408,7 +1385,7 @@ __device__ __forceinline__ void nb_matrix(const LUNb& n, double gm1, double m[16
 // (row r, step t) at (r + 1) * LP_C + t + 1, its j neighbours one step, its k
 // neighbours a row and a step away.  Each cell then assembles its operators
 // from itself and its four neighbours there.
-// Bound by memory: 304 bytes written a cell, 112 read, the ring's again.  The
+// Bound by memory: 288 bytes written a cell, 112 read, the ring's again.  The
 // skewed ring is 340 cells for 256 where the bounding box of the parallelogram
 // was 410, and its 51 KiB (was 67) leave room for three workgroups a CU: 60
 // cases (3.9 M cells) 408 -> 360 us, 20 of them 136 -> 121, 513x129 11.1 -> 10.3 (with xcd_tile).
@@ -2318,7 +2295,7 @@ __device__ __forceinline__ bool asq_bad(const DevConst& C, double q1, double q2,
 }
 
 template <typename T>
-// flags: 1 the q update and monitor follow here (Euler); 2 the SA model's
+// flags: 1 the q update and monitor follow here (Euler); 2 the turbulence models'
 // laminar viscosity and velocities of every cell follow from the state
 // written here (k_sa_prim's values)
 __global__ __launch_bounds__(256) void k_lu_finish(const DevMesh* __restrict__ Ms, int flags) {
