@@ -224,9 +224,9 @@ int32_t ot2d_batch_admit(ot2d_case* c, int32_t icase, const ot2d_params* p, cons
 /* ------------------------------------------------------------ launch choices
  * Launch shapes that change speed but not results: sweep (0, 1 or 2) picks
  * the FP32 LU-SGS sweep's LDS ring depth and producer count (15 slots and
- * 3 producer waves, 18 and 3, 12 and 4); sa_lane picks how
- * many adjacent columns a workgroup of the SA k solve takes (-1 and 1: 8, 0:
- * 16 where columns hold up to 256 cells).
+ * 3 producer waves, 18 and 3, 12 and 4); sa_lane picks how many adjacent
+ * columns a workgroup of the SA k solve takes (-1 and 1: 8, 0: 16 where
+ * columns hold up to 256 cells).
  * Every choice gives bit-identical states.  No counterpart in the reference,
  * whose loops have one shape. */
 int32_t ot2d_set_launch(ot2d_case* c, int32_t sweep, int32_t sa_lane);
@@ -236,10 +236,12 @@ int32_t ot2d_get_launch(ot2d_case* c, int32_t* sweep, int32_t* sa_lane);
  * each candidate times `steps` captured steps from the case's current state
  * (HIP events on the case's stream, best of three interleaved rounds), the
  * state (q, eddy viscosity, step counters, status) is put back after each,
- * and the fastest is set on the case.  Results are cached per class in
+ * and the default stays set on the case unless another wins by more than 1 %
+ * and by more than the rounds of both differ.  Results are cached per class in
  * the process and, when OT2D_TUNE_CACHE names a file, in that file (one line
- * per class, read at the first call, appended after each search); a cached
- * class is set without measuring.  Either way the chosen step is captured
+ * per class, read at the first call, appended after each search; lines of a
+ * library with another set of choices are passed over); a cached class is set
+ * without measuring.  Either way the chosen step is captured
  * before the call returns, so the next ot2d_iterate starts at once.
  * *measured (may be NULL) is 1 when a search ran, 0 on a cache hit.
  * Allocates a copy of the state while it runs. */

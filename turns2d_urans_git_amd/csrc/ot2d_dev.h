@@ -241,7 +241,8 @@ __device__ __forceinline__ void part_columns(double (&a)[PCOL_M], const double (
 // Tile of this workgroup among the n of its record, or -1: xcd_deal.  Against
 // tiles in dispatch order: 385x97 with 401x401, FP32 operators 27.7 -> 23.6
 // us, viscous terms 23.5 -> 21.5; 60 cases: viscous terms 231 -> 223, residual
-// 260 -> 254, SA right-hand side 189 -> 182.
+// 260 -> 254, SA right-hand side 189 -> 182 (with launches filled up to a
+// multiple of 8 a record; without, 21.9 and 18.9, 218, 254 and 176).
 __device__ __forceinline__ int xcd_tile(int n) { return xcd_deal((int)blockIdx.x, n); }
 
 constexpr int RES_TJ = 32;

@@ -717,7 +717,7 @@ __device__ __forceinline__ void face_states_weno(const double* sf0, int stv, int
 // ceil(552 / NT) passes: one (NT = 576) where few tiles leave a CU one
 // workgroup and the passes' latency counts, three (NT = 256) where tiles fill
 // the chip and idle lanes of the last pass cost issue slots.  513x129 (256
-// tiles): 10 us (576), 13 (256), 15.5 with a pass or two per direction before;
+// tiles): 9.5 us (576), 13 (256), 15.5 with a pass or two per direction before;
 // 385x97 with 401x401, WENO5 (1206 tiles): 38 / 41 / 47; 60 cases (15200
 // tiles): 333 (576), 270 (256; 254 with xcd_tile), 301 before.  FP64 issue binds the last
 // (800 operations a face).
@@ -1929,8 +1929,8 @@ __global__ __launch_bounds__(64 * (2 + NP)) void k_lu_sweep32(const DevMesh* __r
 // and its record) or from the halo-row records, 16 columns at a time.
 //
 // Bound by the dependent chain of ni + nk steps, each about 95 instructions
-// of one wave (215 ns).  Forward / backward: 141 / 147 us at 513x129, 70 / 73
-// at 257x65, 196 / 204 for 385x97 beside 401x401, 14 / 14 at 33x17.  The
+// of one wave (205 ns).  Forward / backward: 143 / 145 us at 513x129, 72 / 73
+// at 257x65, 201 / 201 for 385x97 beside 401x401, 14 / 14 at 33x17.  The
 // sweep it replaced ran one wave per instance with ceil(nk/64) rows per
 // lane, applying both terms on every lane: 569 / 565, 203 / 202, 1740 / 1583
 // and 32 / 31 us, so no size is left to it.
@@ -2912,7 +2912,7 @@ hipError_t launch_rbc(const DevMesh* dM, int nmi, hipStream_t st) {
 
 // every FP64 case: the ring's 12 slots (62 KB) leave room for two workgroups
 // on a CU, and three producers of five steps in flight cover the records'
-// latency at 215 ns a step
+// latency at 205 ns a step
 static hipError_t launch_lu64(const DevMesh* dM, const DevMesh* hM, int nmi, int fuse_update, Marks* mk,
                               hipStream_t st) {
   constexpr int S = 12, NP = 3, PD = 5;
@@ -2964,7 +2964,10 @@ static hipError_t launch_lu64(const DevMesh* dM, const DevMesh* hM, int nmi, int
 // more than half a CU's, so that a CU takes one workgroup at a time.  Two that
 // share a CU while others stand idle are the last to end: 50 cases (211
 // blocks) 494 us with two of S = 15 to a CU, 409 with one; 60 cases 530 and
-// 487; 120 cases (513 blocks, two rounds of them) 871 and 832.
+// 487; 120 cases (513 blocks, two rounds of them) 871 and 832.  The same where
+// cohorts overlap (the order lifted, us for a step of all): 4 of 7 cases 623
+// with two to a CU and 610 with one, 8 of 7 1065 and 1032, 4 of 24 2743 and
+// 2684; and for 1000 cases of 33x17, 436 and 439.
 constexpr size_t lu32_lds(int S) {
   const size_t ring = (size_t)S * LU32_NV * 1024 + 16 * ((S * 8 + 15) / 16), half = 80 * 1024 + 16;
   return ring > half ? ring : half;

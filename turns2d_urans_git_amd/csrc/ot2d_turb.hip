@@ -9,8 +9,9 @@
 //                                                    instance); the final ones with the
 //                                                    eddy viscosity of the halo ring
 //                                      k_sa_rhs      convection, diffusion, source and the
-//                                                    two scalar tridiagonal systems, in
-//                                                    gather form (one thread per cell)
+//                                                    two scalar tridiagonal systems: what
+//                                                    the stencil reads once per cell of a
+//                                                    32x8 tile in LDS, then each cell's row
 //                                      k_sa_solve_j  tridiagonal solve along j, one wave per row
 //                                      k_sa_solve_k  tridiagonal solve along k, 8 or 16 adjacent
 //                                                    j columns per workgroup, nu-tilde update and
@@ -235,9 +236,9 @@ __device__ __forceinline__ Tri lds_tri(const double (&g)[3][N], int c) {
 }
 
 // Bound by latency at the 12 waves a CU its LDS (41 KB) and registers (168)
-// allow; FP64 issue alone is 97 us of the 60-case batch's 223 us (286 us with
-// each array in memory of its own, 77 KB and 8 waves a CU); 513x129: 9.7 us
-// both ways.
+// allow; FP64 issue alone is 97 us of the 60-case batch's 218 us (286 us with
+// each array in memory of its own, 77 KB and 8 waves a CU); 513x129: 9.4 us
+// (9.7 both ways when that was changed).
 // With norms set, the residual is complete once this kernel has added the
 // viscous terms, so each tile also takes its residual-norm partials here
 // (the tiles and thread-to-cell map are the residual's: 32x8 tiles, k-tile
@@ -562,9 +563,9 @@ __device__ __forceinline__ void sa_half(double va, double na, double vb, double 
 // what the stencil reads of a cell (nu-tilde, vnul, contravariant velocities,
 // velocities, metrics) is formed once for the tile and its one-cell ring in
 // LDS.  Bound by FP64 issue (about 1100 operations a cell, 40 divisions among
-// them).  60 cases (3.9 M cells): 175 us; with every thread gathering its
+// them).  60 cases (3.9 M cells): 176 us; with every thread gathering its
 // neighbours' planes and forming their quantities again 256 us (two
-// divisions a neighbour, 160-220 registers).  513x129: 8.1 us (9).
+// divisions a neighbour, 160-220 registers).  513x129: 8.3 us (9).
 constexpr int SAR_N = VIS_NR;
 struct SaLds {
   double nt[SAR_N], vn[SAR_N], U[SAR_N], V[SAR_N], u[SAR_N], v[SAR_N], xx[SAR_N], xy[SAR_N], yx[SAR_N], yy[SAR_N];
@@ -739,8 +740,8 @@ __global__ __launch_bounds__(VIS_THREADS, 4) void k_sa_rhs(const DevMesh* __rest
 // lsolvej (src/samodel2d.f:1306-1344) and s1, sjmat*bjmat of vmu_sa
 // (src/samodel2d.f:148-152) for the k row blockIdx.x, one wave.
 // Bound by one memory round trip and the parts' chain at one case (513x129:
-// 5.5 us; by two lanes from both ends out of LDS 37 us), by HBM in a batch
-// (60 cases, 3.9 M cells, 40 bytes a cell: 36 us; one lane per line side, 99 us).
+// 5.3 us; by two lanes from both ends out of LDS 37 us), by HBM in a batch
+// (60 cases, 3.9 M cells, 40 bytes a cell: 38 us; one lane per line side, 99 us).
 __global__ __launch_bounds__(64) void k_sa_solve_j(const DevMesh* __restrict__ Ms) {
   __shared__ __attribute__((aligned(16))) double buf[PART_BUF];
   const DevMesh& M = Ms[blockIdx.y];
@@ -755,10 +756,11 @@ __global__ __launch_bounds__(64) void k_sa_solve_j(const DevMesh* __restrict__ M
 // clip (src/samodel2d.f:157-188), then the interior eddy viscosity (c_turm)
 // for TC adjacent j columns.  8 columns are half a 128-byte line; with the
 // neighbouring workgroup on the same XCD the other half comes out of its L2,
-// and twice the workgroups of 16 columns hide more latency: 60 cases 102 us
-// (16 columns 111, 4 columns 126; 8 without the runs per XCD 137; lane per line
-// and an update pass of its own 125), 20 cases 35 (16: 37), 513x129 8.0 (16:
-// 8.9, 4: 7.6; two lanes per column from both ends 17.4).
+// and twice the workgroups of 16 columns hide more latency: 60 cases 94 us;
+// with empty workgroups among them 102 (16 columns 111, 4 columns 126; 8 without
+// the runs per XCD 137; lane per line and an update pass of its own 125), 20
+// cases 35 (16: 37).  513x129 7.7 (16: 8.8, 4: 7.6; two lanes per column from
+// both ends 17.4).
 constexpr int SAK_NT = 512;
 template <int TC>
 __global__ __launch_bounds__(SAK_NT) void k_sa_solve_k(const DevMesh* __restrict__ Ms, int ovl) {
